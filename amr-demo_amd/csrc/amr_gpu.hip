@@ -304,10 +304,10 @@ __device__ __forceinline__ void flux_boundary(const InstDev &ip, int side, const
     for (int k = 0; k < 4; ++k) F[k] = fx[k] * nrm[0] + fy[k] * nrm[1];
 }
 
-// Per-cell CFL candidate, solver_time_step_2d_module.F90:107-116, evaluated
-// without FMA contraction so that it reproduces the reference bit for bit;
-// cfl_h = cfl * sqrt(vol), the patch's numerator.
-__device__ __forceinline__ double cfl_candidate_h(const double q[4], double cfl_h)
+// Per-cell wave speed and CFL candidate, solver_time_step_2d_module.F90:107-116,
+// evaluated without FMA contraction so that they reproduce the reference bit
+// for bit; cfl_h = cfl * sqrt(vol), the patch's numerator.
+__device__ __forceinline__ double wave_speed(const double q[4])
 {
 #pragma clang fp contract(off)
     double oneOrho = 1.0 / q[0];
@@ -316,9 +316,10 @@ __device__ __forceinline__ double cfl_candidate_h(const double q[4], double cfl_
     double V2 = u * u + v * v;
     double pOverRho = 0.4 * (q[3] * oneOrho - 0.5 * V2);
     double c = sqrt(1.4 * pOverRho);
-    double eig = sqrt(V2) + c;
-    return cfl_h / eig;
+    return sqrt(V2) + c;
 }
+
+__device__ __forceinline__ double cfl_candidate_h(const double q[4], double cfl_h) { return cfl_h / wave_speed(q); }
 
 __device__ __forceinline__ double cfl_candidate(const double q[4], double cfl, double vol)
 {
@@ -1454,6 +1455,384 @@ __global__ __launch_bounds__(N * N, MINW) void stage_kernel_pp(StageArgs a)
     if (a.norm_part) sum_reduce_store<N2>(sq, &a.norm_part[blockIdx.x], red);
 }
 
+// ---------------------------------------------------------------------------
+// Row-marching stage kernel: one wave, its own workgroup, advances
+// P = 64 / (N R) patches together.  The lanes are P patches x R rows x N columns;
+// the wave walks the patches' rows R at a time (N / R steps), every lane
+// evaluating its cell's +x and +y faces from its record in registers and its
+// two neighbours' in LDS.  The faces left over, the -x and -y edges of the P
+// patches, are one round ahead of the march (all 64 lanes busy with R = 2, half
+// of them with R = 4).  The arithmetic of a face is stage_kernel's, operation
+// for operation: the results are bit for bit those of the other designs.
+//
+// What bounds the small patches is the instruction stream: of a 4x4 patch's 40
+// faces 8 are left over, of a 2x2 patch's 12 faces 4, and stage_kernel spends a
+// round with few lanes busy on them (or, DESIGN 0, three rounds for 2.5), decodes
+// a task list per workgroup and passes two workgroup barriers.  Here 8 4x4
+// patches take 2 + 2 + 1 full rounds, every index is a shift of the lane id, and
+// one wave needs no barrier (its LDS operations execute in order).  LDS holds
+// the rows in flight and the halo only, 9 KB (R = 4) or 14 KB (R = 2) a wave.
+// Measured, us per SSP-RK3 step, DESIGN 0 -> this: 2x2 patches 262k quadrants
+// 238 -> 104, 16k 26.8 -> 17.6; 4x4 patches 176k quadrants (adaptive) 404 -> 240,
+// 21k 43.3 -> 29.1, 256 21.5 -> 13.3.
+// ---------------------------------------------------------------------------
+struct Rec {
+    double r, ru, rv, rE, p, ir, sr;
+};
+
+// The record of one state: store_rec's values, in registers.
+__device__ __forceinline__ Rec make_rec(double r, double ru, double rv, double rE)
+{
+    Rec c;
+    double rsr;
+    c.r = r; c.ru = ru; c.rv = rv; c.rE = rE;
+    fsqrt_rsq(r, c.sr, rsr);
+    c.ir = rsr * rsr;
+    const double u = ru * c.ir, v = rv * c.ir;
+    c.p = (1.4 - 1.0) * fma(-(0.5 * r), fma(u, u, v * v), rE);
+    return c;
+}
+__device__ __forceinline__ Prim prim_of(const Rec &c)
+{
+    Prim P;
+    P.r = c.r; P.ru = c.ru; P.rv = c.rv; P.rE = c.rE; P.p = c.p; P.sr = c.sr;
+    P.u = c.ru * c.ir;
+    P.v = c.rv * c.ir;
+    P.H = (c.rE + c.p) * c.ir;     // E + p/rho
+    return P;
+}
+__device__ __forceinline__ OPrim oprim_of(const Rec &c, bool xdir)
+{
+    OPrim o;
+    o.r = c.r; o.rE = c.rE; o.p = c.p; o.sr = c.sr;
+    o.rn = xdir ? c.ru : c.rv;
+    o.rt = xdir ? c.rv : c.ru;
+    o.un = o.rn * c.ir;
+    o.ut = o.rt * c.ir;
+    o.H = (c.rE + c.p) * c.ir;
+    return o;
+}
+
+// Which vectors beside the stage state a stage reads: its base state U0, its
+// accumulator, or both.
+enum { VEC_BASE = 0, VEC_ACC = 1, VEC_BOTH = 2 };
+
+// LDS accesses before it are not moved past it by the compiler; the wave's
+// LDS operations execute in order, so nothing is waited for.
+__device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
+
+// The value taken anew where it stands: an address built on it is computed
+// beside its use (from a scalar base) instead of being kept in registers from
+// the kernel's start.
+__device__ __forceinline__ unsigned here(unsigned v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+template <int N, int R, int VEC>
+__global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
+{
+    constexpr int N2 = N * N, P = 64 / (N * R), STEPS = N / R, QS = NFLD * N2;
+    constexpr int NE = P * N;                      // edge cells per side of the wave's patches
+    constexpr int HR = 4 * NE / 64;                // halo cells per lane
+    static_assert(R == 2 || R == 4, "two or four rows a step");
+    // records, seven doubles each (a stride free of bank conflicts): the rows of
+    // the step by lane, the row above them, the +x ghosts, the +y ghosts
+    constexpr int RS = 7, ABOVE = 64 * RS, GX = ABOVE + NE * RS, GY = GX + NE * RS;
+    // fluxes on their way to the neighbour lanes, over the step's records, which
+    // nothing reads any more then: +x by lane, +y of all but the top row
+    constexpr int FX = 0, FY = 4 * 64;
+    static_assert(FY + 4 * (64 - NE) <= ABOVE, "the fluxes fit");
+    __shared__ double rec[GY + NE * RS];
+    __shared__ double low[2][NFLD * NE];           // -x edge fluxes; -y fluxes of the bottom row
+    __shared__ double top[NFLD * NE];              // +y fluxes of the top row, for the next step
+    __shared__ double f2[2][NFLD * NE];            // +x, +y: second fine neighbours' fluxes, walls
+
+    typedef const double __attribute__((address_space(1))) gdbl;
+    typedef const char __attribute__((address_space(1))) gchar;
+    gdbl *const Us = (gdbl *)a.Us;
+    const int lane = threadIdx.x;
+    const int nq = a.m.nquad;
+    const int g = xcd_block(blockIdx.x, gridDim.x);
+    const int ci = lane % N, rr = (lane / N) % R, p = lane / (N * R);
+    const int e = p * N + ci;                      // position along the wave's -y and +y edges
+    // the lane's halo cells: sides -x, -y, +x, +y of the wave's patches in turn
+    int2 nb[HR];
+    int tq[HR], tk[HR];
+#pragma unroll
+    for (int j = 0; j < HR; ++j) {
+        const int t = lane + 64 * j, k4 = t / NE, te = t % NE;
+        tq[j] = min(g * P + te / N, nq - 1);
+        tk[j] = te % N;
+        nb[j] = *(const int2 *)(a.m.nbr + (size_t)tq[j] * 8 + (k4 & 1) * 4 + (k4 >> 1) * 2);
+    }
+    // the rows of the first two steps (past the last patch: the buffer's
+    // padding, never stored); a uniform base and a 32-bit byte offset per lane
+    const unsigned off = 8 * (p * QS + rr * N + ci);
+    auto row_load = [&](const double *src, int s, double u[4]) {
+        gchar *b = (gchar *)(gdbl *)(src + (size_t)g * (P * QS) + R * N * s);
+        const unsigned o = here(off);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) u[f] = *(gdbl *)(b + f * N2 * 8 + o);
+    };
+    double raw[4], nraw[4];
+    row_load(a.Us, 0, raw);
+    if (STEPS > 1) row_load(a.Us, 1, nraw);
+    const int quad = min(g * P + p, nq - 1);
+    const bool active = g * P + p < nq;
+    const int lev = a.m.level[quad], inst = a.m.inst[quad];
+    auto cell_load = [&](size_t o, double u[4]) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) u[f] = Us[o + f * N2];
+    };
+    auto is_y = [&](int j) { return (((lane + 64 * j) / NE) & 1) != 0; };
+    auto is_high = [&](int j) { return HR == 2 ? j == 1 : lane >= 2 * NE; };
+    // edge cell of a patch at the high or low end of the side's normal
+    auto edge = [&](int j, bool high) {
+        return is_y(j) ? (high ? (N - 1) * N : 0) + tk[j] : tk[j] * N + (high ? N - 1 : 0);
+    };
+    double gh[HR][4], own[HR][4], sec[HR][4];
+#pragma unroll
+    for (int j = 0; j < HR; ++j) cell_load((size_t)tq[j] * QS + edge(j, is_high(j)), own[j]);
+    // the ghost across the side (a wall: the own edge cell), and the second fine
+    // neighbour's cell on the coarse side of a hanging face
+    bool second = false;
+#pragma unroll
+    for (int j = 0; j < HR; ++j) {
+        cell_load(nb[j].x < 0 ? (size_t)tq[j] * QS + edge(j, is_high(j)) : (size_t)nb[j].x * QS + edge(j, !is_high(j)),
+                  gh[j]);
+        second = second || nb[j].y >= 0;
+    }
+    const bool any_second = __any(second);
+    if (any_second) {
+#pragma unroll
+        for (int j = 0; j < HR; ++j)
+            cell_load((size_t)(nb[j].y < 0 ? tq[j] : nb[j].y) * QS + edge(j, !is_high(j)), sec[j]);
+    }
+    const double h = ldexp(a.m.ip[inst].h_base, -lev) / (double)N;
+    const double dt = a.mode != MODE_RHS ? a.dt_cur[inst] : 0.0;
+    const double ninvV = ldexp(a.m.ip[inst].ninv_vol0, 2 * lev);
+
+    auto put_rec = [&](int t, const Rec &c) {
+        rec[t] = c.r; rec[t + 1] = c.ru; rec[t + 2] = c.rv; rec[t + 3] = c.rE;
+        rec[t + 4] = c.p; rec[t + 5] = c.ir; rec[t + 6] = c.sr;
+    };
+    auto get_prim = [&](int t) {
+        Rec c;
+        c.r = rec[t]; c.ru = rec[t + 1]; c.rv = rec[t + 2]; c.rE = rec[t + 3];
+        c.p = rec[t + 4]; c.ir = rec[t + 5]; c.sr = rec[t + 6];
+        return prim_of(c);
+    };
+    Rec R0 = make_rec(raw[0], raw[1], raw[2], raw[3]);
+    put_rec(lane * RS, R0);
+
+    // ---- the low edges' faces, and every second fine neighbour's flux ----------
+    bool wall = false;
+#pragma unroll
+    for (int j = 0; j < HR; ++j) wall = wall || nb[j].x < 0;
+    const bool any_wall = __any(wall);
+#pragma unroll
+    for (int j = 0; j < HR; ++j) {
+        const bool y = is_y(j), high = is_high(j);
+        const int te = (lane + 64 * j) % NE;
+        Rec c = make_rec(gh[j][0], gh[j][1], gh[j][2], gh[j][3]);
+        if (high) put_rec((y ? GY : GX) + te * RS, c);
+        if (HR == 2 && j == 1 && !any_second && !any_wall) continue;
+        const double th = __shfl(h, (te / N) * (N * R), 64);
+        double *const d = high ? f2[y] + te : low[y] + te;
+        const Rec o = make_rec(own[j][0], own[j][1], own[j][2], own[j][3]);
+        OPrim A = oprim_of(c, !y), O = oprim_of(o, !y);
+        const double hf = nb[j].y >= 0 ? 0.5 * th : th;
+        double G[4] = {0.0, 0.0, 0.0, 0.0}, S[4];
+        if (HR == 1 || j == 0) {
+            if (HR == 1 && any_second) {       // the high sides' lanes: the second neighbour's flux
+                if (high) {
+                    A = O;
+                    O = oprim_of(make_rec(sec[j][0], sec[j][1], sec[j][2], sec[j][3]), !y);
+                }
+            }
+            flux_normal(A, O, hf, G);
+        }
+        if (any_second && !(HR == 1 && !__any(!high && nb[j].y >= 0))) {
+            const OPrim B = oprim_of(make_rec(sec[j][0], sec[j][1], sec[j][2], sec[j][3]), !y);
+            if (HR == 2 && j == 1) {
+                flux_normal(O, B, hf, G);
+            } else {
+                flux_normal(B, O, hf, S);
+                if (!high && nb[j].y >= 0) {
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) G[f] += S[f];
+                }
+            }
+        }
+        d[0] = G[0]; d[NE] = y ? G[2] : G[1]; d[2 * NE] = y ? G[1] : G[2]; d[3 * NE] = G[3];
+        if (any_wall) {
+            if (nb[j].x < 0) {                 // a wall's flux in its place
+                const int tinst = a.m.inst[tq[j]];
+                const double nh = high ? th : -th, fe = high ? (double)N : 0.0;
+                const double nrm[2] = {y ? 0.0 : nh, y ? nh : 0.0};
+                double F[4];
+                flux_boundary(a.m.ip[tinst], 2 * y + high, nrm, own[j], a.m.org + 2 * (size_t)tq[j],
+                              y ? tk[j] + 0.5 : fe, y ? fe : tk[j] + 0.5, th, a.m.t_step[tinst], F);
+#pragma unroll
+                for (int f = 0; f < 4; ++f) d[f * NE] = high ? F[f] : -F[f];
+            }
+        }
+    }
+    // what the lane's own patch has across its high sides
+    const int lx = HR == 2 ? p * N : 2 * NE + p * N, ly = lx + NE;
+    const int nax = __shfl(nb[HR - 1].x, lx, 64), nbx = __shfl(nb[HR - 1].y, lx, 64);
+    const int nay = __shfl(nb[HR - 1].x, ly, 64), nby = __shfl(nb[HR - 1].y, ly, 64);
+    const bool ex = ci == N - 1, ey = rr == R - 1; // on the +x edge; on the +y edge in the last step
+    const bool wx = ex && nax < 0, wy = ey && nay < 0, hx2 = ex && nbx >= 0, hy2 = ey && nby >= 0;
+    const bool any_hi = any_second || any_wall;
+    const double hx = hx2 ? 0.5 * h : h;
+    const bool frozen = a.mode != MODE_RHS && dt == 0.0;
+    const bool any_frozen = __any(frozen);
+    const bool needB = VEC != VEC_ACC && (a.mode == MODE_SO ? a.U0 != nullptr : a.mode != MODE_RHS);
+    const bool needA = VEC != VEC_BASE && !a.first;
+    const double c2dt = a.c2 * dt;
+    double sq = 0.0, eig = 0.0;
+
+#pragma unroll(STEPS <= 2 ? STEPS : 1)
+    for (int s = 0; s < STEPS; ++s) {
+        const bool last = s == STEPS - 1;
+        // the next rows' records; the lowest of them is the row above this step's
+        Rec R1;
+        if (!last) {
+            R1 = make_rec(nraw[0], nraw[1], nraw[2], nraw[3]);
+            if (rr == 0) put_rec(ABOVE + e * RS, R1);
+            if (s + 2 < STEPS) row_load(a.Us, s + 2, nraw);
+        }
+        lds_order();
+        const Prim L = prim_of(R0);
+        const Prim RX = get_prim(ex ? GX + (p * N + rr + R * s) * RS : (lane + 1) * RS);
+        const Prim RY = get_prim(ey ? (last ? GY : ABOVE) + e * RS : (lane + N) * RS);
+        double FA[4], FB[4];
+        flux_face<true>(L, RX, hx, FA);
+        flux_face<false>(L, RY, last && hy2 ? 0.5 * h : h, FB);
+        // both fluxes complete here (see stage_kernel)
+        asm volatile("" : "+v"(FA[0]), "+v"(FA[1]), "+v"(FA[2]), "+v"(FA[3]), "+v"(FB[0]), "+v"(FB[1]),
+                     "+v"(FB[2]), "+v"(FB[3]));
+        const double U[4] = {L.r, L.ru, L.rv, L.rE};
+        if (any_hi) {          // second fine neighbours' fluxes after the first ones; walls
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                const double vx = f2[0][f * NE + p * N + R * s + rr], vy = f2[1][f * NE + e];
+                FA[f] = wx ? vx : hx2 ? FA[f] + vx : FA[f];
+                if (last) FB[f] = wy ? vy : hy2 ? FB[f] + vy : FB[f];
+            }
+        }
+        double B[4] = {0.0, 0.0, 0.0, 0.0}, A[4] = {0.0, 0.0, 0.0, 0.0};
+        if (VEC != VEC_ACC && needB) row_load(a.U0, s, B);
+        if (VEC != VEC_BASE && needA) row_load(a.Acc, s, A);
+        // the fluxes of the low faces: the neighbour lane's, the edges', the top
+        // row's of the step before
+        double *const fx = rec + FX + lane % NE + lane / NE * (NFLD * NE);
+        double *const fy = rec + FY + (p * (R - 1) + rr) * N + ci;
+        constexpr int SY = 64 - NE;                // stride of a field of the +y fluxes
+        const double *const lox = ci == 0 ? low[0] + p * N + R * s + rr : fx - 1;
+        double fyb[4];
+        if (rr == 0) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) fyb[f] = s == 0 ? low[1][f * NE + e] : top[f * NE + e];
+        }
+        lds_order();
+#pragma unroll
+        for (int f = 0; f < 4; ++f) fx[f * NE] = FA[f];
+        if (!ey) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) fy[f * SY] = FB[f];
+        } else if (!last) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) top[f * NE + e] = FB[f];
+        }
+        lds_order();
+        if (rr != 0) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) fyb[f] = fy[f * SY - N];
+        }
+        double k4[4], out[4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            const double Rf = (FA[f] - lox[f * NE]) + (FB[f] - fyb[f]);
+            k4[f] = Rf * ninvV;
+        }
+        lds_order();
+        if (!last) {
+            put_rec(lane * RS, R1);
+            R0 = R1;
+        }
+        if (a.norm_part && active) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) sq = fma(k4[f], k4[f], sq);
+        }
+        // the stage update (stage_update's arithmetic on the vectors loaded above)
+        if (VEC == VEC_ACC) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                A[f] = a.first ? dt * k4[f] : fma(A[f], a.c1, dt * k4[f]);
+                out[f] = fma(a.c2, A[f], U[f]);
+            }
+        } else if (VEC == VEC_BOTH) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                if (a.mode == MODE_RK4_FINAL) {
+                    out[f] = fma(dt / 6.0, A[f] + k4[f], B[f]);
+                } else {
+                    A[f] = a.first ? k4[f] : fma(2.0, k4[f], A[f]);
+                    out[f] = fma(c2dt, k4[f], B[f]);
+                }
+            }
+        } else if (a.mode == MODE_RHS) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) out[f] = k4[f];
+        } else if (needB) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) out[f] = fma(c2dt, k4[f], fma(a.c0, B[f], a.c1 * U[f]));
+        } else {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) out[f] = fma(c2dt, k4[f], a.c1 * U[f]);
+        }
+        if (any_frozen && frozen) {            // past its stop an instance keeps its state bit for bit
+#pragma unroll
+            for (int f = 0; f < 4; ++f) out[f] = U[f];
+        }
+        if (active) {
+            typedef double __attribute__((address_space(1))) gout;
+            typedef char __attribute__((address_space(1))) gcout;
+            gcout *const ob = (gcout *)(gout *)(a.Uout + (size_t)g * (P * QS) + R * N * s);
+            const unsigned o = here(off);
+#pragma unroll
+            for (int f = 0; f < 4; ++f) __builtin_nontemporal_store(out[f], (gout *)(ob + f * N2 * 8 + o));
+            if (VEC == VEC_ACC || (VEC == VEC_BOTH && a.mode == MODE_RK4_ACC)) {
+                gcout *const ab = (gcout *)(gout *)(a.Acc + (size_t)g * (P * QS) + R * N * s);
+#pragma unroll
+                for (int f = 0; f < 4; ++f) *(gout *)(ab + f * N2 * 8 + o) = A[f];
+            }
+        }
+        if (a.role & ROLE_CFL) eig = fmax(eig, wave_speed(out));
+    }
+    if (a.role & ROLE_CFL) {
+        // the smallest quotient of a lane's cells is that of its largest speed
+        // (division rounds monotonically)
+        const double cand = ldexp(a.m.ip[inst].cfl_h0, -lev) / eig;
+        const int i0 = __builtin_amdgcn_readfirstlane(inst);
+        const int sub = blockIdx.x & (NSLOT - 1);
+        if (__all(inst == i0)) {
+            const double v = wave_min(active ? cand : INFINITY);
+            if (lane == 0) atomicMin(&a.slot[i0 * NSLOT + sub], d2bits(v));
+        } else if (active) {
+            atomicMin(&a.slot[inst * NSLOT + sub], d2bits(cand));
+        }
+    }
+    if (a.norm_part) {
+        sq = wave_sum(sq);
+        if (lane == 0) a.norm_part[blockIdx.x] = sq;
+    }
+}
+
 // Standalone CFL minimum (physics_time_step): one thread per cell.
 template <int N, int PPB>
 __global__ __launch_bounds__((Tile<N, PPB>::BLK)) void cfl_kernel(MeshDev m, const double *U,
@@ -1724,6 +2103,7 @@ struct amrgpu_ctx {
     bool org_ok = false, need_org = false;
     int nblocks = 0;
     int variant = -1;
+    bool tile_chosen = false;       // by amrgpu_set_tile / amrgpu_autotune: kept across remeshes
     int cap_quad = 0, cap_inst = 0, cap_blocks = 0;
     size_t cap_state = 0;
     int cur = 0;
@@ -1765,6 +2145,7 @@ const TileVariant kVariants[] = {
     {8, 1, 1, 1}, {8, 1, 4, 1}, {8, 2, 4, 1}, {8, 1, 5, 1},
     {16, 1, 3, 2},
     {16, 1, 5, 1},
+    {2, 16, 3, 3}, {4, 4, 3, 3}, {4, 8, 3, 3},
 };
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
@@ -1798,11 +2179,16 @@ int grid_of(const amrgpu_ctx *c, int v, int nquad)
 // (every tile computes the same bits): for n = 8 and 16 the paired-faces
 // tile with one patch per workgroup, four and five waves per SIMD, the
 // fastest or within 2 % of it on the meshes measured (207k to 16.8M cells).
-int default_variant(int n)
+// n = 2 and 4: the row-marching kernel, faster than the others at every size
+// measured (16 to 262k quadrants).  n = 4 takes two rows a step, with fewer
+// instructions a patch, where its waves of 8 patches fill the chip (256 CUs x
+// 11 waves x 8 = 22k quadrants), else four, with twice the waves: 4k quadrants
+// 18.2 against 15.9 us a step, 20k 29.0 and 29.2, 66k 83.3 and 86.7.
+int default_variant(int n, int nquad)
 {
     switch (n) {
-    case 2: return 0;
-    case 4: return 2;
+    case 2: return 20;
+    case 4: return nquad < 20000 ? 21 : 22;
     case 8: return 15;
     case 16: return 19;
     default: return -1;
@@ -1843,6 +2229,21 @@ int launch_v(amrgpu_ctx *c, const StageArgs &a)
     return AMRGPU_OK;
 }
 
+template <int N, int R>
+int launch_rows(amrgpu_ctx *c, const StageArgs &a)
+{
+    constexpr int P = 64 / (N * R);
+    const dim3 nblk((c->nquad + P - 1) / P);
+    if (a.mode == MODE_LSERK)
+        hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC_ACC>), nblk, dim3(64), 0, c->stream, a);
+    else if (a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL)
+        hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC_BOTH>), nblk, dim3(64), 0, c->stream, a);
+    else
+        hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC_BASE>), nblk, dim3(64), 0, c->stream, a);
+    HIPCHK(hipGetLastError());
+    return AMRGPU_OK;
+}
+
 int launch_stage(amrgpu_ctx *c, const StageArgs &a)
 {
     switch (c->variant) {
@@ -1866,6 +2267,9 @@ int launch_stage(amrgpu_ctx *c, const StageArgs &a)
     case 17: return launch_v<8, 1, 5, 1>(c, a);
     case 18: return launch_pp<16, 3>(c, a);
     case 19: return launch_v<16, 1, 5, 1>(c, a);
+    case 20: return launch_rows<2, 2>(c, a);
+    case 21: return launch_rows<4, 4>(c, a);
+    case 22: return launch_rows<4, 2>(c, a);
     default: set_err("bad tile variant %d", c->variant); return AMRGPU_ERR_ARG;
     }
 }
@@ -2167,14 +2571,17 @@ static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need
     c->cap_quad = capq;
     c->cap_inst = ninst;
     c->cap_state = (size_t)capq * 4 * n2;
+    // the row-marching kernel reads (and drops) the cells of up to 15 patches
+    // past the last one
+    const size_t pad = (size_t)16 * 4 * n2;
     c->cap_blocks = capq + 64;   // enough for one patch per workgroup
     const size_t cq = (size_t)c->cap_quad, cs = c->cap_state;
     HIPCHK(hipMalloc(&c->d_nbr, sizeof(int) * 8 * cq));
     HIPCHK(hipMalloc(&c->d_level, sizeof(int) * cq));
     HIPCHK(hipMalloc(&c->d_inst, sizeof(int) * cq));
     HIPCHK(hipMalloc(&c->d_ip, sizeof(InstDev) * c->cap_inst));
-    for (int i = 0; i < 3; ++i) HIPCHK(hipMalloc(&c->U[i], sizeof(double) * cs));
-    if (need_acc) HIPCHK(hipMalloc(&c->Acc, sizeof(double) * cs));
+    for (int i = 0; i < 3; ++i) HIPCHK(hipMalloc(&c->U[i], sizeof(double) * (cs + pad)));
+    if (need_acc) HIPCHK(hipMalloc(&c->Acc, sizeof(double) * (cs + pad)));
     HIPCHK(hipMalloc(&c->d_dt_cur, sizeof(double) * c->cap_inst));
     HIPCHK(hipMalloc(&c->d_t, sizeof(double) * c->cap_inst));
     HIPCHK(hipMalloc(&c->d_slot, sizeof(unsigned long long) * c->cap_inst * NSLOT));
@@ -2224,7 +2631,10 @@ static int upload_mesh(amrgpu_ctx *c, int ncell, const int *level, const int *ce
     if (cell_inst) memcpy(pq, cell_inst, sizeof(int) * (size_t)ncell);
     else memset(pq, 0, sizeof(int) * (size_t)ncell);
     c->nquad = ncell;
-    if (c->variant < 0 || kVariants[c->variant].n != c->n) c->variant = default_variant(c->n);
+    if (!c->tile_chosen || kVariants[c->variant].n != c->n) {
+        c->variant = default_variant(c->n, ncell);
+        c->tile_chosen = false;
+    }
     c->nblocks = grid_of(c, c->variant, ncell);
     if (c->nblocks > c->cap_blocks || (size_t)ncell * 4 * c->n * c->n > c->cap_state) {
         set_err("internal capacity error");
@@ -2801,6 +3211,7 @@ int amrgpu_set_tile(amrgpu_ctx *c, int ppb, int minw, int design)
             HIPCHK(hipStreamSynchronize(c->stream));
             free_graphs(c);
             c->variant = v;
+            c->tile_chosen = true;
             c->nblocks = grid_of(c, v, c->nquad);
             return AMRGPU_OK;
         }
@@ -2908,6 +3319,7 @@ int amrgpu_autotune(amrgpu_ctx *c, int nsteps, int *nvar, int *ppb, int *minw, i
     const int cur0 = c->cur;
     const bool graphs0 = c->graphs_enabled;
     const int variant0 = c->variant, nblocks0 = c->nblocks;
+    const bool chosen0 = c->tile_chosen;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = AMRGPU_OK;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
@@ -2924,6 +3336,7 @@ int amrgpu_autotune(amrgpu_ctx *c, int nsteps, int *nvar, int *ppb, int *minw, i
         char msg[sizeof(g_err)];
         memcpy(msg, g_err, sizeof(msg));
         c->variant = variant0;
+        c->tile_chosen = chosen0;
         c->nblocks = nblocks0;
         c->graphs_enabled = graphs0;
         free_graphs(c);

@@ -201,7 +201,9 @@ int amrgpu_bench(amrgpu_ctx *c, int nsteps, double *ms_total, double *avg_stage_
 int amrgpu_num_cells(const amrgpu_ctx *c);   /* sub-grid cells */
 /* Tile shape of the stage kernel: patches per workgroup, the minimum waves
  * per SIMD reserved by register allocation, and the face-evaluation design
- * (0: face task list, 1: paired +x/+y faces per cell).  amrgpu_autotune
+ * (0: face task list, 1: paired +x/+y faces per cell, 2: the same, persistent
+ * with prefetch, 3: several patches a wave, row by row).  Until one is set, a
+ * default by patch size and quadrant count applies.  amrgpu_autotune
  * times every compiled variant for the mesh's patch size over nsteps steps
  * with direct launches (state and time are restored afterwards), keeps the
  * fastest and reports each variant's ms per step, then sets the launch mode
