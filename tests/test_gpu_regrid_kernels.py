@@ -1,0 +1,76 @@
+"""The kernels a regrid reads the resident state with (gradient indicator,
+density tags, tagger features) at quadrant counts around their workgroups'
+patches and with values at the edges of their arithmetic."""
+import numpy as np
+import pytest
+
+import amrhip
+
+pytestmark = pytest.mark.gpu
+
+
+def forest(n, splits, seed):
+    """a 2 x 1 brick, periodic in x, with `splits` quadrants of it refined in
+    turn (3 more quadrants each, hanging faces), random positive states"""
+    rng = np.random.default_rng(seed)
+    f = amrhip.Forest(2, 1, (1, 0), 0.0, 0.0, 1.0, n, 0, 6)
+    for k in range(splits):
+        flags = np.zeros(f.nquad, np.int32)
+        flags[(7 * k) % f.nquad] = 1
+        f.refine(flags)
+        f.balance()
+    q = f.soln()
+    q[..., 0] = np.exp(rng.uniform(-1.5, 1.0, q.shape[:3]))
+    q[..., 1:3] = rng.uniform(-1.0, 1.0, q.shape[:3] + (2,))
+    q[..., 3] = rng.uniform(2.0, 5.0, q.shape[:3])
+    return f
+
+
+def context(f):
+    g = amrhip.Gpu()
+    g.setup(f.n, 3, [amrhip.make_inst(1.0)], *f.external())
+    return g
+
+
+@pytest.mark.parametrize("n", [2, 4, 8, 16])
+@pytest.mark.parametrize("splits", [0, 1, 5, 24])
+def test_indicator_and_tags(n, splits):
+    """bit for bit the host's indicator; the density tags of the patch minima
+    and maxima"""
+    f = forest(n, splits, 10 * n + splits)
+    print(f"n={n} quads={f.nquad}", flush=True)
+    g = context(f)
+    assert np.array_equal(g.indicator(), f.indicator())
+    rho = f.soln()[..., 0].reshape(f.nquad, -1)
+    lo, hi = float(np.median(rho.min(axis=1))), float(np.median(rho.max(axis=1)))
+    exp = (rho.min(axis=1) <= lo) | (rho.max(axis=1) >= hi)
+    assert np.array_equal(g.feature_tags([1, 2], [lo, hi]), exp.astype(np.int32))
+    g.close()
+
+
+@pytest.mark.parametrize("case", ["rest", "negative zeros", "tiny", "huge", "mixed scales", "single spike"])
+def test_features_at_the_edges_of_the_quotient(oracle, case):
+    """momenta that vanish, signed zeros, and scales outside the range the
+    product form of the quotient covers: bit for bit the oracle's quotients"""
+    f = forest(8, 9, 5)
+    q = f.soln()
+    if case == "rest":
+        q[..., 1:3] = 0.0
+    elif case == "negative zeros":
+        q[..., 1] = -0.0
+        q[..., 2] = np.where(np.arange(8) % 3 == 0, -0.0, q[..., 2])
+    elif case == "tiny":
+        q[...] *= 2.0 ** -500
+    elif case == "huge":
+        q[...] *= 2.0 ** 600
+    elif case == "mixed scales":
+        q[::2] *= 2.0 ** 450
+        q[1::3, ..., 2] *= 2.0 ** -900
+    else:
+        q[..., 1] = 0.0
+        q[:, 3, 5, 1] = -2.5e-7
+    ci, fi, _, soln = f.external()
+    g = context(f)
+    exp = oracle.tagger_features(8, ci, fi, soln)
+    assert np.array_equal(g.tagger_features(), exp)
+    g.close()
