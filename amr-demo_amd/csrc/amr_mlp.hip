@@ -9,14 +9,21 @@
 // src/solver/src/tagging_methods_module.F90:14-71); features, labels and the
 // network are defined in include/amr_tagger.h.
 //
-// Work decomposition.  A workgroup of four waves takes 64 samples at a time
-// ("chunk"); wave w owns samples 16w..16w+15 through the forward pass and the
-// backward pass down to the pre-activation gradients, while the weight
-// gradients (a reduction over samples) are split by output tile across the
-// waves and stay in registers across the workgroup's chunks.  W1 (48 KB BF16)
-// is staged in LDS once per workgroup; one chunk of features (48 KB) is staged
-// per chunk.  Each workgroup writes one partial gradient; a second kernel sums
-// the partials in a fixed order (bitwise reproducible) and applies Adam.
+// Work decomposition of a gradient.  A minibatch is a few thousand samples of a
+// small network: 2 MFLOP a workgroup if one held 64 samples and all of its
+// weight gradients, on a fraction of the CUs.  Three kernels instead, each
+// spread over the chip:
+//   backprop_kernel  16 samples a workgroup, wave w the 16-wide tile w of every
+//                    layer: forward, loss, and the gradients down to the
+//                    pre-activations, written out transposed (hidden unit major);
+//   wgrad_kernel     the weight gradients, reductions over samples, by output
+//                    tile: a partial sum per `chunks` chunks of 64 samples, its
+//                    dW1 split over 12 waves, its other parts one workgroup;
+//   reduce_kernel    sums the partials in a fixed order (bitwise reproducible)
+//                    and applies Adam.
+// Every sum has the operands and the order it has when one workgroup walks its
+// chunks with the weight gradients in registers, which is how it was before: 42.3
+// + 9.5 us a minibatch of 4096 (32 workgroups of 256 CUs), now 9.1 + 9.2 + 3.5.
 //
 // MFMA operand layouts (lane l, r = l % 16, g = l / 16):
 //   16x16x32: A[i][k]: lane holds A[r][8g + t], B[k][j]: lane holds
@@ -45,7 +52,6 @@ static_assert(NP == AMR_MLP_NPARAM, "parameter layout");
 constexpr int NPP = (NP + 1 + 63) / 64 * 64;     // partial row: gradient + loss, padded
 constexpr int SX = NIN + 8;                      // LDS row strides (elements)
 constexpr int SH = NH + 8;
-constexpr int SZ = 16 + 8;
 constexpr int ROWS = 64;                         // samples per chunk
 constexpr int BLK = 256;
 
@@ -214,30 +220,9 @@ __global__ __launch_bounds__(256) void pool16_kernel(const double *__restrict__ 
 // ---------------------------------------------------------------------------
 // shared pieces of the network kernels
 // ---------------------------------------------------------------------------
-struct __attribute__((aligned(16))) NetLds {     // rows read as 16-byte vectors
-    uint16_t W1[NH * SX];
-    uint16_t X[ROWS * SX];
-    uint16_t W2[NH * SH];
-    uint16_t W3[16 * SH];       // rows 3..15 zero
-    uint16_t H1[ROWS * SH];
-    uint16_t H2[ROWS * SH];
-    float b[2 * NH + 4];
-    float Z[ROWS * 4];
-};
-
-struct __attribute__((aligned(16))) TrainLds {
-    NetLds net;
-    uint16_t dA2[ROWS * SH];
-    uint16_t dA1[ROWS * SH];
-    uint16_t dZ[ROWS * SZ];     // classes 3..15 zero
-    float w[ROWS];
-    int y[ROWS];
-    float bg[2 * NH + 4];       // bias gradients, loss in bg[2*NH+3]
-    float loss[ROWS];
-};
-
 struct Weights {
-    const uint16_t *W1, *W2, *W3;   // BF16 copies: [64][384], [64][64], [16][64]
+    const uint16_t *W1, *W2, *W3;   // BF16 copies: [64][384], [64][64], [16][64] (rows 3..15 zero)
+    const uint16_t *W2t;            // W2 transposed
     const float *P;                 // FP32 master (biases read from here)
 };
 
@@ -262,87 +247,6 @@ __device__ void stage_weights(Lds &s, const Weights &wt)
         s.b[NH + tid] = wt.P[OB2 + tid];
     }
     if (tid < 4) s.b[2 * NH + tid] = tid < NOUT ? wt.P[OB3 + tid] : 0.0f;
-}
-
-// Feature rows of one chunk into LDS; rows past `count` are zero.
-__device__ void stage_rows(NetLds &s, const uint16_t *__restrict__ X, const int *__restrict__ perm,
-                           long long first, int local0, int count)
-{
-    for (int i = threadIdx.x; i < ROWS * NIN / 8; i += BLK) {
-        const int row = i / (NIN / 8), c8 = i % (NIN / 8);
-        const int loc = local0 + row;
-        uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        if (loc < count) {
-            const long long g = first + loc;
-            const long long src = perm ? (long long)perm[g] : g;
-            v = ((const uint4 *)(X + (size_t)src * NIN))[c8];
-        }
-        *(uint4 *)&s.X[row * SX + c8 * 8] = v;
-    }
-}
-
-// Forward pass of wave w's 16 samples: H1, H2 (BF16, ReLU) and logits Z.
-__device__ void forward_rows(NetLds &s)
-{
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int row = 16 * w + r;
-    {
-        f4v acc[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int kk = 0; kk < NIN / 32; ++kk) {
-            const s8v a = *(const s8v *)&s.X[row * SX + 32 * kk + 8 * g];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const s8v bv = *(const s8v *)&s.W1[(16 * c + r) * SX + 32 * kk + 8 * g];
-                acc[c] = mfma32(a, bv, acc[c]);
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int smp = 16 * w + 4 * g + t, h = 16 * c + r;
-                s.H1[smp * SH + h] = f2bf(fmaxf(acc[c][t] + s.b[h], 0.0f));
-            }
-    }
-    __syncthreads();
-    {
-        f4v acc[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < NH / 32; ++kk) {
-            const s8v a = *(const s8v *)&s.H1[row * SH + 32 * kk + 8 * g];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const s8v bv = *(const s8v *)&s.W2[(16 * c + r) * SH + 32 * kk + 8 * g];
-                acc[c] = mfma32(a, bv, acc[c]);
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int smp = 16 * w + 4 * g + t, h = 16 * c + r;
-                s.H2[smp * SH + h] = f2bf(fmaxf(acc[c][t] + s.b[NH + h], 0.0f));
-            }
-    }
-    __syncthreads();
-    {
-        f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < NH / 32; ++kk) {
-            const s8v a = *(const s8v *)&s.H2[row * SH + 32 * kk + 8 * g];
-            const s8v bv = *(const s8v *)&s.W3[r * SH + 32 * kk + 8 * g];
-            acc = mfma32(a, bv, acc);
-        }
-        if (r < NOUT)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) s.Z[(16 * w + 4 * g + t) * 4 + r] = acc[t] + s.b[2 * NH + r];
-    }
-    __syncthreads();
 }
 
 // Inference: logits (optional) and argmax class (optional) of `count` rows.
@@ -450,179 +354,200 @@ struct GradArgs {
     const int *perm;       // nullptr: rows first.. in order
     long long first;
     int count;             // rows of this launch
-    int chunks;            // chunks per workgroup
+    int chunks;            // chunks per partial sum
+    int ld;                // rows of the buffers below: count up to whole partial sums
     float cw[3];           // class weights
     float scale;           // 1 / sum of row weights
-    float *partial;        // [gridDim.x][NPP]
+    // activations and pre-activation gradients, [64][ld] (dZ: [3][ld])
+    uint16_t *H1, *H2, *dA1, *dA2, *dZ;
+    float *loss;           // [ld]
+    float *partial;        // [partial sums][NPP]
 };
 
-// Loss and parameter gradient partials of `chunks` chunks per workgroup.
-__global__ __launch_bounds__(BLK) void grad_kernel(Weights wt, GradArgs ga)
+// Forward pass, loss and pre-activation gradients of 16 samples.  Latency bounds
+// it: every CU has one workgroup or two, its operands come straight from memory
+// or L2 (all loads of a layer in flight together), and the three exchanges
+// between the waves go through LDS.
+__global__ __launch_bounds__(BLK) void backprop_kernel(Weights wt, GradArgs ga)
 {
-    __shared__ TrainLds s;
-    NetLds &n = s.net;
+    __shared__ __attribute__((aligned(16))) uint16_t h1s[16 * SH], h2s[16 * SH], a2s[16 * SH];
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
-    stage_weights(n, wt);
-    for (int i = tid; i < ROWS * SZ; i += BLK) s.dZ[i] = 0;
-    if (tid < 2 * NH + 4) s.bg[tid] = 0.0f;
-
-    f4v g1[4][6], g2[4], g3;
+    const int row0 = blockIdx.x * 16, loc = row0 + r;      // the lane's sample
+    const bool valid = loc < ga.count;                     // rows past the last: features and weight zero
+    const long long gi = ga.first + (valid ? loc : 0);
+    const long long src = ga.perm ? (long long)ga.perm[gi] : gi;
+    constexpr int KK = NIN / 32;
+    s8v xa[KK], wb[KK];
+    const uint16_t *const xrow = ga.X + (size_t)src * NIN + 8 * g;
+    const uint16_t *const wrow = wt.W1 + (16 * w + r) * NIN + 8 * g;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-#pragma unroll
-        for (int b = 0; b < 6; ++b) g1[a][b] = f4v{0.f, 0.f, 0.f, 0.f};
-        g2[a] = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int kk = 0; kk < KK; ++kk) {
+        wb[kk] = *(const s8v *)(wrow + 32 * kk);
+        xa[kk] = valid ? *(const s8v *)(xrow + 32 * kk) : s8v{0, 0, 0, 0, 0, 0, 0, 0};
     }
-    g3 = f4v{0.f, 0.f, 0.f, 0.f};
-
-    for (int k = 0; k < ga.chunks; ++k) {
-        const int local0 = (blockIdx.x * ga.chunks + k) * ROWS;
-        stage_rows(n, ga.X, ga.perm, ga.first, local0, ga.count);
-        if (tid < ROWS) {
-            const int loc = local0 + tid;
-            int yy = 0;
-            float wv = 0.0f;
-            if (loc < ga.count) {
-                const long long gi = ga.first + loc;
-                yy = ga.y[ga.perm ? (long long)ga.perm[gi] : gi];
-                wv = ga.cw[yy];
-            }
-            s.y[tid] = yy;
-            s.w[tid] = wv;
-        }
-        __syncthreads();
-        forward_rows(n);
-
-        // softmax cross-entropy, one thread per sample
-        if (tid < ROWS) {
-            const float z[3] = {n.Z[tid * 4], n.Z[tid * 4 + 1], n.Z[tid * 4 + 2]};
-            const float m = fmaxf(z[0], fmaxf(z[1], z[2]));
-            const float e0 = expf(z[0] - m), e1 = expf(z[1] - m), e2 = expf(z[2] - m);
-            const float S = e0 + e1 + e2;
-            const int yy = s.y[tid];
-            const float wv = s.w[tid], gs = wv * ga.scale;
-            const float p[3] = {e0 / S, e1 / S, e2 / S};
+    const int yy = valid ? ga.y[src] : 0;
+    const int hid = 16 * w + r;                            // the lane's unit of either hidden layer
+    s8v w2b[2], w3b[2], w2t[2];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) s.dZ[tid * SZ + c] = f2bf(gs * (p[c] - (c == yy ? 1.0f : 0.0f)));
-            s.loss[tid] = wv > 0.0f ? gs * (logf(S) - (z[yy] - m)) : 0.0f;
-        }
-        __syncthreads();
-
-        // dW3 += dZ^T H2 (wave w: hidden tile w)
-#pragma unroll
-        for (int kk = 0; kk < ROWS / 32; ++kk) {
-            s8v a, bv;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int smp = 32 * kk + 8 * g + t;
-                a[t] = (short)s.dZ[smp * SZ + r];
-                bv[t] = (short)n.H2[smp * SH + 16 * w + r];
-            }
-            g3 = mfma32(a, bv, g3);
-        }
-        // dA2 = (dZ W3) * [H2 > 0] for wave w's samples
-        {
-            const s4v a = *(const s4v *)&s.dZ[(16 * w + r) * SZ + 4 * g];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                s4v bv;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) bv[t] = (short)n.W3[(4 * g + t) * SH + 16 * c + r];
-                const f4v d = mfma(a, bv, f4v{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int idx = (16 * w + 4 * g + t) * SH + 16 * c + r;
-                    s.dA2[idx] = f2bf(bf2f(n.H2[idx]) > 0.0f ? d[t] : 0.0f);
-                }
-            }
-        }
-        __syncthreads();
-        // dA1 = (dA2 W2) * [H1 > 0] for wave w's samples
-        {
-            f4v acc[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[c] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < NH / 32; ++kk) {
-                const s8v a = *(const s8v *)&s.dA2[(16 * w + r) * SH + 32 * kk + 8 * g];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    s8v bv;
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) bv[t] = (short)n.W2[(32 * kk + 8 * g + t) * SH + 16 * c + r];
-                    acc[c] = mfma32(a, bv, acc[c]);
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int idx = (16 * w + 4 * g + t) * SH + 16 * c + r;
-                    s.dA1[idx] = f2bf(bf2f(n.H1[idx]) > 0.0f ? acc[c][t] : 0.0f);
-                }
-        }
-        // dW2 += dA2^T H1 (wave w: output-row tile w)
-#pragma unroll
-        for (int kk = 0; kk < ROWS / 32; ++kk) {
-            s8v a;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) a[t] = (short)s.dA2[(32 * kk + 8 * g + t) * SH + 16 * w + r];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                s8v bv;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) bv[t] = (short)n.H1[(32 * kk + 8 * g + t) * SH + 16 * c + r];
-                g2[c] = mfma32(a, bv, g2[c]);
-            }
-        }
-        __syncthreads();
-        // dW1 += dA1^T X (wave w: feature tiles 6w..6w+5)
-#pragma unroll
-        for (int kk = 0; kk < ROWS / 32; ++kk) {
-            s8v a[4];
-#pragma unroll
-            for (int hc = 0; hc < 4; ++hc)
-#pragma unroll
-                for (int t = 0; t < 8; ++t) a[hc][t] = (short)s.dA1[(32 * kk + 8 * g + t) * SH + 16 * hc + r];
-#pragma unroll
-            for (int fi = 0; fi < 6; ++fi) {
-                s8v bv;
-#pragma unroll
-                for (int t = 0; t < 8; ++t)
-                    bv[t] = (short)n.X[(32 * kk + 8 * g + t) * SX + 16 * (6 * w + fi) + r];
-#pragma unroll
-                for (int hc = 0; hc < 4; ++hc) g1[hc][fi] = mfma32(a[hc], bv, g1[hc][fi]);
-            }
-        }
-        // bias gradients and loss: fixed summation order over the chunk's samples
-        if (tid < NH) {
-            float acc = 0.0f;
-            for (int q = 0; q < ROWS; ++q) acc += bf2f(s.dA1[q * SH + tid]);
-            s.bg[tid] += acc;
-        } else if (tid < 2 * NH) {
-            float acc = 0.0f;
-            for (int q = 0; q < ROWS; ++q) acc += bf2f(s.dA2[q * SH + tid - NH]);
-            s.bg[tid] += acc;
-        } else if (tid < 2 * NH + NOUT) {
-            float acc = 0.0f;
-            for (int q = 0; q < ROWS; ++q) acc += bf2f(s.dZ[q * SZ + tid - 2 * NH]);
-            s.bg[tid] += acc;
-        } else if (tid == 2 * NH + 3) {
-            float acc = 0.0f;
-            for (int q = 0; q < ROWS; ++q) acc += s.loss[q];
-            s.bg[tid] += acc;
-        }
-        __syncthreads();
+    for (int kk = 0; kk < 2; ++kk) {
+        w2b[kk] = *(const s8v *)(wt.W2 + hid * NH + 32 * kk + 8 * g);
+        w2t[kk] = *(const s8v *)(wt.W2t + hid * NH + 32 * kk + 8 * g);
+        w3b[kk] = *(const s8v *)(wt.W3 + r * NH + 32 * kk + 8 * g);
     }
+    s4v w3t = s4v{0, 0, 0, 0};                             // W3[class 4g + t][unit]
+    if (g == 0)
+#pragma unroll
+        for (int t = 0; t < NOUT; ++t) w3t[t] = (short)wt.W3[t * NH + hid];
+    const float b1 = wt.P[OB1 + hid], b2 = wt.P[OB2 + hid], b3 = wt.P[OB3 + (r < NOUT ? r : 0)];
 
-    float *part = ga.partial + (size_t)blockIdx.x * NPP;
+    // a layer's values of the lane's unit, samples 4g..4g+3: to the other waves
+    // by sample, to the weight gradients by unit
+    auto put = [&](const uint16_t v[4], uint16_t *lds, uint16_t *out) {
+        ushort4 q;
+        q.x = v[0]; q.y = v[1]; q.z = v[2]; q.w = v[3];
+        *(ushort4 *)(out + (size_t)hid * ga.ld + row0 + 4 * g) = q;
+        if (lds)
 #pragma unroll
-    for (int hc = 0; hc < 4; ++hc)
+            for (int t = 0; t < 4; ++t) lds[(4 * g + t) * SH + hid] = v[t];
+    };
+    f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int fi = 0; fi < 6; ++fi)
+    for (int kk = 0; kk < KK; ++kk) acc = mfma32(xa[kk], wb[kk], acc);
+    uint16_t h1[4], h2[4], da[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-                part[OW1 + (16 * hc + 4 * g + t) * NIN + 16 * (6 * w + fi) + r] = g1[hc][fi][t];
+    for (int t = 0; t < 4; ++t) h1[t] = f2bf(fmaxf(acc[t] + b1, 0.0f));
+    put(h1, h1s, ga.H1);
+    __syncthreads();
+    acc = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) acc = mfma32(*(const s8v *)&h1s[r * SH + 32 * kk + 8 * g], w2b[kk], acc);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) h2[t] = f2bf(fmaxf(acc[t] + b2, 0.0f));
+    put(h2, h2s, ga.H2);
+    __syncthreads();
+    // logits (every wave all of them): lane holds class r of samples 4g..4g+3,
+    // gathered to the sample's lanes
+    f4v zc = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) zc = mfma32(*(const s8v *)&h2s[r * SH + 32 * kk + 8 * g], w3b[kk], zc);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) zc[t] += b3;
+    float z[NOUT];
+#pragma unroll
+    for (int c = 0; c < NOUT; ++c) {
+        const int from = (r >> 2) * 16 + c;
+        const float v0 = __shfl(zc[0], from, 64), v1 = __shfl(zc[1], from, 64);
+        const float v2 = __shfl(zc[2], from, 64), v3 = __shfl(zc[3], from, 64);
+        z[c] = (r & 2) ? ((r & 1) ? v3 : v2) : ((r & 1) ? v1 : v0);
+    }
+    // softmax cross-entropy of sample r
+    const float m = fmaxf(z[0], fmaxf(z[1], z[2]));
+    const float e0 = expf(z[0] - m), e1 = expf(z[1] - m), e2 = expf(z[2] - m);
+    const float S = e0 + e1 + e2;
+    const float wv = valid ? ga.cw[yy] : 0.0f, gs = wv * ga.scale;
+    const float pr[3] = {e0 / S, e1 / S, e2 / S};
+    uint16_t dz[NOUT];
+#pragma unroll
+    for (int c = 0; c < NOUT; ++c) dz[c] = f2bf(gs * (pr[c] - (c == yy ? 1.0f : 0.0f)));
+    if (w == 0 && g == 0) {
+        const float zy = yy == 0 ? z[0] : yy == 1 ? z[1] : z[2];
+        ga.loss[loc] = wv > 0.0f ? gs * (logf(S) - (zy - m)) : 0.0f;
+#pragma unroll
+        for (int c = 0; c < NOUT; ++c) ga.dZ[(size_t)c * ga.ld + loc] = dz[c];
+    }
+    // dA2 = (dZ W3) * [H2 > 0]: classes 4g..4g+3 of sample r, all but 0..2 zero
+    s4v az = s4v{0, 0, 0, 0};
+    if (g == 0)
+#pragma unroll
+        for (int c = 0; c < NOUT; ++c) az[c] = (short)dz[c];
+    acc = mfma(az, w3t, f4v{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int t = 0; t < 4; ++t) da[t] = f2bf(bf2f(h2[t]) > 0.0f ? acc[t] : 0.0f);
+    put(da, a2s, ga.dA2);
+    __syncthreads();
+    // dA1 = (dA2 W2) * [H1 > 0]
+    acc = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) acc = mfma32(*(const s8v *)&a2s[r * SH + 32 * kk + 8 * g], w2t[kk], acc);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) da[t] = f2bf(bf2f(h1[t]) > 0.0f ? acc[t] : 0.0f);
+    put(da, nullptr, ga.dA1);
+}
+
+// Weight gradients of one partial sum (blockIdx.x), reductions over samples.
+// blockIdx.y 0..2: dW1 += dA1^T X for 128 features, wave w hidden tile w.  A lane
+// loads eight consecutive features (16 bytes) of its eight samples and pairs
+// samples by byte permutes, so feature tile j is features 8r + j: no transpose
+// through LDS.  blockIdx.y 3: dW2, dW3, biases and loss.
+constexpr int WG_FEATURES = 128;
+__global__ __launch_bounds__(BLK) void wgrad_kernel(GradArgs ga)
+{
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.x * ga.chunks * ROWS, rows = ga.chunks * ROWS;
+    float *const part = ga.partial + (size_t)blockIdx.x * NPP;
+    if (blockIdx.y < NIN / WG_FEATURES) {
+        const int f0 = WG_FEATURES * blockIdx.y + 8 * r;
+        f4v acc[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] = f4v{0.f, 0.f, 0.f, 0.f};
+        // a chunk's loads in flight together, the ids of its rows a chunk ahead
+        long long src[2][8];
+        auto ids = [&](int c0) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const long long gi = ga.first + min(c0 + 32 * k + 8 * g + t, ga.count - 1);
+                    src[k][t] = ga.perm ? (long long)ga.perm[gi] : gi;
+                }
+        };
+        ids(row0);
+        for (int c0 = row0; c0 < row0 + rows; c0 += ROWS) {
+            s8v a[2];
+            uint4 x[2][8];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                a[k] = *(const s8v *)(ga.dA1 + (size_t)(16 * w + r) * ga.ld + c0 + 32 * k + 8 * g);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    x[k][t] = *(const uint4 *)(ga.X + (size_t)src[k][t] * NIN + f0);
+                    if (c0 + 32 * k + 8 * g + t >= ga.count) x[k][t] = make_uint4(0u, 0u, 0u, 0u);
+                }
+            }
+            ids(min(c0 + ROWS, row0 + rows - ROWS));
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    union { unsigned u[4]; s8v v; } b;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const unsigned lo = (&x[k][2 * q].x)[j >> 1], hi = (&x[k][2 * q + 1].x)[j >> 1];
+                        // halves j & 1 of two samples, the first one low
+                        b.u[q] = __builtin_amdgcn_perm(hi, lo, (j & 1) ? 0x07060302u : 0x05040100u);
+                    }
+                    acc[j] = mfma32(a[k], b.v, acc[j]);
+                }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            float *o = part + OW1 + (16 * w + 4 * g + t) * NIN + f0;
+            *(float4 *)o = make_float4(acc[0][t], acc[1][t], acc[2][t], acc[3][t]);
+            *(float4 *)(o + 4) = make_float4(acc[4][t], acc[5][t], acc[6][t], acc[7][t]);
+        }
+        return;
+    }
+    f4v g2[4], g3 = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) g2[c] = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = row0; s0 < row0 + rows; s0 += 32) {
+        auto units = [&](const uint16_t *T, int u) { return *(const s8v *)(T + (size_t)u * ga.ld + s0 + 8 * g); };
+        const s8v a = units(ga.dA2, 16 * w + r);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) g2[c] = mfma32(a, units(ga.H1, 16 * c + r), g2[c]);
+        const s8v z = r < NOUT ? units(ga.dZ, r) : s8v{0, 0, 0, 0, 0, 0, 0, 0};
+        g3 = mfma32(z, units(ga.H2, 16 * w + r), g3);
+    }
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -630,12 +555,34 @@ __global__ __launch_bounds__(BLK) void grad_kernel(Weights wt, GradArgs ga)
     if (g == 0)
 #pragma unroll
         for (int t = 0; t < NOUT; ++t) part[OW3 + t * NH + 16 * w + r] = g3[t];
-    if (tid < NH) {
-        part[OB1 + tid] = s.bg[tid];
-        part[OB2 + tid] = s.bg[NH + tid];
+    // bias gradients and loss: each chunk's samples in order, then the chunks
+    if (tid >= 2 * NH + NOUT + 1) return;
+    const uint16_t *const T = tid < NH ? ga.dA1 + (size_t)tid * ga.ld
+                              : tid < 2 * NH ? ga.dA2 + (size_t)(tid - NH) * ga.ld
+                                             : ga.dZ + (size_t)min(tid - 2 * NH, NOUT - 1) * ga.ld;
+    float sum = 0.0f;
+    for (int k = 0; k < ga.chunks; ++k) {
+        const int c0 = row0 + k * ROWS;
+        float acc = 0.0f;
+        if (tid < 2 * NH + NOUT) {
+            uint4 v[ROWS / 8];
+#pragma unroll
+            for (int q = 0; q < ROWS / 8; ++q) v[q] = *(const uint4 *)(T + c0 + 8 * q);
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q) {
+                const unsigned d = (&v[q / 8].x)[(q % 8) / 2];
+                acc += bf2f((uint16_t)((q & 1) ? d >> 16 : d & 0xffffu));
+            }
+        } else {
+            float v[ROWS];
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q) v[q] = ga.loss[c0 + q];
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q) acc += v[q];
+        }
+        sum += acc;
     }
-    if (tid < NOUT) part[OB3 + tid] = s.bg[2 * NH + tid];
-    if (tid == 0) part[NP] = s.bg[2 * NH + 3];
+    part[tid < NH ? OB1 + tid : tid < 2 * NH ? OB2 + tid - NH : tid < 2 * NH + NOUT ? OB3 + tid - 2 * NH : NP] = sum;
 }
 
 struct AdamArgs {
@@ -643,39 +590,66 @@ struct AdamArgs {
     float lr, beta1, beta2, eps, bc1, bc2;   // bc = 1 / (1 - beta^t)
 };
 
-// Sum of the partials in workgroup order; optional Adam update and BF16 copy.
-__global__ __launch_bounds__(256) void reduce_kernel(const float *__restrict__ partial, int nparts,
-                                                     float *__restrict__ grad, float *__restrict__ loss,
-                                                     float *P, float *M, float *V, uint16_t *W1b,
-                                                     uint16_t *W2b, uint16_t *W3b, AdamArgs ad)
+// Sum of the partials in their order; optional Adam update and BF16 copies.  The
+// loads of AHEAD partials are in flight together (the sum stays sequential): with
+// one after the other their latency was most of the kernel's time.
+__device__ __forceinline__ void put_bf16(int p, float x, uint16_t *W1b, uint16_t *W2b, uint16_t *W2t, uint16_t *W3b)
 {
+    const uint16_t v = f2bf(x);
+    if (p < OB1) {
+        W1b[p] = v;
+    } else if (p >= OW2 && p < OB2) {
+        const int q = p - OW2;
+        W2b[q] = v;
+        W2t[(q % NH) * NH + q / NH] = v;
+    } else if (p >= OW3 && p < OB3) {
+        W3b[p - OW3] = v;
+    }
+}
+
+__global__ __launch_bounds__(64) void reduce_kernel(const float *__restrict__ partial, int nparts,
+                                                    float *__restrict__ grad, float *__restrict__ loss, float *P,
+                                                    float *M, float *V, uint16_t *W1b, uint16_t *W2b, uint16_t *W2t,
+                                                    uint16_t *W3b, AdamArgs ad)
+{
+#pragma clang fp contract(off)
+    constexpr int AHEAD = 32;
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p > NP) return;
+    const bool param = ad.on && p < NP;
+    const float m0 = param ? M[p] : 0.0f, v0 = param ? V[p] : 0.0f, x0 = param ? P[p] : 0.0f;
     float gsum = 0.0f;
-    for (int b = 0; b < nparts; ++b) gsum += partial[(size_t)b * NPP + p];
+    int b = 0;
+    for (; b + AHEAD <= nparts; b += AHEAD) {
+        float v[AHEAD];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) v[k] = partial[(size_t)(b + k) * NPP + p];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) gsum += v[k];
+    }
+#pragma unroll 8
+    for (; b < nparts; ++b) gsum += partial[(size_t)b * NPP + p];
     if (p == NP) {
         if (loss) *loss = gsum;
         return;
     }
     if (grad) grad[p] = gsum;
     if (!ad.on) return;
-    const float m = ad.beta1 * M[p] + (1.0f - ad.beta1) * gsum;
-    const float v = ad.beta2 * V[p] + (1.0f - ad.beta2) * gsum * gsum;
+    // the multiply-adds are written out: an update's bits do not depend on what
+    // the compiler finds to fuse
+    const float m = fmaf(1.0f - ad.beta1, gsum, ad.beta1 * m0);
+    const float v = fmaf(gsum, (1.0f - ad.beta2) * gsum, ad.beta2 * v0);
     M[p] = m;
     V[p] = v;
-    const float x = P[p] - ad.lr * (m * ad.bc1) / (sqrtf(v * ad.bc2) + ad.eps);
+    const float x = x0 - ad.lr * (m * ad.bc1) / (sqrtf(v * ad.bc2) + ad.eps);
     P[p] = x;
-    if (p < OB1) W1b[p] = f2bf(x);
-    else if (p >= OW2 && p < OB2) W2b[p - OW2] = f2bf(x);
-    else if (p >= OW3 && p < OB3) W3b[p - OW3] = f2bf(x);
+    put_bf16(p, x, W1b, W2b, W2t, W3b);
 }
 
-__global__ void bf16_copy_kernel(const float *P, uint16_t *W1b, uint16_t *W2b, uint16_t *W3b)
+__global__ void bf16_copy_kernel(const float *P, uint16_t *W1b, uint16_t *W2b, uint16_t *W2t, uint16_t *W3b)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < OB1) W1b[p] = f2bf(P[p]);
-    else if (p >= OW2 && p < OB2) W2b[p - OW2] = f2bf(P[p]);
-    else if (p >= OW3 && p < OB3) W3b[p - OW3] = f2bf(P[p]);
+    if (p < NP) put_bf16(p, P[p], W1b, W2b, W2t, W3b);
 }
 
 #define MCHK(x)                                                                               \
@@ -715,9 +689,12 @@ int grow(T **p, size_t *cap, size_t need, bool keep, size_t used)
 struct amr_mlp {
     hipStream_t stream = nullptr;
     float *P = nullptr, *M = nullptr, *V = nullptr, *grad = nullptr, *loss = nullptr;
-    uint16_t *W1b = nullptr, *W2b = nullptr, *W3b = nullptr;
+    uint16_t *W1b = nullptr, *W2b = nullptr, *W2t = nullptr, *W3b = nullptr;
     float *partial = nullptr;
     size_t cap_partial = 0;
+    uint16_t *act = nullptr;    // GradArgs' activations and gradients
+    float *row_loss = nullptr;
+    size_t cap_act = 0, cap_row_loss = 0;
     uint16_t *X = nullptr;      // scratch rows (host uploads, context features)
     size_t cap_X = 0;
     int *y = nullptr, *perm = nullptr, *cls = nullptr;
@@ -739,7 +716,7 @@ struct amr_tagset {
 
 namespace {
 
-Weights weights_of(const amr_mlp *m) { return Weights{m->W1b, m->W2b, m->W3b, m->P}; }
+Weights weights_of(const amr_mlp *m) { return Weights{m->W1b, m->W2b, m->W3b, m->W2t, m->P}; }
 
 int launch_infer(amr_mlp *m, const uint16_t *dX, int count, float *dlogits, int *dcls, hipStream_t st)
 {
@@ -757,17 +734,26 @@ int launch_grad(amr_mlp *m, const uint16_t *dX, const int *dy, const int *dperm,
                 const float cw[3], float scale, int chunks, const AdamArgs &ad, float *dloss)
 {
     int nblk = (count + ROWS * chunks - 1) / (ROWS * chunks);
+    const size_t ld = (size_t)nblk * chunks * ROWS;
     int rc = grow(&m->partial, &m->cap_partial, (size_t)nblk * NPP, false, 0);
+    if (!rc) rc = grow(&m->act, &m->cap_act, ld * (4 * NH + NOUT), false, 0);
+    if (!rc) rc = grow(&m->row_loss, &m->cap_row_loss, ld, false, 0);
     if (rc) return rc;
     GradArgs ga;
     ga.X = dX; ga.y = dy; ga.perm = dperm; ga.first = first; ga.count = count; ga.chunks = chunks;
+    ga.ld = (int)ld;
     ga.cw[0] = cw[0]; ga.cw[1] = cw[1]; ga.cw[2] = cw[2];
     ga.scale = scale;
+    ga.H1 = m->act; ga.H2 = ga.H1 + ld * NH; ga.dA1 = ga.H2 + ld * NH; ga.dA2 = ga.dA1 + ld * NH;
+    ga.dZ = ga.dA2 + ld * NH;
+    ga.loss = m->row_loss;
     ga.partial = m->partial;
-    hipLaunchKernelGGL(grad_kernel, dim3(nblk), dim3(BLK), 0, m->stream, weights_of(m), ga);
+    hipLaunchKernelGGL(backprop_kernel, dim3((unsigned)(ld / 16)), dim3(BLK), 0, m->stream, weights_of(m), ga);
     MCHK(hipGetLastError());
-    hipLaunchKernelGGL(reduce_kernel, dim3((NP + 1 + 255) / 256), dim3(256), 0, m->stream, m->partial, nblk,
-                       m->grad, dloss, m->P, m->M, m->V, m->W1b, m->W2b, m->W3b, ad);
+    hipLaunchKernelGGL(wgrad_kernel, dim3(nblk, NIN / WG_FEATURES + 1), dim3(BLK), 0, m->stream, ga);
+    MCHK(hipGetLastError());
+    hipLaunchKernelGGL(reduce_kernel, dim3((NP + 1 + 63) / 64), dim3(64), 0, m->stream, m->partial, nblk,
+                       m->grad, dloss, m->P, m->M, m->V, m->W1b, m->W2b, m->W2t, m->W3b, ad);
     MCHK(hipGetLastError());
     return AMRGPU_OK;
 }
@@ -803,6 +789,7 @@ amr_mlp_t *amr_mlp_create(unsigned long long seed)
     ok = ok && hipMalloc((void **)&m->loss, sizeof(float) * 4) == hipSuccess;
     ok = ok && hipMalloc((void **)&m->W1b, sizeof(uint16_t) * NH * NIN) == hipSuccess;
     ok = ok && hipMalloc((void **)&m->W2b, sizeof(uint16_t) * NH * NH) == hipSuccess;
+    ok = ok && hipMalloc((void **)&m->W2t, sizeof(uint16_t) * NH * NH) == hipSuccess;
     ok = ok && hipMalloc((void **)&m->W3b, sizeof(uint16_t) * 16 * NH) == hipSuccess;
     ok = ok && hipMemset(m->W3b, 0, sizeof(uint16_t) * 16 * NH) == hipSuccess;
     if (!ok) {
@@ -821,7 +808,7 @@ void amr_mlp_destroy(amr_mlp_t *m)
 {
     if (!m) return;
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    void *bufs[] = {m->P, m->M, m->V, m->grad, m->loss, m->W1b, m->W2b, m->W3b, m->partial,
+    void *bufs[] = {m->P, m->M, m->V, m->grad, m->loss, m->W1b, m->W2b, m->W2t, m->W3b, m->partial, m->act, m->row_loss,
                     m->X, m->y, m->perm, m->cls, m->logits};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
@@ -845,7 +832,7 @@ int amr_mlp_set_params(amr_mlp_t *m, const float *params)
     MCHK(hipMemset(m->M, 0, sizeof(float) * NP));
     MCHK(hipMemset(m->V, 0, sizeof(float) * NP));
     hipLaunchKernelGGL(bf16_copy_kernel, dim3((NP + 255) / 256), dim3(256), 0, m->stream, m->P, m->W1b, m->W2b,
-                       m->W3b);
+                       m->W2t, m->W3b);
     MCHK(hipGetLastError());
     MCHK(hipStreamSynchronize(m->stream));
     m->step = 0;

@@ -74,3 +74,29 @@ def test_features_at_the_edges_of_the_quotient(oracle, case):
     exp = oracle.tagger_features(8, ci, fi, soln)
     assert np.array_equal(g.tagger_features(), exp)
     g.close()
+
+
+@pytest.mark.parametrize("batch", [64, 2176, 4096, 6208])
+def test_training_step_follows_the_gradient(batch):
+    """minibatches whose partial sums span one, two and three chunks, the last
+    one of 6208 rows part empty: from zero moments Adam moves every parameter
+    by lr against its gradient's sign (the step is lr g / (|g| + eps)), and the
+    loss it reports is the gradient call's"""
+    from test_tagger_oracle import random_problem
+    P, X, y, cw = random_problem(90, n=batch)
+    m, lr = amrhip.Mlp(0), 1e-3
+    m.set_params(P)
+    loss, g = m.grad(X, y, cw)
+    ts = amrhip.Tagset()
+    ts.append(X, y)
+    losses = m.train(ts, epochs=1, batch=batch, lr=lr, cw=cw, seed=1)
+    step = m.params() - P
+    # the two sum in other orders: FP32 sums of `batch` terms differ by a few
+    # parts in 1e6 of the largest, so a gradient over 1e-3 of its block's
+    # largest keeps its sign; the step is exact to the rounding of P
+    big = np.abs(g) > 1e-3 * np.abs(g).max()
+    assert big.sum() > 500
+    assert np.allclose(step[big], -lr * np.sign(g[big]), rtol=0, atol=1e-6 + 2.0 ** -23 * np.abs(P).max())
+    assert abs(losses[0] - loss) <= 1e-5 * abs(loss)
+    m.close()
+    ts.close()
