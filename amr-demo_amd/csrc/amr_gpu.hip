@@ -24,6 +24,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "amr_hip.h"
@@ -91,8 +92,15 @@ struct StageArgs {
     int mode;
     int first;           // first stage of an accumulating scheme
     int role;            // ROLE_CFL: the stage folds the next step's CFL minimum
-    const double *dt_cur;// ninst: the step's dt (dt_prep_kernel)
-    unsigned long long *slot;
+    double *dt_cur;      // ninst: the step's dt (dt_prep_kernel, or the step's first stage)
+    unsigned long long *slot;      // CFL sub-slots that ROLE_CFL fills
+    // a first stage that forms the step's dt itself (SELF kernels; else null):
+    const unsigned long long *slot_in;   // the current state's CFL sub-slots
+    unsigned long long *slot_clear;      // to be empty when the next step fills them
+    const double *t_in;  // ninst: time at the start of the step
+    double *t_out;       // ninst: time at its end
+    double *t_step;      // MeshDev's, for the step's other stages
+    int use_cfl;
     double *norm_part;
     int per_block;       // persistent design: patches per workgroup (a contiguous range)
 };
@@ -379,16 +387,16 @@ template <int BLK>
 __device__ void cfl_reduce(double cand, int inst, bool active, int uinst,
                            unsigned long long *slot, double *red)
 {
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, sub = blockIdx.x & (NSLOT - 1);
     if (uinst < 0) {
-        if (active) atomicMin(&slot[inst * NSLOT + (blockIdx.x & (NSLOT - 1))], d2bits(cand));
+        if (active) atomicMin(&slot[inst * NSLOT + sub], d2bits(cand));
         return;
     }
     double v = active ? cand : INFINITY;
     v = wave_min(v);
     constexpr int NW = (BLK + 63) / 64;
     if (NW == 1) {
-        if (tid == 0) atomicMin(&slot[uinst * NSLOT + (blockIdx.x & (NSLOT - 1))], d2bits(v));
+        if (tid == 0) atomicMin(&slot[uinst * NSLOT + sub], d2bits(v));
         return;
     }
     __syncthreads();
@@ -397,7 +405,7 @@ __device__ void cfl_reduce(double cand, int inst, bool active, int uinst,
     if (tid == 0) {
         double m = red[0];
         for (int w = 1; w < NW; ++w) m = fmin(m, red[w]);
-        atomicMin(&slot[uinst * NSLOT + (blockIdx.x & (NSLOT - 1))], d2bits(m));
+        atomicMin(&slot[uinst * NSLOT + sub], d2bits(m));
     }
 }
 
@@ -415,6 +423,33 @@ __device__ void sum_reduce_store(double v, double *out, double *red)
         for (int w = 1; w < NW; ++w) s += red[w];
         *out = s;
     }
+}
+
+// All-reduce within aligned groups of W lanes by DPP moves (no LDS round
+// trips): pairs, quads, then each half-row and row against its mirror image;
+// the four rows of a whole wave as scalars.
+template <int W, class Op>
+__device__ __forceinline__ double group_reduce(double v, Op op)
+{
+    if (W >= 2) v = op(v, dpp_f64<0xB1>(v));     // quad_perm 1,0,3,2
+    if (W >= 4) v = op(v, dpp_f64<0x4E>(v));     // quad_perm 2,3,0,1
+    if (W >= 8) v = op(v, dpp_f64<0x141>(v));    // row_half_mirror
+    if (W >= 16) v = op(v, dpp_f64<0x140>(v));   // row_mirror
+    if (W >= 64) v = op(op(lane_f64(v, 0), lane_f64(v, 16)), op(lane_f64(v, 32), lane_f64(v, 48)));
+    return v;
+}
+
+// dt of the step: min(input dt, CFL minimum, time left).
+__device__ __forceinline__ double limited_dt(double dt_cap, double t_end, double cfl_min, double t, int use_cfl)
+{
+    double dt = dt_cap;
+    if (use_cfl && cfl_min < dt) dt = cfl_min;
+    if (t_end > 0.0) {
+        double rem = t_end - t;
+        if (rem < 0.0) rem = 0.0;
+        if (rem < dt) dt = rem;
+    }
+    return dt;
 }
 
 // CFL minimum of instance inst over its sub-slots; called by a whole wave
@@ -435,17 +470,24 @@ __device__ __forceinline__ double slot_min(const unsigned long long *slot, int i
 __device__ __forceinline__ double step_dt(const InstDev &ip, const unsigned long long *slot,
                                           const double *t_inst, int inst, int use_cfl)
 {
-    double dt = ip.dt_cap;
-    if (use_cfl) {
-        double c = slot_min(slot, inst);
-        if (c < dt) dt = c;
+    const double c = use_cfl ? slot_min(slot, inst) : INFINITY;
+    return limited_dt(ip.dt_cap, ip.t_end, c, t_inst[inst], use_cfl);
+}
+
+// The bookkeeping of a step's dt by its first stage, by a whole wave that holds
+// the first quadrant of a run of the instance's quadrants (all such waves write
+// the same): dt and start time for the step's other stages, the time at its end,
+// and the sub-slots that the next step fills emptied.
+__device__ __forceinline__ void publish_dt(const StageArgs &a, int inst, double dt, double t)
+{
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) {
+        a.dt_cur[inst] = dt;
+        a.t_step[inst] = t;
+        a.t_out[inst] = t + dt;
     }
-    if (ip.t_end > 0.0) {
-        double rem = ip.t_end - t_inst[inst];
-        if (rem < 0.0) rem = 0.0;
-        if (rem < dt) dt = rem;
-    }
-    return dt;
+#pragma unroll
+    for (int k = 0; k < NSLOT / 64; ++k) a.slot_clear[(size_t)inst * NSLOT + lane + 64 * k] = DBL_INF_BITS;
 }
 
 // ---------------------------------------------------------------------------
@@ -613,7 +655,8 @@ __device__ __forceinline__ void stage_update(const StageArgs &a, size_t base, in
     }
 }
 
-template <int N, int PPB, int MINW, int DESIGN>
+// SELF: the first stage of a step without dt_prep_kernel (one-patch tiles).
+template <int N, int PPB, int MINW, int DESIGN, bool SELF = false>
 __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(StageArgs a)
 {
     using TL = Tile<N, PPB>;
@@ -744,9 +787,16 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
         const cinst4 *ipc = (const cinst4 *)a.m.ip;
         hw = actw ? ldexp(ipc[inw].h_base, -levw) / (double)N : 0.0;
         // the step's dt and start time, written by the step's prep kernel
-        dtw = actw && a.mode != MODE_RHS ? ((const cdbl4 *)a.dt_cur)[inw] : 0.0;
-        const double tw = actw ? ((const cdbl4 *)a.m.t_step)[inw] : 0.0;
+        static_assert(!SELF || SMETA, "one paired-face patch per workgroup");
+        if (!SELF) dtw = actw && a.mode != MODE_RHS ? ((const cdbl4 *)a.dt_cur)[inw] : 0.0;
+        const double tw = actw ? ((const cdbl4 *)(SELF ? a.t_in : a.m.t_step))[inw] : 0.0;
         tpw = tw;
+        if constexpr (SELF) {
+            typedef const int __attribute__((address_space(4))) cint4;
+            const double c = a.use_cfl ? slot_min(a.slot_in, inw) : INFINITY;
+            dtw = uniform_f64(limited_dt(ipc[inw].dt_cap, ipc[inw].t_end, c, tw, a.use_cfl));
+            if (tid < 64 && (lb == 0 || ((const cint4 *)a.m.inst)[lb - 1] != inw)) publish_dt(a, inw, dtw, tw);
+        }
         if (!SMETA && c == 0) {
             pquad[p] = actw ? lb * PPB + p : -1;
             plevel[p] = levw;
@@ -1530,7 +1580,8 @@ __device__ __forceinline__ unsigned here(unsigned v)
     return v;
 }
 
-template <int N, int R, int VEC>
+// SELF: the first stage of a step without dt_prep_kernel.
+template <int N, int R, int VEC, bool SELF = false>
 __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
 {
     constexpr int N2 = N * N, P = 64 / (N * R), STEPS = N / R, QS = NFLD * N2;
@@ -1611,7 +1662,22 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
             cell_load((size_t)(nb[j].y < 0 ? tq[j] : nb[j].y) * QS + edge(j, !is_high(j)), sec[j]);
     }
     const double h = ldexp(a.m.ip[inst].h_base, -lev) / (double)N;
-    const double dt = a.mode != MODE_RHS ? a.dt_cur[inst] : 0.0;
+    double dt = 0.0;
+    if (!SELF && a.mode != MODE_RHS) dt = a.dt_cur[inst];
+    const double *const t_step = SELF ? a.t_in : a.m.t_step;
+    if (SELF) {
+        // an instance of the wave at a time, nearly always the only one
+        const bool lead = active && (quad == 0 || a.m.inst[quad - 1] != inst);
+        unsigned long long todo = __ballot(true);
+        do {
+            const int i = __builtin_amdgcn_readlane(inst, __ffsll(todo) - 1);
+            const double c = a.use_cfl ? slot_min(a.slot_in, i) : INFINITY, t = a.t_in[i];
+            const double d = limited_dt(a.m.ip[i].dt_cap, a.m.ip[i].t_end, c, t, a.use_cfl);
+            if (__any(lead && inst == i)) publish_dt(a, i, d, t);
+            if (inst == i) dt = d;
+            todo &= ~__ballot(inst == i);
+        } while (todo);
+    }
     const double ninvV = ldexp(a.m.ip[inst].ninv_vol0, 2 * lev);
 
     auto put_rec = [&](int t, const Rec &c) {
@@ -1674,7 +1740,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
                 const double nrm[2] = {y ? 0.0 : nh, y ? nh : 0.0};
                 double F[4];
                 flux_boundary(a.m.ip[tinst], 2 * y + high, nrm, own[j], a.m.org + 2 * (size_t)tq[j],
-                              y ? tk[j] + 0.5 : fe, y ? fe : tk[j] + 0.5, th, a.m.t_step[tinst], F);
+                              y ? tk[j] + 0.5 : fe, y ? fe : tk[j] + 0.5, th, t_step[tinst], F);
 #pragma unroll
                 for (int f = 0; f < 4; ++f) d[f * NE] = high ? F[f] : -F[f];
             }
@@ -1837,7 +1903,8 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
 // Standalone CFL minimum (physics_time_step): one thread per cell.
 template <int N, int PPB>
 __global__ __launch_bounds__((Tile<N, PPB>::BLK)) void cfl_kernel(MeshDev m, const double *U,
-                                                                unsigned long long *slot)
+                                                                unsigned long long *slot,
+                                                                unsigned long long *clear)
 {
     using TL = Tile<N, PPB>;
     constexpr int N2 = TL::N2;
@@ -1870,11 +1937,15 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK)) void cfl_kernel(MeshDev m, con
         cand = cfl_candidate(q, m.ip[inst].cfl, h * h);
     }
     cfl_reduce<TL::BLK>(cand, inst, active, uinst, slot, red);
+    // other sub-slots emptied on the way (those that the first step fills)
+    if (clear)
+        for (int i = blockIdx.x * TL::BLK + tid; i < m.ninst * NSLOT; i += gridDim.x * TL::BLK) clear[i] = DBL_INF_BITS;
 }
 
 __global__ void slot_reset_kernel(unsigned long long *slot, int ninst)
 {
-    for (int i = threadIdx.x; i < ninst * NSLOT; i += blockDim.x) slot[i] = DBL_INF_BITS;
+    const int n = ninst * NSLOT;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) slot[i] = DBL_INF_BITS;
 }
 
 // The step's dt and time update, ahead of its first stage: one wave per
@@ -1914,20 +1985,6 @@ __global__ void soa_to_aos_kernel(const double *soa, double *aos, long long ncel
     double *d = aos + t * NFLD;
 #pragma unroll
     for (int f = 0; f < 4; ++f) d[f] = soa[(q * NFLD + f) * n2 + c];
-}
-
-// All-reduce within aligned groups of W lanes by DPP moves (no LDS round
-// trips): pairs, quads, then each half-row and row against its mirror image;
-// the four rows of a whole wave as scalars.
-template <int W, class Op>
-__device__ __forceinline__ double group_reduce(double v, Op op)
-{
-    if (W >= 2) v = op(v, dpp_f64<0xB1>(v));     // quad_perm 1,0,3,2
-    if (W >= 4) v = op(v, dpp_f64<0x4E>(v));     // quad_perm 2,3,0,1
-    if (W >= 8) v = op(v, dpp_f64<0x141>(v));    // row_half_mirror
-    if (W >= 16) v = op(v, dpp_f64<0x140>(v));   // row_mirror
-    if (W >= 64) v = op(op(lane_f64(v, 0), lane_f64(v, 16)), op(lane_f64(v, 32), lane_f64(v, 48)));
-    return v;
 }
 
 // Project-defined density-gradient indicator: the largest
@@ -2117,14 +2174,26 @@ struct amrgpu_ctx {
     InstDev *d_ip = nullptr;
     double *U[3] = {nullptr, nullptr, nullptr};
     double *Acc = nullptr;
-    double *d_dt_cur = nullptr, *d_t = nullptr;
-    unsigned long long *d_slot = nullptr;
+    // per-instance clocks, cap_inst each in one allocation: the time (two, by
+    // tb: a step of self_dt reads one and writes the other), the last dt, the
+    // time at the step start
+    double *d_clock = nullptr;
+    unsigned long long *d_slot_sets = nullptr; // three sets of CFL sub-slots, by sb
+    int tb = 0, sb = 0;
+    bool self_dt = false;                      // this run's steps have no dt_prep_kernel
+    bool all_inst = true;                      // every instance has quadrants
+    double *t_now(int ahead = 0) const { return d_clock + (size_t)((tb + ahead) & 1) * cap_inst; }
+    double *dt_cur() const { return d_clock + (size_t)2 * cap_inst; }
+    double *t_step() const { return d_clock + (size_t)3 * cap_inst; }
+    unsigned long long *slots(int ahead = 0) const
+    {
+        return d_slot_sets + (size_t)((sb + ahead) % 3) * cap_inst * NSLOT;
+    }
     double *d_norm = nullptr;
     double *d_stage = nullptr;      // AoS staging for up/download
     int *d_map = nullptr;           // regrid source map
     double *d_ind = nullptr;        // per-quadrant indicator
     double *d_org = nullptr;        // per-quadrant lower-left corner
-    double *d_tstep = nullptr;      // per-instance time at the step start
     bool org_ok = false, need_org = false;
     int nblocks = 0;
     int variant = -1;
@@ -2152,7 +2221,7 @@ MeshDev mesh_of(const amrgpu_ctx *c)
     MeshDev m;
     m.nquad = c->nquad; m.ninst = c->ninst;
     m.nbr = c->d_nbr; m.level = c->d_level; m.inst = c->d_inst; m.ip = c->d_ip;
-    m.org = c->d_org; m.t_step = c->d_tstep;
+    m.org = c->d_org; m.t_step = c->t_step();
     return m;
 }
 
@@ -2202,8 +2271,9 @@ int grid_of(const amrgpu_ctx *c, int v, int nquad)
 
 // Stage-kernel tile used until amrgpu_set_tile / amrgpu_autotune picks one
 // (every tile computes the same bits): for n = 8 and 16 the paired-faces
-// tile with one patch per workgroup, four and five waves per SIMD, the
-// fastest or within 2 % of it on the meshes measured (207k to 16.8M cells).
+// tile with one patch per workgroup and five waves per SIMD, the fastest or
+// within 2 % of it on the meshes measured (1k to 16.8M cells; four waves at 8x8:
+// 4096 quadrants 28.0 against 26.9 us a step, 18750 94.5 against 90.2).
 // n = 2 and 4: the row-marching kernel, faster than the others at every size
 // measured (16 to 262k quadrants).  n = 4 takes two rows a step, with fewer
 // instructions a patch, where its waves of 8 patches fill the chip (256 CUs x
@@ -2214,7 +2284,7 @@ int default_variant(int n, int nquad)
     switch (n) {
     case 2: return 20;
     case 4: return nquad < 20000 ? 21 : 22;
-    case 8: return 15;
+    case 8: return 17;
     case 16: return 19;
     default: return -1;
     }
@@ -2249,6 +2319,13 @@ template <int N, int PPB, int MINW, int D>
 int launch_v(amrgpu_ctx *c, const StageArgs &a)
 {
     int nblk = (c->nquad + PPB - 1) / PPB;
+    if constexpr (D == 1 && PPB == 1 && MINW >= 4) {
+        if (a.slot_in) {
+            hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D, true>), dim3(nblk), dim3(Tile<N, PPB>::BLK), 0, c->stream, a);
+            HIPCHK(hipGetLastError());
+            return AMRGPU_OK;
+        }
+    }
     hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D>), dim3(nblk), dim3(Tile<N, PPB>::BLK), 0, c->stream, a);
     HIPCHK(hipGetLastError());
     return AMRGPU_OK;
@@ -2259,12 +2336,14 @@ int launch_rows(amrgpu_ctx *c, const StageArgs &a)
 {
     constexpr int P = 64 / (N * R);
     const dim3 nblk((c->nquad + P - 1) / P);
-    if (a.mode == MODE_LSERK)
-        hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC_ACC>), nblk, dim3(64), 0, c->stream, a);
-    else if (a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL)
-        hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC_BOTH>), nblk, dim3(64), 0, c->stream, a);
-    else
-        hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC_BASE>), nblk, dim3(64), 0, c->stream, a);
+    auto go = [&](auto vec) {
+        constexpr int VEC = decltype(vec)::value;
+        if (a.slot_in) hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC, true>), nblk, dim3(64), 0, c->stream, a);
+        else hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC>), nblk, dim3(64), 0, c->stream, a);
+    };
+    if (a.mode == MODE_LSERK) go(std::integral_constant<int, VEC_ACC>());
+    else if (a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL) go(std::integral_constant<int, VEC_BOTH>());
+    else go(std::integral_constant<int, VEC_BASE>());
     HIPCHK(hipGetLastError());
     return AMRGPU_OK;
 }
@@ -2299,16 +2378,17 @@ int launch_stage(amrgpu_ctx *c, const StageArgs &a)
     }
 }
 
-int launch_cfl(amrgpu_ctx *c, const double *U)
+// CFL minimum of the state U into the sub-slots `slot` (empty before).
+int launch_cfl(amrgpu_ctx *c, const double *U, unsigned long long *slot, unsigned long long *clear)
 {
-    int ppb = ppb_of(c->n);
-    int nblk = (c->nquad + ppb - 1) / ppb;
+    const int ppb = ppb_of(c->n);
+    const dim3 nblk((c->nquad + ppb - 1) / ppb);
     MeshDev m = mesh_of(c);
     switch (c->n) {
-    case 2: hipLaunchKernelGGL((cfl_kernel<2, 16>), dim3(nblk), dim3(64), 0, c->stream, m, U, c->d_slot); break;
-    case 4: hipLaunchKernelGGL((cfl_kernel<4, 8>), dim3(nblk), dim3(128), 0, c->stream, m, U, c->d_slot); break;
-    case 8: hipLaunchKernelGGL((cfl_kernel<8, 4>), dim3(nblk), dim3(256), 0, c->stream, m, U, c->d_slot); break;
-    case 16: hipLaunchKernelGGL((cfl_kernel<16, 1>), dim3(nblk), dim3(256), 0, c->stream, m, U, c->d_slot); break;
+    case 2: hipLaunchKernelGGL((cfl_kernel<2, 16>), nblk, dim3(64), 0, c->stream, m, U, slot, clear); break;
+    case 4: hipLaunchKernelGGL((cfl_kernel<4, 8>), nblk, dim3(128), 0, c->stream, m, U, slot, clear); break;
+    case 8: hipLaunchKernelGGL((cfl_kernel<8, 4>), nblk, dim3(256), 0, c->stream, m, U, slot, clear); break;
+    case 16: hipLaunchKernelGGL((cfl_kernel<16, 1>), nblk, dim3(256), 0, c->stream, m, U, slot, clear); break;
     default: set_err("unsupported nelem_subgrid %d", c->n); return AMRGPU_ERR_ARG;
     }
     HIPCHK(hipGetLastError());
@@ -2337,8 +2417,8 @@ StageArgs base_args(amrgpu_ctx *c)
     StageArgs a;
     memset(&a, 0, sizeof(a));
     a.m = mesh_of(c);
-    a.dt_cur = c->d_dt_cur;
-    a.slot = c->d_slot;
+    a.dt_cur = c->dt_cur();
+    a.slot = c->slots();
     return a;
 }
 
@@ -2405,18 +2485,58 @@ int build_step(amrgpu_ctx *c, int cur, std::vector<StageArgs> &st, bool with_nor
     }
 }
 
+// Tiles whose first stage can form the step's dt itself.
+bool has_self(int v)
+{
+    return kVariants[v].design == 3 || (kVariants[v].design == 1 && kVariants[v].ppb == 1 && kVariants[v].minw >= 4);
+}
+
+// Whether the steps of a run have no dt_prep_kernel.  That saves a launch and its
+// gap, 1.6-2 us a step; every first-stage wave reduces its instance's sub-slots
+// instead (four loads a lane beside the halo's), so meshes of many waves keep the
+// kernel.  us per SSP-RK3 step with / without it, one problem each: 8x8, 256
+// quadrants 15.3 / 13.6, 4137 30.1 / 28.9, 18750 93.7 / 90.2, 41170 180.5 / 182.8;
+// 16x16, 256 17.4 / 15.7, 4455 83.3 / 83.1, 7159 122.6 / 125.9; the row-marching
+// tiles, whose waves hold several patches: 4x4, 1024 14.0 / 12.2, 16384 30.5 /
+// 29.1, 65536 84.8 / 85.8; 2x2, 37750 35.5 / 34.6, 65536 36.1 / 36.9.
+bool wants_self(const amrgpu_ctx *c)
+{
+    const TileVariant &v = kVariants[c->variant];
+    const long long waves = (long long)c->nblocks * (v.design == 1 ? std::max(1, v.n * v.n / 64) : 1);
+    return !c->graphs_enabled && c->all_inst && has_self(c->variant) && waves <= (v.design == 1 ? 20000 : 4000);
+}
+
+// The step's dt: a kernel ahead of its first stage, or that stage's own.
+int begin_step(amrgpu_ctx *c, std::vector<StageArgs> &st)
+{
+    if (!c->self_dt) {
+        hipLaunchKernelGGL(dt_prep_kernel, dim3(std::max(1, c->ninst)), dim3(64), 0, c->stream, mesh_of(c),
+                           c->scheme != 2, c->dt_cur(), c->t_now(), c->t_step(), c->slots());
+        HIPCHK(hipGetLastError());
+        return AMRGPU_OK;
+    }
+    StageArgs &f = st.front();
+    f.slot_in = c->slots();
+    f.slot_clear = c->slots(2);
+    f.t_in = c->t_now();
+    f.t_out = c->t_now(1);
+    f.t_step = c->t_step();
+    f.use_cfl = c->scheme != 2;
+    for (auto &a : st) a.slot = c->slots(1);
+    c->tb ^= 1;
+    c->sb = (c->sb + 1) % 3;
+    return AMRGPU_OK;
+}
+
 int enqueue_step(amrgpu_ctx *c, int cur, bool with_norm, int *next)
 {
     std::vector<StageArgs> st;
     int nx = build_step(c, cur, st, with_norm);
     if (nx < 0) { set_err("bad time scheme %d", c->scheme); return AMRGPU_ERR_ARG; }
-    hipLaunchKernelGGL(dt_prep_kernel, dim3(std::max(1, c->ninst)), dim3(64), 0, c->stream, mesh_of(c),
-                       c->scheme != 2, c->d_dt_cur, c->d_t, c->d_tstep, c->d_slot);
-    HIPCHK(hipGetLastError());
-    for (auto &a : st) {
-        int rc = launch_stage(c, a);
-        if (rc) return rc;
-    }
+    int rc = begin_step(c, st);
+    if (rc) return rc;
+    for (auto &a : st)
+        if ((rc = launch_stage(c, a))) return rc;
     *next = nx;
     return AMRGPU_OK;
 }
@@ -2432,14 +2552,14 @@ void free_mesh(amrgpu_ctx *c)
     free_graphs(c);
     (void)hipFree(c->d_nbr); (void)hipFree(c->d_level); (void)hipFree(c->d_inst); (void)hipFree(c->d_ip);
     for (int i = 0; i < 3; ++i) (void)hipFree(c->U[i]);
-    (void)hipFree(c->Acc); (void)hipFree(c->d_dt_cur); (void)hipFree(c->d_t); (void)hipFree(c->d_slot);
+    (void)hipFree(c->Acc); (void)hipFree(c->d_clock); (void)hipFree(c->d_slot_sets);
     (void)hipFree(c->d_norm); (void)hipFree(c->d_stage);
-    (void)hipFree(c->d_map); (void)hipFree(c->d_ind); (void)hipFree(c->d_org); (void)hipFree(c->d_tstep);
-    c->d_map = nullptr; c->d_ind = nullptr; c->d_org = nullptr; c->d_tstep = nullptr;
+    (void)hipFree(c->d_map); (void)hipFree(c->d_ind); (void)hipFree(c->d_org);
+    c->d_map = nullptr; c->d_ind = nullptr; c->d_org = nullptr;
     c->org_ok = false;
     c->d_nbr = c->d_level = c->d_inst = nullptr; c->d_ip = nullptr;
     c->U[0] = c->U[1] = c->U[2] = nullptr; c->Acc = nullptr;
-    c->d_dt_cur = c->d_t = nullptr; c->d_slot = nullptr; c->d_norm = nullptr;
+    c->d_clock = nullptr; c->d_slot_sets = nullptr; c->d_norm = nullptr;
     c->d_stage = nullptr;
     c->nquad = 0;
     c->cap_quad = c->cap_inst = c->cap_blocks = 0;
@@ -2580,6 +2700,14 @@ static int validate_cells(int n2, int ninst, int ncell, const int *cell_info, co
     return AMRGPU_OK;
 }
 
+// Every set of CFL sub-slots empty: where the instances change.
+static int empty_slots(amrgpu_ctx *c)
+{
+    hipLaunchKernelGGL(slot_reset_kernel, dim3(16), dim3(256), 0, c->stream, c->d_slot_sets, 3 * c->cap_inst);
+    HIPCHK(hipGetLastError());
+    return AMRGPU_OK;
+}
+
 // Buffers are kept across setups and remeshes (an adaptive run changes the
 // mesh once per regrid interval) and grown with 25% headroom when the mesh
 // outgrows them.  *fresh tells whether they were reallocated.
@@ -2607,15 +2735,14 @@ static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need
     HIPCHK(hipMalloc(&c->d_ip, sizeof(InstDev) * c->cap_inst));
     for (int i = 0; i < 3; ++i) HIPCHK(hipMalloc(&c->U[i], sizeof(double) * (cs + pad)));
     if (need_acc) HIPCHK(hipMalloc(&c->Acc, sizeof(double) * (cs + pad)));
-    HIPCHK(hipMalloc(&c->d_dt_cur, sizeof(double) * c->cap_inst));
-    HIPCHK(hipMalloc(&c->d_t, sizeof(double) * c->cap_inst));
-    HIPCHK(hipMalloc(&c->d_slot, sizeof(unsigned long long) * c->cap_inst * NSLOT));
+    HIPCHK(hipMalloc(&c->d_clock, sizeof(double) * 4 * c->cap_inst));
+    HIPCHK(hipMalloc(&c->d_slot_sets, sizeof(unsigned long long) * 3 * c->cap_inst * NSLOT));
+    if (int rc = empty_slots(c)) return rc;
     HIPCHK(hipMalloc(&c->d_norm, sizeof(double) * c->cap_blocks));
     HIPCHK(hipMalloc(&c->d_stage, sizeof(double) * cs));
     HIPCHK(hipMalloc(&c->d_map, sizeof(int) * cq));
     HIPCHK(hipMalloc(&c->d_ind, sizeof(double) * cq));
     HIPCHK(hipMalloc(&c->d_org, sizeof(double) * 2 * cq));
-    HIPCHK(hipMalloc(&c->d_tstep, sizeof(double) * c->cap_inst));
     return AMRGPU_OK;
 }
 
@@ -2656,6 +2783,12 @@ static int upload_mesh(amrgpu_ctx *c, int ncell, const int *level, const int *ce
     if (cell_inst) memcpy(pq, cell_inst, sizeof(int) * (size_t)ncell);
     else memset(pq, 0, sizeof(int) * (size_t)ncell);
     c->nquad = ncell;
+    c->all_inst = c->ninst == 1;
+    if (cell_inst && c->ninst > 1) {
+        std::vector<char> has(c->ninst, 0);
+        for (int q = 0; q < ncell; ++q) has[cell_inst[q]] = 1;
+        c->all_inst = std::find(has.begin(), has.end(), 0) == has.end();
+    }
     if (!c->tile_chosen || kVariants[c->variant].n != c->n) {
         c->variant = default_variant(c->n, ncell);
         c->tile_chosen = false;
@@ -2706,6 +2839,7 @@ int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
     free_graphs(c);
     bool fresh;
     rc = ensure_capacity(c, nelem_subgrid, ncell, ninst, time_scheme == 4 || time_scheme == 5, &fresh);
+    if (!rc && !fresh) rc = empty_slots(c);
     if (rc) return rc;
     c->n = nelem_subgrid; c->ninst = ninst; c->scheme = time_scheme;
     c->cur = 0;
@@ -2733,9 +2867,9 @@ int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
     }
     HIPCHK(hipMemcpyAsync(c->d_ip, c->h_ip.data(), sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
     std::vector<double> zeros(ninst, 0.0);
-    HIPCHK(hipMemcpyAsync(c->d_t, zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d_tstep, zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d_dt_cur, zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->t_now(), zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->t_step(), zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->dt_cur(), zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
     rc = upload_mesh(c, ncell, levels_of(ncell, cell_info).data(), cell_inst, nbr.data());
     if (rc) return rc;
     c->org_ok = false;
@@ -2843,9 +2977,9 @@ static int remesh_to(amrgpu_ctx *c, int ncell, const int *level, const int *cell
         double *keep = nullptr;
         int *map = nullptr;
         std::vector<double> t(c->ninst), dt(c->ninst), ts(c->ninst);
-        HIPCHK(hipMemcpyAsync(t.data(), c->d_t, sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipMemcpyAsync(dt.data(), c->d_dt_cur, sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipMemcpyAsync(ts.data(), c->d_tstep, sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipMemcpyAsync(t.data(), c->t_now(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipMemcpyAsync(dt.data(), c->dt_cur(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipMemcpyAsync(ts.data(), c->t_step(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipMalloc(&keep, sizeof(double) * old_state));
         HIPCHK(hipMalloc(&map, sizeof(int) * ncell));
         HIPCHK(hipMemcpyAsync(keep, c->U[c->cur], sizeof(double) * old_state, hipMemcpyDeviceToDevice, c->stream));
@@ -2856,9 +2990,9 @@ static int remesh_to(amrgpu_ctx *c, int ncell, const int *level, const int *cell
         rc = ensure_capacity(c, c->n, ncell + ncell / 2, ninst, c->scheme == 4 || c->scheme == 5, &fresh);
         if (rc) { (void)hipFree(keep); (void)hipFree(map); return rc; }
         HIPCHK(hipMemcpyAsync(c->d_ip, c->h_ip.data(), sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->d_t, t.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->d_dt_cur, dt.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->d_tstep, ts.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipMemcpyAsync(c->t_now(), t.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipMemcpyAsync(c->dt_cur(), dt.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipMemcpyAsync(c->t_step(), ts.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
         hipLaunchKernelGGL(remap_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
                            keep, c->U[0], map, ncells, n2);
         HIPCHK(hipGetLastError());
@@ -2880,12 +3014,12 @@ static int remesh_to(amrgpu_ctx *c, int ncell, const int *level, const int *cell
         for (int i = 0; i < c->ninst; ++i) empty = empty || !has[i];
         if (empty) {
             std::vector<double> dt(c->ninst);
-            HIPCHK(hipMemcpyAsync(dt.data(), c->d_dt_cur, sizeof(double) * c->ninst, hipMemcpyDeviceToHost,
+            HIPCHK(hipMemcpyAsync(dt.data(), c->dt_cur(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost,
                                   c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
             for (int i = 0; i < c->ninst; ++i)
                 if (!has[i]) dt[i] = 0.0;
-            HIPCHK(hipMemcpyAsync(c->d_dt_cur, dt.data(), sizeof(double) * c->ninst, hipMemcpyHostToDevice,
+            HIPCHK(hipMemcpyAsync(c->dt_cur(), dt.data(), sizeof(double) * c->ninst, hipMemcpyHostToDevice,
                                   c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
         }
@@ -3045,12 +3179,12 @@ int amrgpu_rhs(amrgpu_ctx *c, double *rhs)
 int amrgpu_cfl(amrgpu_ctx *c, double *dt_inst)
 {
     if (!c || !dt_inst || !c->nquad) { set_err("amrgpu_cfl: no mesh"); return AMRGPU_ERR_ARG; }
-    hipLaunchKernelGGL(slot_reset_kernel, dim3(1), dim3(256), 0, c->stream, c->d_slot, c->ninst);
+    hipLaunchKernelGGL(slot_reset_kernel, dim3(1), dim3(256), 0, c->stream, c->slots(), c->ninst);
     HIPCHK(hipGetLastError());
-    int rc = launch_cfl(c, c->U[c->cur]);
+    int rc = launch_cfl(c, c->U[c->cur], c->slots(), nullptr);
     if (rc) return rc;
     std::vector<unsigned long long> b((size_t)c->ninst * NSLOT);
-    HIPCHK(hipMemcpyAsync(b.data(), c->d_slot, sizeof(unsigned long long) * b.size(), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(b.data(), c->slots(), sizeof(unsigned long long) * b.size(), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     for (int i = 0; i < c->ninst; ++i) {
         unsigned long long mn = DBL_INF_BITS;
@@ -3063,10 +3197,18 @@ int amrgpu_cfl(amrgpu_ctx *c, double *dt_inst)
 static int prime_run(amrgpu_ctx *c)
 {
     if (int rc = geometry_ready(c)) return rc;
-    // CFL slot of the current state for the first step's dt
-    hipLaunchKernelGGL(slot_reset_kernel, dim3(1), dim3(256), 0, c->stream, c->d_slot, c->ninst);
+    // CFL sub-slots of the current state for the first step's dt
+    c->self_dt = wants_self(c);
+    if (c->self_dt) {
+        // of the three sets the next one is empty; the one after it, which the
+        // last step read, is emptied on the way for the first step to fill
+        if (c->scheme == 2) return AMRGPU_OK;
+        c->sb = (c->sb + 1) % 3;
+        return launch_cfl(c, c->U[c->cur], c->slots(), c->slots(1));
+    }
+    hipLaunchKernelGGL(slot_reset_kernel, dim3(1), dim3(256), 0, c->stream, c->slots(), c->ninst);
     HIPCHK(hipGetLastError());
-    if (c->scheme != 2) return launch_cfl(c, c->U[c->cur]);
+    if (c->scheme != 2) return launch_cfl(c, c->U[c->cur], c->slots(), nullptr);
     return AMRGPU_OK;
 }
 
@@ -3142,8 +3284,8 @@ int amrgpu_run(amrgpu_ctx *c, int nsteps, int use_graph, double *resnorm)
 int amrgpu_get_time(amrgpu_ctx *c, double *t_inst, double *dt_inst)
 {
     if (!c || !c->nquad) { set_err("amrgpu_get_time: no mesh"); return AMRGPU_ERR_ARG; }
-    if (t_inst) HIPCHK(hipMemcpyAsync(t_inst, c->d_t, sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
-    if (dt_inst) HIPCHK(hipMemcpyAsync(dt_inst, c->d_dt_cur, sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
+    if (t_inst) HIPCHK(hipMemcpyAsync(t_inst, c->t_now(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
+    if (dt_inst) HIPCHK(hipMemcpyAsync(dt_inst, c->dt_cur(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return AMRGPU_OK;
 }
@@ -3151,8 +3293,8 @@ int amrgpu_get_time(amrgpu_ctx *c, double *t_inst, double *dt_inst)
 int amrgpu_set_time(amrgpu_ctx *c, const double *t_inst)
 {
     if (!c || !c->nquad || !t_inst) { set_err("amrgpu_set_time: no mesh"); return AMRGPU_ERR_ARG; }
-    HIPCHK(hipMemcpyAsync(c->d_t, t_inst, sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d_tstep, t_inst, sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->t_now(), t_inst, sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->t_step(), t_inst, sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return AMRGPU_OK;
 }
@@ -3199,8 +3341,7 @@ int amrgpu_bench(amrgpu_ctx *c, int nsteps, double *ms_total, double *avg_stage_
     // per-stage kernel durations: direct launches bracketed by events
     for (int s = 0; s < nsteps; ++s) {
         int nx = build_step(c, c->cur, st, false);
-        hipLaunchKernelGGL(dt_prep_kernel, dim3(std::max(1, c->ninst)), dim3(64), 0, c->stream, mesh_of(c),
-                           c->scheme != 2, c->d_dt_cur, c->d_t, c->d_tstep, c->d_slot);
+        if ((rc = begin_step(c, st))) return rc;
         HIPCHK(hipEventRecord(ev[(size_t)s * (ns + 1)], c->stream));
         for (int k = 0; k < ns; ++k) {
             rc = launch_stage(c, st[k]);
@@ -3275,7 +3416,7 @@ int amrgpu_get_tile(amrgpu_ctx *c, int *ppb, int *minw, int *design)
 static int restore_trial(amrgpu_ctx *c, int cur0, size_t nstate, const std::vector<double> &t0)
 {
     HIPCHK(hipMemcpyAsync(c->U[cur0], c->d_stage, sizeof(double) * nstate, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d_t, t0.data(), sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->t_now(), t0.data(), sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->cur = cur0;
     return AMRGPU_OK;
@@ -3338,7 +3479,7 @@ int amrgpu_autotune(amrgpu_ctx *c, int nsteps, int *nvar, int *ppb, int *minw, i
     // per-instance time, and restore both afterwards, on every exit path
     const size_t nstate = (size_t)c->nquad * 4 * c->n * c->n;
     std::vector<double> t0(c->ninst);
-    HIPCHK(hipMemcpyAsync(t0.data(), c->d_t, sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(t0.data(), c->t_now(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(c->d_stage, c->U[c->cur], sizeof(double) * nstate, hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     const int cur0 = c->cur;
@@ -3478,11 +3619,12 @@ int amrgpu_cfl_noalloc(int nelem_subgrid, int nquad, int ninst, const double *h_
     m.inst = d_inst;
     m.ip = ip;
     const int ppb = ppb_of(nelem_subgrid), nblk = (nquad + ppb - 1) / ppb;
+    unsigned long long *const none = nullptr;
     switch (nelem_subgrid) {
-    case 2: hipLaunchKernelGGL((cfl_kernel<2, 16>), dim3(nblk), dim3(64), 0, st, m, d_U, slot); break;
-    case 4: hipLaunchKernelGGL((cfl_kernel<4, 8>), dim3(nblk), dim3(128), 0, st, m, d_U, slot); break;
-    case 8: hipLaunchKernelGGL((cfl_kernel<8, 4>), dim3(nblk), dim3(256), 0, st, m, d_U, slot); break;
-    default: hipLaunchKernelGGL((cfl_kernel<16, 1>), dim3(nblk), dim3(256), 0, st, m, d_U, slot); break;
+    case 2: hipLaunchKernelGGL((cfl_kernel<2, 16>), dim3(nblk), dim3(64), 0, st, m, d_U, slot, none); break;
+    case 4: hipLaunchKernelGGL((cfl_kernel<4, 8>), dim3(nblk), dim3(128), 0, st, m, d_U, slot, none); break;
+    case 8: hipLaunchKernelGGL((cfl_kernel<8, 4>), dim3(nblk), dim3(256), 0, st, m, d_U, slot, none); break;
+    default: hipLaunchKernelGGL((cfl_kernel<16, 1>), dim3(nblk), dim3(256), 0, st, m, d_U, slot, none); break;
     }
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(noalloc_finish_kernel, dim3(ninst), dim3(64), 0, st, slot, ninst, d_dt);

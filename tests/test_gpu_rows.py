@@ -76,3 +76,68 @@ def test_default_tile_follows_the_mesh_until_one_is_set():
     setup(8)
     assert g.tile() == (8, 1, 0)
     g.close()
+
+
+@pytest.mark.parametrize("scheme", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n,own,other", [(2, (16, 3, 3), (16, 1, 0)), (4, (4, 3, 3), (8, 1, 1)), (4, (8, 3, 3), (8, 1, 0)),
+                                          (8, (1, 5, 1), (2, 4, 1)), (16, (1, 5, 1), (1, 4, 0))])
+def test_steps_without_a_prep_launch(n, own, other, scheme):
+    """small meshes: the first stage forms the step's dt, in rotating sets of
+    CFL sub-slots and two clocks; a tile that has a kernel ahead for it gives
+    the same states, times and step sizes through runs of one and several
+    steps, a CFL query, a new time, a new state, a remesh, an instance without
+    quadrants, and a change to graph replay and back"""
+    forests = [small_forest(n, 31, False, 1, 3), small_forest(n, 32, True, 1, 2), small_forest(n, 33, True, 0, 0)]
+    insts = [amrhip.make_inst(1.0, (1, 0, 2, 1), 0.2, 2e-3), amrhip.make_inst(1.0, (0,) * 4, 0.15, 1e-3, 2.5e-3),
+             # (SSP-RK2 takes the cap itself, not the CFL minimum: a stable one there)
+             amrhip.make_inst(1.0, (0,) * 4, 0.25, 1.0 if scheme != 2 else 3e-3)]
+    arrays = amrhip.batch_external(forests)
+    nq = [f.nquad for f in forests]
+    gs = []
+    for tile in (own, other):
+        g = amrhip.Gpu()
+        g.setup(n, scheme, insts, *arrays[:4], arrays[4])
+        g.set_tile(*tile)
+        gs.append(g)
+
+    def both(what):
+        got = [what(g) for g in gs]
+        a, b = ([np.asarray(x) for x in (r if isinstance(r, tuple) else (r,))] for r in got)
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
+
+    def state(g):
+        return (g.soln(), *g.time())
+
+    def run(k):
+        for g in gs:
+            g.run(k)
+        both(state)
+
+    run(1)
+    run(4)
+    both(lambda g: g.cfl())
+    run(2)
+    for g in gs:
+        g.set_time([1e-4, 1e-3, 0.0])
+    run(3)
+    new = gs[0].soln() * 1.01
+    for g in gs:
+        g.upload(new)
+    run(1)
+    gs[0].set_graphs(True)
+    run(3)
+    gs[0].set_graphs(False)
+    run(2)
+    # the same mesh again, then without the last instance's quadrant
+    ci, fi, _, _, inst = arrays
+    src = np.arange(sum(nq), dtype=np.int32)
+    for g in gs:
+        g.remesh(ci, fi, src, inst)
+    run(2)
+    ci2, fi2, _, _, inst2 = amrhip.batch_external(forests[:2])
+    for g in gs:
+        g.remesh(ci2, fi2, src[:nq[0] + nq[1]], inst2)
+    run(3)
+    for g in gs:
+        g.close()
