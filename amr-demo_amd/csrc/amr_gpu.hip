@@ -1942,6 +1942,37 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK)) void cfl_kernel(MeshDev m, con
         for (int i = blockIdx.x * TL::BLK + tid; i < m.ninst * NSLOT; i += gridDim.x * TL::BLK) clear[i] = DBL_INF_BITS;
 }
 
+__global__ void slot_min_kernel(const unsigned long long *slot, int ninst, double *dt)
+{
+    // one wave per instance
+    const int i = blockIdx.x;
+    if (i < ninst) {
+        const double m = slot_min(slot, i);
+        if (threadIdx.x == 0) dt[i] = m;
+    }
+}
+
+// The instances' time and step start time as given (null: 0) and, with dt, no last
+// dt.  One small workgroup: an instance is 24 bytes.
+__global__ void clock_kernel(double *t, double *dt, double *t_step, const double *t_inst, int ninst)
+{
+    for (int i = threadIdx.x; i < ninst; i += blockDim.x) {
+        const double v = t_inst ? t_inst[i] : 0.0;
+        t[i] = v;
+        t_step[i] = v;
+        if (dt) dt[i] = 0.0;
+    }
+}
+
+// Sums of n partial sums, a workgroup's share each.
+__global__ __launch_bounds__(256) void norm_kernel(const double *part, int n, double *out)
+{
+    __shared__ double red[4];
+    double s = 0.0;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) s += part[i];
+    sum_reduce_store<256>(s, &out[blockIdx.x], red);
+}
+
 __global__ void slot_reset_kernel(unsigned long long *slot, int ninst)
 {
     const int n = ninst * NSLOT;
@@ -2167,9 +2198,82 @@ extern "C" void amr_set_error(const char *fmt, ...)
     va_end(ap);
 }
 
+namespace {
+
+// Pinned host memory.  Copies between it and the device are plain DMA, where
+// pageable ones go through the runtime's own staging one call at a time; making
+// it costs 70-400 us and more, so contexts borrow it while copies are under way
+// and give it back at the next wait: at most PIN_KEEP bytes wait for the next
+// borrower, the rest is freed.
+struct PinBlock {
+    void *p = nullptr;
+    size_t cap = 0;
+};
+constexpr size_t PIN_KEEP = (size_t)64 << 20;
+std::mutex g_pin_lock;
+std::vector<PinBlock> g_pin_free;
+size_t g_pin_bytes = 0;
+
+void pin_give(PinBlock &b)
+{
+    if (!b.p) return;
+    bool keep;
+    {
+        std::lock_guard<std::mutex> hold(g_pin_lock);
+        keep = g_pin_bytes + b.cap <= PIN_KEEP;
+        if (keep) {
+            g_pin_free.push_back(b);
+            g_pin_bytes += b.cap;
+        }
+    }
+    if (!keep) (void)hipHostFree(b.p);
+    b = PinBlock();
+}
+
+// A block of at least `bytes` (the smallest that waits, or a new one with a
+// quarter to spare) in place of b, whose contents are dropped.
+int pin_take(PinBlock &b, size_t bytes)
+{
+    if (b.cap >= bytes) return AMRGPU_OK;
+    pin_give(b);
+    {
+        std::lock_guard<std::mutex> hold(g_pin_lock);
+        int best = -1;
+        for (int k = 0; k < (int)g_pin_free.size(); ++k)
+            if (g_pin_free[k].cap >= bytes && (best < 0 || g_pin_free[k].cap < g_pin_free[best].cap)) best = k;
+        if (best >= 0) {
+            b = g_pin_free[best];
+            g_pin_bytes -= b.cap;
+            g_pin_free.erase(g_pin_free.begin() + best);
+            return AMRGPU_OK;
+        }
+    }
+    const size_t cap = (bytes + bytes / 4 + 65535) / 65536 * 65536;
+    HIPCHK(hipHostMalloc(&b.p, cap, hipHostMallocPortable));
+    b.cap = cap;
+    return AMRGPU_OK;
+}
+
+// Arrays of the caller pass through RING_SLOTS pinned chunks, the host's copy of
+// one beside the DMA of the others.  Each DMA costs some 20 us to start and end:
+// 5.4 MB in and out again around ten steps takes 881 us a call with chunks of
+// 2 MB, 907 with 1 MB, 993 with 512 KB, 964 with 4 MB (1070 with pageable copies).
+// The calling thread copies: an OpenMP team is as fast, but its threads spin for a
+// while after each loop, in the way of everything else the process runs (a
+// 16-instance adaptive batch 74 -> 104 ms).
+constexpr int RING_SLOTS = 3;
+constexpr size_t RING_CHUNK = (size_t)2 << 20;
+
+}  // namespace
+
 struct amrgpu_ctx {
     int n = 0, nquad = 0, ninst = 0, scheme = 3;
     hipStream_t stream = nullptr;
+    // one allocation: instances, clocks, CFL sub-slots, norm partials and
+    // indicator by capacity (ensure_capacity), then the mesh packed by its own
+    // size (place_mesh): corners, face table, levels, instance ids, source map
+    char *d_block = nullptr;
+    size_t mesh_off = 0;
     int *d_nbr = nullptr, *d_level = nullptr, *d_inst = nullptr;
     InstDev *d_ip = nullptr;
     double *U[3] = {nullptr, nullptr, nullptr};
@@ -2209,8 +2313,11 @@ struct amrgpu_ctx {
     // autotuner measures it faster.
     bool graphs_enabled = false;
     std::vector<InstDev> h_ip;
-    int *h_pin = nullptr;      // pinned staging of the mesh uploads (ints)
-    size_t h_pin_cap = 0;
+    // pinned memory: small results (kept); mesh uploads and the chunks that states
+    // and other arrays of the caller travel through, with an event per chunk
+    // (borrowed until nothing is pending on them)
+    PinBlock res, up, ring;
+    hipEvent_t ring_ev[RING_SLOTS] = {};
     int cu_count = 256;        // compute units of the context's device
 };
 
@@ -2422,6 +2529,11 @@ StageArgs base_args(amrgpu_ctx *c)
     return a;
 }
 
+constexpr int NORM_DIRECT = 2048, NORM_PARTS = 64;
+
+// Where the residual's sums of squares go, one per workgroup (finish_norm).
+double *norm_out(const amrgpu_ctx *c) { return c->nblocks > NORM_DIRECT ? c->d_norm : (double *)c->res.p; }
+
 // Stage launches of one step starting from state buffer `cur`; returns the
 // buffer holding the new state.  Shu-Osher forms need the stage state and
 // the step's base state only (2 reads + 1 write per cell-stage).
@@ -2435,14 +2547,14 @@ int build_step(amrgpu_ctx *c, int cur, std::vector<StageArgs> &st, bool with_nor
     case 1:
         a.Us = A; a.U0 = nullptr; a.Uout = B; a.mode = MODE_SO; a.c0 = 0; a.c1 = 1; a.c2 = 1;
         a.role = cfl;
-        if (with_norm) a.norm_part = c->d_norm;
+        if (with_norm) a.norm_part = norm_out(c);
         st.push_back(a);
         return (cur + 1) % 3;
     case 2:
         a.Us = A; a.U0 = nullptr; a.Uout = B; a.mode = MODE_SO; a.c0 = 0; a.c1 = 1; a.c2 = 1;
         a.role = 0; st.push_back(a);
         a.Us = B; a.U0 = A; a.Uout = A; a.c0 = 0.5; a.c1 = 0.5; a.c2 = 0.5;
-        a.role = 0; if (with_norm) a.norm_part = c->d_norm; st.push_back(a);
+        a.role = 0; if (with_norm) a.norm_part = norm_out(c); st.push_back(a);
         return cur;
     case 3:
         a.Us = A; a.U0 = nullptr; a.Uout = B; a.mode = MODE_SO; a.c0 = 0; a.c1 = 1; a.c2 = 1;
@@ -2450,7 +2562,7 @@ int build_step(amrgpu_ctx *c, int cur, std::vector<StageArgs> &st, bool with_nor
         a.Us = B; a.U0 = A; a.Uout = C; a.c0 = 0.75; a.c1 = 0.25; a.c2 = 0.25;
         a.role = 0; st.push_back(a);
         a.Us = C; a.U0 = A; a.Uout = A; a.c0 = 1.0 / 3.0; a.c1 = 2.0 / 3.0; a.c2 = 2.0 / 3.0;
-        a.role = cfl; if (with_norm) a.norm_part = c->d_norm; st.push_back(a);
+        a.role = cfl; if (with_norm) a.norm_part = norm_out(c); st.push_back(a);
         return cur;
     case 4:
         a.Acc = c->Acc;
@@ -2459,7 +2571,7 @@ int build_step(amrgpu_ctx *c, int cur, std::vector<StageArgs> &st, bool with_nor
         a.Us = B; a.Uout = C; a.first = 0; a.c2 = 0.5; a.role = 0; st.push_back(a);
         a.Us = C; a.Uout = B; a.c2 = 1.0; a.role = 0; st.push_back(a);
         a.Us = B; a.Uout = A; a.mode = MODE_RK4_FINAL; a.role = cfl;
-        if (with_norm) a.norm_part = c->d_norm; st.push_back(a);
+        if (with_norm) a.norm_part = norm_out(c); st.push_back(a);
         return cur;
     case 5: {
         static const double ra[5] = {0.0,
@@ -2474,7 +2586,7 @@ int build_step(amrgpu_ctx *c, int cur, std::vector<StageArgs> &st, bool with_nor
         for (int s = 0; s < 5; ++s) {
             a.Us = X; a.U0 = nullptr; a.Uout = Y; a.first = (s == 0); a.c1 = ra[s]; a.c2 = rb[s];
             a.role = s == 4 ? cfl : 0;
-            a.norm_part = (s == 4 && with_norm) ? c->d_norm : nullptr;
+            a.norm_part = (s == 4 && with_norm) ? norm_out(c) : nullptr;
             st.push_back(a);
             double *tmp = X; X = Y; Y = tmp;
         }
@@ -2550,11 +2662,9 @@ void free_graphs(amrgpu_ctx *c)
 void free_mesh(amrgpu_ctx *c)
 {
     free_graphs(c);
-    (void)hipFree(c->d_nbr); (void)hipFree(c->d_level); (void)hipFree(c->d_inst); (void)hipFree(c->d_ip);
-    for (int i = 0; i < 3; ++i) (void)hipFree(c->U[i]);
-    (void)hipFree(c->Acc); (void)hipFree(c->d_clock); (void)hipFree(c->d_slot_sets);
-    (void)hipFree(c->d_norm); (void)hipFree(c->d_stage);
-    (void)hipFree(c->d_map); (void)hipFree(c->d_ind); (void)hipFree(c->d_org);
+    (void)hipFree(c->d_block);
+    (void)hipFree(c->U[0]);             // U[1], U[2], Acc and d_stage are parts of it
+    c->d_block = nullptr;
     c->d_map = nullptr; c->d_ind = nullptr; c->d_org = nullptr;
     c->org_ok = false;
     c->d_nbr = c->d_level = c->d_inst = nullptr; c->d_ip = nullptr;
@@ -2566,10 +2676,105 @@ void free_mesh(amrgpu_ctx *c)
     c->cap_state = 0;
 }
 
-// face_info (reference format) -> per-quadrant face table
-int build_nbr(int ncell, int nface, const int *face_info, std::vector<int> &nbr)
+// The packed mesh's arrays in a block that starts at `base`, for ncell quadrants:
+// corners, face table, levels, instance ids, source map.
+struct MeshPlace {
+    double *org;
+    int *nbr, *level, *inst, *map, *end;
+};
+MeshPlace place_mesh(char *base, int ncell)
 {
-    nbr.assign((size_t)ncell * 8, -2);
+    MeshPlace m;
+    m.org = (double *)base;
+    m.nbr = (int *)(m.org + 2 * (size_t)ncell);
+    m.level = m.nbr + 8 * (size_t)ncell;
+    m.inst = m.level + ncell;
+    m.map = m.inst + ncell;
+    m.end = m.map + ncell;
+    return m;
+}
+constexpr size_t MESH_BYTES = 2 * sizeof(double) + 11 * sizeof(int);     // per quadrant
+
+// Wait for the stream; the borrowed pinned memory goes back.
+int sync_stream(amrgpu_ctx *c)
+{
+    HIPCHK(hipStreamSynchronize(c->stream));
+    pin_give(c->up);
+    pin_give(c->ring);
+    return AMRGPU_OK;
+}
+
+// The pinned area of mesh uploads, free for `bytes` to be written.
+int take_up(amrgpu_ctx *c, size_t bytes)
+{
+    if (c->up.p)
+        if (int rc = sync_stream(c)) return rc;
+    return pin_take(c->up, bytes);
+}
+
+int take_ring(amrgpu_ctx *c)
+{
+    if (c->ring.p)
+        HIPCHK(hipStreamSynchronize(c->stream));     // (mesh uploads may be under way beside it)
+    if (int rc = pin_take(c->ring, RING_SLOTS * RING_CHUNK)) return rc;
+    for (hipEvent_t &e : c->ring_ev)
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return AMRGPU_OK;
+}
+
+// The caller's `bytes` at src to the device; src may change once it returns, the
+// copy is ordered on the stream.
+int copy_in(amrgpu_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    if (int rc = take_ring(c)) return rc;
+    int k = 0;
+    for (size_t at = 0; at < bytes; at += RING_CHUNK, ++k) {
+        const int slot = k % RING_SLOTS;
+        const size_t n = std::min(RING_CHUNK, bytes - at);
+        char *pin = (char *)c->ring.p + slot * RING_CHUNK;
+        if (k >= RING_SLOTS) HIPCHK(hipEventSynchronize(c->ring_ev[slot]));
+        memcpy(pin, (const char *)src + at, n);
+        HIPCHK(hipMemcpyAsync((char *)dst + at, pin, n, hipMemcpyHostToDevice, c->stream));
+        if (bytes > RING_SLOTS * RING_CHUNK) HIPCHK(hipEventRecord(c->ring_ev[slot], c->stream));
+    }
+    return AMRGPU_OK;
+}
+
+// `bytes` of the device at src, after what the stream holds, to the caller.
+int copy_out(amrgpu_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    if (int rc = take_ring(c)) return rc;
+    const int chunks = (int)((bytes + RING_CHUNK - 1) / RING_CHUNK);
+    auto size = [&](int k) { return std::min(RING_CHUNK, bytes - k * RING_CHUNK); };
+    auto fetch = [&](int k) {
+        const int slot = k % RING_SLOTS;
+        HIPCHK(hipMemcpyAsync((char *)c->ring.p + slot * RING_CHUNK, (const char *)src + k * RING_CHUNK, size(k),
+                              hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipEventRecord(c->ring_ev[slot], c->stream));
+        return AMRGPU_OK;
+    };
+    if (chunks == 1) {
+        HIPCHK(hipMemcpyAsync(c->ring.p, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        memcpy(dst, c->ring.p, bytes);
+        return sync_stream(c);
+    }
+    for (int k = 0; k < std::min(chunks, RING_SLOTS); ++k)
+        if (int rc = fetch(k)) return rc;
+    for (int k = 0; k < chunks; ++k) {
+        const int slot = k % RING_SLOTS;
+        HIPCHK(hipEventSynchronize(c->ring_ev[slot]));
+        memcpy((char *)dst + k * RING_CHUNK, (char *)c->ring.p + slot * RING_CHUNK, size(k));
+        if (k + RING_SLOTS < chunks)
+            if (int rc = fetch(k + RING_SLOTS)) return rc;
+    }
+    return sync_stream(c);
+}
+
+// face_info (reference format) -> per-quadrant face table
+int build_nbr(int ncell, int nface, const int *face_info, int *nbr)
+{
+    std::fill(nbr, nbr + (size_t)ncell * 8, -2);
     auto setside = [&](int q, int s, int a, int b) -> int {
         if (q < 0 || q >= ncell || s < 0 || s > 3) return -1;
         int *e = &nbr[(size_t)q * 8 + 2 * s];
@@ -2654,7 +2859,11 @@ void amrgpu_destroy(amrgpu_ctx *c)
     if (!c) return;
     (void)hipStreamSynchronize(c->stream);
     free_mesh(c);
-    if (c->h_pin) (void)hipHostFree(c->h_pin);
+    for (hipEvent_t e : c->ring_ev)
+        if (e) (void)hipEventDestroy(e);
+    pin_give(c->up);
+    pin_give(c->res);
+    pin_give(c->ring);
     (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -2666,6 +2875,8 @@ int amrgpu_staging(amrgpu_ctx *c, double **buf, size_t *ndoubles)
     *ndoubles = c->cap_state;
     return AMRGPU_OK;
 }
+
+int amrgpu_fetch(amrgpu_ctx *c, void *dst, const void *src, size_t bytes) { return copy_out(c, dst, src, bytes); }
 
 int amrgpu_num_cells(const amrgpu_ctx *c) { return c ? c->nquad * c->n * c->n : 0; }
 int amrgpu_num_quads(const amrgpu_ctx *c) { return c ? c->nquad : 0; }
@@ -2728,60 +2939,41 @@ static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need
     // past the last one
     const size_t pad = (size_t)16 * 4 * n2;
     c->cap_blocks = capq + 64;   // enough for one patch per workgroup
-    const size_t cq = (size_t)c->cap_quad, cs = c->cap_state;
-    HIPCHK(hipMalloc(&c->d_nbr, sizeof(int) * 8 * cq));
-    HIPCHK(hipMalloc(&c->d_level, sizeof(int) * cq));
-    HIPCHK(hipMalloc(&c->d_inst, sizeof(int) * cq));
-    HIPCHK(hipMalloc(&c->d_ip, sizeof(InstDev) * c->cap_inst));
-    for (int i = 0; i < 3; ++i) HIPCHK(hipMalloc(&c->U[i], sizeof(double) * (cs + pad)));
-    if (need_acc) HIPCHK(hipMalloc(&c->Acc, sizeof(double) * (cs + pad)));
-    HIPCHK(hipMalloc(&c->d_clock, sizeof(double) * 4 * c->cap_inst));
-    HIPCHK(hipMalloc(&c->d_slot_sets, sizeof(unsigned long long) * 3 * c->cap_inst * NSLOT));
-    if (int rc = empty_slots(c)) return rc;
-    HIPCHK(hipMalloc(&c->d_norm, sizeof(double) * c->cap_blocks));
-    HIPCHK(hipMalloc(&c->d_stage, sizeof(double) * cs));
-    HIPCHK(hipMalloc(&c->d_map, sizeof(int) * cq));
-    HIPCHK(hipMalloc(&c->d_ind, sizeof(double) * cq));
-    HIPCHK(hipMalloc(&c->d_org, sizeof(double) * 2 * cq));
-    return AMRGPU_OK;
+    const size_t cq = (size_t)c->cap_quad, cs = c->cap_state, vec = (cs + pad + 31) / 32 * 32;
+    HIPCHK(hipMalloc((void **)&c->U[0], sizeof(double) * ((need_acc ? 4 : 3) * vec + cs)));
+    c->U[1] = c->U[0] + vec;
+    c->U[2] = c->U[1] + vec;
+    c->Acc = need_acc ? c->U[2] + vec : nullptr;
+    c->d_stage = (need_acc ? c->Acc : c->U[2]) + vec;
+    size_t at = 0;
+    auto part = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    const size_t ip = part(sizeof(InstDev) * c->cap_inst), clock = part(sizeof(double) * 4 * c->cap_inst);
+    const size_t slot = part(sizeof(unsigned long long) * 3 * c->cap_inst * NSLOT);
+    const size_t norm = part(sizeof(double) * c->cap_blocks), ind = part(sizeof(double) * cq);
+    c->mesh_off = part(MESH_BYTES * cq);
+    if (hipMalloc((void **)&c->d_block, at) != hipSuccess) {
+        free_mesh(c);
+        set_err("%s:%d device allocation of %zu bytes failed", __FILE__, __LINE__, at);
+        return AMRGPU_ERR_HIP;
+    }
+    c->d_ip = (InstDev *)(c->d_block + ip);
+    c->d_clock = (double *)(c->d_block + clock);
+    c->d_slot_sets = (unsigned long long *)(c->d_block + slot);
+    c->d_norm = (double *)(c->d_block + norm);
+    c->d_ind = (double *)(c->d_block + ind);
+    return empty_slots(c);
 }
 
-// Levels of the reference's cell_info (already validated).
-static std::vector<int> levels_of(int ncell, const int *cell_info)
+// The device mesh is a new one of ncell quadrants with these instance ids (null:
+// all 0): its arrays' places, the tile and what hangs on them.
+static int new_mesh(amrgpu_ctx *c, int ncell, const int *cell_inst)
 {
-    std::vector<int> level(ncell);
-    for (int q = 0; q < ncell; ++q) level[q] = cell_info[3 * q + 1];
-    return level;
-}
-
-// Upload the face table, levels and instances of a mesh already validated.
-// Pinned host staging for the uploads of setup, remesh and origins: copies
-// from it are plain asynchronous DMA, where pageable ones go through the
-// runtime's own staging call by call.  Every user synchronises the stream
-// before it returns, so no copy from the buffer is pending whenever it is
-// written; growing it synchronises first.
-static int pin_staging(amrgpu_ctx *c, size_t nint)
-{
-    if (nint <= c->h_pin_cap) return AMRGPU_OK;
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (c->h_pin) (void)hipHostFree(c->h_pin);
-    c->h_pin = nullptr;
-    c->h_pin_cap = 0;
-    const size_t cap = nint + nint / 2 + 64;
-    HIPCHK(hipHostMalloc((void **)&c->h_pin, sizeof(int) * cap, hipHostMallocDefault));
-    c->h_pin_cap = cap;
-    return AMRGPU_OK;
-}
-
-static int upload_mesh(amrgpu_ctx *c, int ncell, const int *level, const int *cell_inst, const int *nbr)
-{
-    int rc = pin_staging(c, 10 * (size_t)ncell);     // nbr, level, instance
-    if (rc) return rc;
-    int *pn = c->h_pin, *pl = pn + 8 * (size_t)ncell, *pq = pl + ncell;
-    memcpy(pn, nbr, sizeof(int) * 8 * (size_t)ncell);
-    memcpy(pl, level, sizeof(int) * (size_t)ncell);
-    if (cell_inst) memcpy(pq, cell_inst, sizeof(int) * (size_t)ncell);
-    else memset(pq, 0, sizeof(int) * (size_t)ncell);
+    const MeshPlace m = place_mesh(c->d_block + c->mesh_off, ncell);
+    c->d_org = m.org; c->d_nbr = m.nbr; c->d_level = m.level; c->d_inst = m.inst; c->d_map = m.map;
     c->nquad = ncell;
     c->all_inst = c->ninst == 1;
     if (cell_inst && c->ninst > 1) {
@@ -2798,19 +2990,56 @@ static int upload_mesh(amrgpu_ctx *c, int ncell, const int *level, const int *ce
         set_err("internal capacity error");
         return AMRGPU_ERR_ARG;
     }
-    HIPCHK(hipMemcpyAsync(c->d_nbr, pn, sizeof(int) * 8 * (size_t)ncell, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d_level, pl, sizeof(int) * (size_t)ncell, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->d_inst, pq, sizeof(int) * (size_t)ncell, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
     return AMRGPU_OK;
 }
 
-int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
-                 const amrgpu_inst_t *inst, int ncell, const int *cell_info,
-                 const int *cell_inst, int nface, const int *face_info, const double *geom,
-                 const double *soln)
+static void put_ids(int *dst, const int *src, int n)
 {
-    if (!c || !inst || !cell_info || !face_info || ncell <= 0 || ninst <= 0 || nface < 0) {
+    if (src) memcpy(dst, src, sizeof(int) * (size_t)n);
+    else memset(dst, 0, sizeof(int) * (size_t)n);
+}
+
+// The pinned area of small results; a larger one only once nothing reads the old.
+static int take_res(amrgpu_ctx *c, size_t bytes)
+{
+    if (c->res.cap >= bytes && c->res.p) return AMRGPU_OK;
+    if (int rc = sync_stream(c)) return rc;
+    return pin_take(c->res, std::max(bytes, (size_t)65536));
+}
+
+// (called where the stream is idle: nothing else reads the small-results area)
+static int set_clocks(amrgpu_ctx *c, const double *t_inst)
+{
+    const double *src = nullptr;
+    if (t_inst) {
+        if (int rc = take_res(c, sizeof(double) * c->ninst)) return rc;
+        memcpy(c->res.p, t_inst, sizeof(double) * c->ninst);
+        src = (const double *)c->res.p;
+    }
+    hipLaunchKernelGGL(clock_kernel, dim3(1), dim3(64), 0, c->stream, c->t_now(), c->dt_cur(), c->t_step(), src, c->ninst);
+    HIPCHK(hipGetLastError());
+    return AMRGPU_OK;
+}
+
+// The reference-layout state to the device, ordered on the stream.
+static int start_upload(amrgpu_ctx *c, const double *soln)
+{
+    const int n2 = c->n * c->n;
+    const long long ncells = (long long)c->nquad * n2;
+    if (int rc = copy_in(c, c->d_stage, soln, sizeof(double) * 4 * ncells)) return rc;
+    c->cur = 0;
+    hipLaunchKernelGGL(aos_to_soa_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
+                       c->d_stage, c->U[0], ncells, n2);
+    HIPCHK(hipGetLastError());
+    return AMRGPU_OK;
+}
+
+int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
+                      const amrgpu_inst_t *inst, int ncell, const int *cell_info,
+                      const int *cell_inst, int nface, const int *face_info, const double *geom,
+                      const double *soln, const double *t_inst)
+{
+    if (!c || !inst || !cell_info || ncell <= 0 || ninst <= 0 || nface < 0) {
         set_err("amrgpu_setup: bad arguments");
         return AMRGPU_ERR_ARG;
     }
@@ -2831,9 +3060,23 @@ int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
     const int n2 = nelem_subgrid * nelem_subgrid;
     int rc = validate_cells(n2, ninst, ncell, cell_info, cell_inst, "amrgpu_setup");
     if (rc) return rc;
-    std::vector<int> nbr;
-    rc = build_nbr(ncell, nface, face_info, nbr);
+    // the mesh, packed as it lies on the device, is built in the pinned area
+    rc = take_up(c, MESH_BYTES * (size_t)ncell + (sizeof(InstDev) + 4 * sizeof(double)) * ninst);
     if (rc) return rc;
+    const MeshPlace h = place_mesh((char *)c->up.p, ncell);
+    if (face_info) {
+        rc = build_nbr(ncell, nface, face_info, h.nbr);
+        if (rc) return rc;
+    } else {
+        std::fill(h.nbr, h.nbr + 8 * (size_t)ncell, -1);
+    }
+    for (int q = 0; q < ncell; ++q) h.level[q] = cell_info[3 * q + 1];
+    put_ids(h.inst, cell_inst, ncell);
+    if (geom)
+        for (int q = 0; q < ncell; ++q) {
+            h.org[2 * (size_t)q] = geom[12 * (size_t)q];          // corner 0: (x, y) of the lower-left node
+            h.org[2 * (size_t)q + 1] = geom[12 * (size_t)q + 1];
+        }
 
     HIPCHK(hipStreamSynchronize(c->stream));
     free_graphs(c);
@@ -2843,6 +3086,7 @@ int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
     if (rc) return rc;
     c->n = nelem_subgrid; c->ninst = ninst; c->scheme = time_scheme;
     c->cur = 0;
+    c->tb = 0;
     c->h_ip.resize(ninst);
     c->need_org = false;
     for (int i = 0; i < ninst; ++i) {
@@ -2865,20 +3109,28 @@ int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
         d.ninv_vol0 = -1.0 / v0;
         d.cfl_h0 = inst[i].cfl * sqrt(v0);
     }
-    HIPCHK(hipMemcpyAsync(c->d_ip, c->h_ip.data(), sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
-    std::vector<double> zeros(ninst, 0.0);
-    HIPCHK(hipMemcpyAsync(c->t_now(), zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->t_step(), zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->dt_cur(), zeros.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-    rc = upload_mesh(c, ncell, levels_of(ncell, cell_info).data(), cell_inst, nbr.data());
+    rc = new_mesh(c, ncell, cell_inst);
     if (rc) return rc;
-    c->org_ok = false;
-    if (geom) {
-        rc = amrgpu_set_geometry(c, geom);
-        if (rc) return rc;
-    }
-    if (soln) return amrgpu_upload_soln(c, soln);
+    c->org_ok = geom != nullptr;
+    HIPCHK(hipMemcpyAsync(c->d_org, h.org, (size_t)((char *)h.map - (char *)h.org), hipMemcpyHostToDevice, c->stream));
+    // instances and clocks after the mesh in the pinned area
+    InstDev *const hip = (InstDev *)h.end;
+    memcpy(hip, c->h_ip.data(), sizeof(InstDev) * ninst);
+    HIPCHK(hipMemcpyAsync(c->d_ip, hip, sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
+    if ((rc = set_clocks(c, t_inst))) return rc;
+    if (soln) return start_upload(c, soln);
     return AMRGPU_OK;
+}
+
+int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
+                 const amrgpu_inst_t *inst, int ncell, const int *cell_info,
+                 const int *cell_inst, int nface, const int *face_info, const double *geom,
+                 const double *soln)
+{
+    if (!face_info) { set_err("amrgpu_setup: bad arguments"); return AMRGPU_ERR_ARG; }
+    int rc = amrgpu_setup_from(c, nelem_subgrid, time_scheme, ninst, inst, ncell, cell_info, cell_inst, nface,
+                               face_info, geom, soln, nullptr);
+    return rc ? rc : sync_stream(c);
 }
 
 int amrgpu_set_geometry(amrgpu_ctx *c, const double *geom)
@@ -2889,10 +3141,7 @@ int amrgpu_set_geometry(amrgpu_ctx *c, const double *geom)
         org[2 * (size_t)q] = geom[12 * (size_t)q];          // corner 0: (x, y) of the lower-left node
         org[2 * (size_t)q + 1] = geom[12 * (size_t)q + 1];
     }
-    HIPCHK(hipMemcpyAsync(c->d_org, org.data(), sizeof(double) * org.size(), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    c->org_ok = true;
-    return AMRGPU_OK;
+    return amrgpu_set_origins(c, org.data());
 }
 
 int amrgpu_indicator(amrgpu_ctx *c, double *ind)
@@ -2900,9 +3149,7 @@ int amrgpu_indicator(amrgpu_ctx *c, double *ind)
     if (!c || !ind || !c->nquad) { set_err("amrgpu_indicator: no mesh"); return AMRGPU_ERR_ARG; }
     int rc = launch_indicator(c, c->d_ind);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(ind, c->d_ind, sizeof(double) * c->nquad, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return AMRGPU_OK;
+    return copy_out(c, ind, c->d_ind, sizeof(double) * c->nquad);
 }
 
 int amrgpu_feature_tags(amrgpu_ctx *c, int ntags, const int *methods, const double *tols, int *tags)
@@ -2928,9 +3175,7 @@ int amrgpu_feature_tags(amrgpu_ctx *c, int ntags, const int *methods, const doub
     default: set_err("unsupported nelem_subgrid %d", c->n); return AMRGPU_ERR_ARG;
     }
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(tags, d_tags, sizeof(int) * c->nquad, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return AMRGPU_OK;
+    return copy_out(c, tags, d_tags, sizeof(int) * c->nquad);
 }
 
 // The source map of a remesh refers to the old mesh only.
@@ -2946,9 +3191,9 @@ static int check_src(int ncell, const int *src, int nold, const char *who)
     return AMRGPU_OK;
 }
 
-// Remap the state onto a validated new mesh and upload its table.
-static int remesh_to(amrgpu_ctx *c, int ncell, const int *level, const int *cell_inst, const int *nbr,
-                     const int *src)
+// Remap the state onto a validated new mesh and upload its table.  `h` is the
+// table packed in the pinned area (corners unset).
+static int remesh_to(amrgpu_ctx *c, int ncell, const MeshPlace &h, const int *cell_inst)
 {
     const int n2 = c->n * c->n, nold = c->nquad;
     int rc = AMRGPU_OK;
@@ -2957,52 +3202,43 @@ static int remesh_to(amrgpu_ctx *c, int ncell, const int *level, const int *cell
     const long long ncells = (long long)ncell * n2;
     const size_t old_state = (size_t)nold * 4 * n2;
     const bool fits = ncell <= c->cap_quad && (size_t)ncell * 4 * n2 <= c->cap_state;
-    if (fits) {
-        // old state in U[cur], new state into the next buffer; the source
-        // map goes through the staging after the table's part of it
-        const int nx = (c->cur + 1) % 3;
-        rc = pin_staging(c, 11 * (size_t)ncell);
-        if (rc) return rc;
-        int *ps = c->h_pin + 10 * (size_t)ncell;
-        memcpy(ps, src, sizeof(int) * (size_t)ncell);
-        HIPCHK(hipMemcpyAsync(c->d_map, ps, sizeof(int) * ncell, hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL(remap_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
-                           c->U[c->cur], c->U[nx], c->d_map, ncells, n2);
-        HIPCHK(hipGetLastError());
-        c->cur = nx;
-    } else {
-        // keep the old state, time, dt and step start time in scratch
-        // allocations, regrow, remap (the residual of a remeshed state reads
-        // the step start time before any step rewrites it)
-        double *keep = nullptr;
-        int *map = nullptr;
-        std::vector<double> t(c->ninst), dt(c->ninst), ts(c->ninst);
-        HIPCHK(hipMemcpyAsync(t.data(), c->t_now(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipMemcpyAsync(dt.data(), c->dt_cur(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipMemcpyAsync(ts.data(), c->t_step(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
+    const double *from = c->U[c->cur];
+    double *keep = nullptr;
+    int to = (c->cur + 1) % 3;
+    if (!fits) {
+        // keep the old state, time, dt and step start time, regrow (the residual
+        // of a remeshed state reads the step start time before any step
+        // rewrites it)
+        std::vector<double> clk(3 * (size_t)c->ninst);
+        double *const part[3] = {c->t_now(), c->dt_cur(), c->t_step()};
+        for (int k = 0; k < 3; ++k)
+            HIPCHK(hipMemcpyAsync(&clk[k * (size_t)c->ninst], part[k], sizeof(double) * c->ninst, hipMemcpyDeviceToHost,
+                                  c->stream));
         HIPCHK(hipMalloc(&keep, sizeof(double) * old_state));
-        HIPCHK(hipMalloc(&map, sizeof(int) * ncell));
-        HIPCHK(hipMemcpyAsync(keep, c->U[c->cur], sizeof(double) * old_state, hipMemcpyDeviceToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(map, src, sizeof(int) * ncell, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipMemcpyAsync(keep, from, sizeof(double) * old_state, hipMemcpyDeviceToDevice, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
         const int ninst = c->ninst;
         bool fresh;
         rc = ensure_capacity(c, c->n, ncell + ncell / 2, ninst, c->scheme == 4 || c->scheme == 5, &fresh);
-        if (rc) { (void)hipFree(keep); (void)hipFree(map); return rc; }
+        if (rc) { (void)hipFree(keep); return rc; }
         HIPCHK(hipMemcpyAsync(c->d_ip, c->h_ip.data(), sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->t_now(), t.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->dt_cur(), dt.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->t_step(), ts.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL(remap_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
-                           keep, c->U[0], map, ncells, n2);
-        HIPCHK(hipGetLastError());
+        double *const now[3] = {c->t_now(), c->dt_cur(), c->t_step()};
+        for (int k = 0; k < 3; ++k)
+            HIPCHK(hipMemcpyAsync(now[k], &clk[k * (size_t)ninst], sizeof(double) * ninst, hipMemcpyHostToDevice,
+                                  c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
-        (void)hipFree(keep);
-        (void)hipFree(map);
-        c->cur = 0;
+        from = keep;
+        to = 0;
     }
-    rc = upload_mesh(c, ncell, level, cell_inst, nbr);
-    if (rc) return rc;
+    rc = new_mesh(c, ncell, cell_inst);
+    if (rc) { (void)hipFree(keep); return rc; }
+    HIPCHK(hipMemcpyAsync(c->d_nbr, h.nbr, (size_t)((char *)h.end - (char *)h.nbr), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(remap_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream, from, c->U[to],
+                       c->d_map, ncells, n2);
+    HIPCHK(hipGetLastError());
+    c->cur = to;
+    if ((rc = sync_stream(c))) return rc;
+    (void)hipFree(keep);
     // an instance left without quadrants (a batch drops those that reached
     // their stop) no longer advances: no wave publishes its dt any more, so
     // its last dt is cleared here and the time bookkeeping of the stages
@@ -3037,11 +3273,16 @@ int amrgpu_remesh(amrgpu_ctx *c, int ncell, const int *cell_info, const int *cel
     int rc = check_src(ncell, src, c->nquad, "amrgpu_remesh");
     if (!rc) rc = validate_cells(c->n * c->n, c->ninst, ncell, cell_info, cell_inst, "amrgpu_remesh");
     if (rc) return rc;
-    std::vector<int> nbr;
-    rc = build_nbr(ncell, nface, face_info, nbr);
+    rc = take_up(c, MESH_BYTES * (size_t)ncell);
+    if (rc) return rc;
+    const MeshPlace h = place_mesh((char *)c->up.p, ncell);
+    rc = build_nbr(ncell, nface, face_info, h.nbr);
     if (rc) return rc;                 // a refused call leaves the context as it was
+    for (int q = 0; q < ncell; ++q) h.level[q] = cell_info[3 * q + 1];
+    put_ids(h.inst, cell_inst, ncell);
+    put_ids(h.map, src, ncell);
     c->org_ok = false;                 // the new quadrants' coordinates come with amrgpu_set_geometry
-    return remesh_to(c, ncell, levels_of(ncell, cell_info).data(), cell_inst, nbr.data(), src);
+    return remesh_to(c, ncell, h, cell_inst);
 }
 
 int amrgpu_remesh_nbr(amrgpu_ctx *c, int ncell, const int *level, const int *cell_inst, const int *nbr,
@@ -3071,20 +3312,21 @@ int amrgpu_remesh_nbr(amrgpu_ctx *c, int ncell, const int *level, const int *cel
             }
         }
     }
+    rc = take_up(c, MESH_BYTES * (size_t)ncell);
+    if (rc) return rc;
+    const MeshPlace h = place_mesh((char *)c->up.p, ncell);
+    memcpy(h.nbr, nbr, sizeof(int) * 8 * (size_t)ncell);
+    put_ids(h.level, level, ncell);
+    put_ids(h.inst, cell_inst, ncell);
+    put_ids(h.map, src, ncell);
     c->org_ok = false;                 // the new quadrants' coordinates come with amrgpu_set_origins
-    return remesh_to(c, ncell, level, cell_inst, nbr, src);
+    return remesh_to(c, ncell, h, cell_inst);
 }
 
 int amrgpu_set_origins(amrgpu_ctx *c, const double *org)
 {
     if (!c || !c->nquad || !org) { set_err("amrgpu_set_origins: no mesh"); return AMRGPU_ERR_ARG; }
-    // no copy from the staging is pending (its users synchronise first)
-    int rc = pin_staging(c, 4 * (size_t)c->nquad);
-    if (rc) return rc;
-    memcpy(c->h_pin, org, sizeof(double) * 2 * (size_t)c->nquad);
-    HIPCHK(hipMemcpyAsync(c->d_org, c->h_pin, sizeof(double) * 2 * (size_t)c->nquad, hipMemcpyHostToDevice,
-                          c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (int rc = copy_in(c, c->d_org, org, sizeof(double) * 2 * (size_t)c->nquad)) return rc;
     c->org_ok = true;
     return AMRGPU_OK;
 }
@@ -3095,8 +3337,8 @@ int amrgpu_nbr_from_faces(int ncell, int nface, const int *face_info, int *nbr)
         set_err("amrgpu_nbr_from_faces: bad arguments");
         return AMRGPU_ERR_ARG;
     }
-    std::vector<int> t;
-    int rc = build_nbr(ncell, nface, face_info, t);
+    std::vector<int> t((size_t)ncell * 8);         // a refused table leaves the caller's array as it was
+    int rc = build_nbr(ncell, nface, face_info, t.data());
     if (rc) return rc;
     memcpy(nbr, t.data(), sizeof(int) * t.size());
     return AMRGPU_OK;
@@ -3105,15 +3347,8 @@ int amrgpu_nbr_from_faces(int ncell, int nface, const int *face_info, int *nbr)
 int amrgpu_upload_soln(amrgpu_ctx *c, const double *soln)
 {
     if (!c || !soln || !c->nquad) { set_err("amrgpu_upload_soln: no mesh"); return AMRGPU_ERR_ARG; }
-    const int n2 = c->n * c->n;
-    const long long ncells = (long long)c->nquad * n2;
-    HIPCHK(hipMemcpyAsync(c->d_stage, soln, sizeof(double) * 4 * ncells, hipMemcpyHostToDevice, c->stream));
-    c->cur = 0;
-    hipLaunchKernelGGL(aos_to_soa_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
-                       c->d_stage, c->U[0], ncells, n2);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return AMRGPU_OK;
+    int rc = start_upload(c, soln);
+    return rc ? rc : sync_stream(c);
 }
 
 int amrgpu_download_soln(amrgpu_ctx *c, double *soln)
@@ -3124,9 +3359,7 @@ int amrgpu_download_soln(amrgpu_ctx *c, double *soln)
     hipLaunchKernelGGL(soa_to_aos_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
                        c->U[c->cur], c->d_stage, ncells, n2);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(soln, c->d_stage, sizeof(double) * 4 * ncells, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return AMRGPU_OK;
+    return copy_out(c, soln, c->d_stage, sizeof(double) * 4 * ncells);
 }
 
 int amrgpu_download_quads(amrgpu_ctx *c, int first, int count, double *soln)
@@ -3142,9 +3375,7 @@ int amrgpu_download_quads(amrgpu_ctx *c, int first, int count, double *soln)
     hipLaunchKernelGGL(soa_to_aos_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
                        c->U[c->cur] + (size_t)first * 4 * n2, c->d_stage, ncells, n2);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(soln, c->d_stage, sizeof(double) * 4 * ncells, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return AMRGPU_OK;
+    return copy_out(c, soln, c->d_stage, sizeof(double) * 4 * ncells);
 }
 
 // position-dependent walls need the quadrant coordinates of the current mesh
@@ -3171,9 +3402,7 @@ int amrgpu_rhs(amrgpu_ctx *c, double *rhs)
     hipLaunchKernelGGL(soa_to_aos_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
                        c->U[other], c->d_stage, ncells, n2);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(rhs, c->d_stage, sizeof(double) * 4 * ncells, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return AMRGPU_OK;
+    return copy_out(c, rhs, c->d_stage, sizeof(double) * 4 * ncells);
 }
 
 int amrgpu_cfl(amrgpu_ctx *c, double *dt_inst)
@@ -3183,14 +3412,12 @@ int amrgpu_cfl(amrgpu_ctx *c, double *dt_inst)
     HIPCHK(hipGetLastError());
     int rc = launch_cfl(c, c->U[c->cur], c->slots(), nullptr);
     if (rc) return rc;
-    std::vector<unsigned long long> b((size_t)c->ninst * NSLOT);
-    HIPCHK(hipMemcpyAsync(b.data(), c->slots(), sizeof(unsigned long long) * b.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    for (int i = 0; i < c->ninst; ++i) {
-        unsigned long long mn = DBL_INF_BITS;
-        for (int k = 0; k < NSLOT; ++k) mn = std::min(mn, b[(size_t)i * NSLOT + k]);
-        memcpy(&dt_inst[i], &mn, sizeof(double));
-    }
+    // the sub-slots reduced on the device, straight into pinned memory
+    if ((rc = take_res(c, sizeof(double) * c->ninst))) return rc;
+    hipLaunchKernelGGL(slot_min_kernel, dim3(c->ninst), dim3(64), 0, c->stream, c->slots(), c->ninst, (double *)c->res.p);
+    HIPCHK(hipGetLastError());
+    if ((rc = sync_stream(c))) return rc;
+    memcpy(dt_inst, c->res.p, sizeof(double) * c->ninst);
     return AMRGPU_OK;
 }
 
@@ -3234,13 +3461,21 @@ static int step_next(amrgpu_ctx *c, int cur)
     return build_step(c, cur, st, false);
 }
 
+// The residual norm of the run's last stage, whose workgroups left a sum of squares
+// each: in pinned memory where they are few, else in device memory, from where
+// NORM_PARTS workgroups reduce them to as many sums there.
 static int finish_norm(amrgpu_ctx *c, double *resnorm)
 {
-    std::vector<double> part(c->nblocks);
-    HIPCHK(hipMemcpyAsync(part.data(), c->d_norm, sizeof(double) * c->nblocks, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    int n = c->nblocks;
+    if (n > NORM_DIRECT) {
+        hipLaunchKernelGGL(norm_kernel, dim3(NORM_PARTS), dim3(256), 0, c->stream, c->d_norm, n, (double *)c->res.p);
+        HIPCHK(hipGetLastError());
+        n = NORM_PARTS;
+    }
+    if (int rc = sync_stream(c)) return rc;
+    const double *part = (const double *)c->res.p;
     double s = 0.0;
-    for (double v : part) s += v;
+    for (int k = 0; k < n; ++k) s += part[k];
     double rn = sqrt(s);
     if (resnorm) *resnorm = rn;
     if (std::isnan(rn)) { set_err("nan detected in residual"); return AMRGPU_ERR_NAN; }
@@ -3269,7 +3504,8 @@ int amrgpu_run(amrgpu_ctx *c, int nsteps, int use_graph, double *resnorm)
 {
     if (!c || !c->nquad || nsteps < 0) { set_err("amrgpu_run: no mesh"); return AMRGPU_ERR_ARG; }
     if (nsteps == 0) return AMRGPU_OK;
-    int rc = prime_run(c);
+    int rc = take_res(c, sizeof(double) * NORM_DIRECT);
+    if (!rc) rc = prime_run(c);
     if (rc) return rc;
     // the residual norm (NaN check, reported norm) is taken on the last stage
     // of the last step, the only value the reference keeps
@@ -3277,32 +3513,40 @@ int amrgpu_run(amrgpu_ctx *c, int nsteps, int use_graph, double *resnorm)
         rc = one_step(c, use_graph != 0, s == nsteps - 1);
         if (rc) return rc;
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
     return finish_norm(c, resnorm);
 }
 
 int amrgpu_get_time(amrgpu_ctx *c, double *t_inst, double *dt_inst)
 {
     if (!c || !c->nquad) { set_err("amrgpu_get_time: no mesh"); return AMRGPU_ERR_ARG; }
-    if (t_inst) HIPCHK(hipMemcpyAsync(t_inst, c->t_now(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
-    if (dt_inst) HIPCHK(hipMemcpyAsync(dt_inst, c->dt_cur(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    // both times and the last dt lie together: one copy
+    const size_t ci = c->cap_inst;
+    if (int rc = take_res(c, sizeof(double) * 3 * ci)) return rc;
+    HIPCHK(hipMemcpyAsync(c->res.p, c->d_clock, sizeof(double) * 3 * ci, hipMemcpyDeviceToHost, c->stream));
+    if (int rc = sync_stream(c)) return rc;
+    const double *h = (const double *)c->res.p;
+    if (t_inst) memcpy(t_inst, h + c->tb * ci, sizeof(double) * c->ninst);
+    if (dt_inst) memcpy(dt_inst, h + 2 * ci, sizeof(double) * c->ninst);
     return AMRGPU_OK;
 }
 
 int amrgpu_set_time(amrgpu_ctx *c, const double *t_inst)
 {
     if (!c || !c->nquad || !t_inst) { set_err("amrgpu_set_time: no mesh"); return AMRGPU_ERR_ARG; }
-    HIPCHK(hipMemcpyAsync(c->t_now(), t_inst, sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->t_step(), t_inst, sizeof(double) * c->ninst, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return AMRGPU_OK;
+    if (int rc = sync_stream(c)) return rc;
+    if (int rc = take_res(c, sizeof(double) * c->ninst)) return rc;
+    memcpy(c->res.p, t_inst, sizeof(double) * c->ninst);
+    hipLaunchKernelGGL(clock_kernel, dim3(1), dim3(64), 0, c->stream, c->t_now(), (double *)nullptr, c->t_step(),
+                       (const double *)c->res.p, c->ninst);
+    HIPCHK(hipGetLastError());
+    return sync_stream(c);
 }
 
 int amrgpu_bench(amrgpu_ctx *c, int nsteps, double *ms_total, double *avg_stage_ms, int *nstages)
 {
     if (!c || !c->nquad || nsteps <= 0) { set_err("amrgpu_bench: no mesh"); return AMRGPU_ERR_ARG; }
-    int rc = prime_run(c);
+    int rc = take_res(c, sizeof(double) * NORM_DIRECT);
+    if (!rc) rc = prime_run(c);
     if (rc) return rc;
     // in graph mode, capture the graphs of every starting buffer before timing
     if (c->graphs_enabled) {
@@ -3364,7 +3608,6 @@ int amrgpu_bench(amrgpu_ctx *c, int nsteps, double *ms_total, double *avg_stage_
     // one more step carrying the residual norm: NaN check of the result
     rc = one_step(c, false, true);
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(c->stream));
     return finish_norm(c, nullptr);
 }
 
@@ -3560,16 +3803,6 @@ __global__ void noalloc_prep_kernel(InstDev *ip, unsigned long long *slot, int n
     for (int i = threadIdx.x; i < ninst * NSLOT; i += blockDim.x) slot[i] = DBL_INF_BITS;
 }
 
-__global__ void noalloc_finish_kernel(const unsigned long long *slot, int ninst, double *dt)
-{
-    // one wave per instance
-    const int i = blockIdx.x;
-    if (i < ninst) {
-        const double m = slot_min(slot, i);
-        if (threadIdx.x == 0) dt[i] = m;
-    }
-}
-
 int noalloc_scratch(void **out)
 {
     int dev = 0;
@@ -3627,7 +3860,7 @@ int amrgpu_cfl_noalloc(int nelem_subgrid, int nquad, int ninst, const double *h_
     default: hipLaunchKernelGGL((cfl_kernel<16, 1>), dim3(nblk), dim3(256), 0, st, m, d_U, slot, none); break;
     }
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(noalloc_finish_kernel, dim3(ninst), dim3(64), 0, st, slot, ninst, d_dt);
+    hipLaunchKernelGGL(slot_min_kernel, dim3(ninst), dim3(64), 0, st, slot, ninst, d_dt);
     HIPCHK(hipGetLastError());
     return AMRGPU_OK;
 }

@@ -989,15 +989,7 @@ int amrgpu_tagger_features_host(amrgpu_ctx *c, uint16_t *X)
     uint16_t *d = nullptr;
     MCHK(hipMalloc((void **)&d, sizeof(uint16_t) * (size_t)nquad * NIN));
     rc = amrgpu_tagger_features(c, d);
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(X, d, sizeof(uint16_t) * (size_t)nquad * NIN, hipMemcpyDeviceToHost,
-                                      (hipStream_t)st);
-        if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)st);
-        if (e != hipSuccess) {
-            amr_set_error("amrgpu_tagger_features_host: %s", hipGetErrorString(e));
-            rc = AMRGPU_ERR_HIP;
-        }
-    }
+    if (!rc) rc = amrgpu_fetch(c, X, d, sizeof(uint16_t) * (size_t)nquad * NIN);
     (void)hipFree(d);
     return rc;
 }
@@ -1077,9 +1069,7 @@ int amr_mlp_predict_ctx(amr_mlp_t *m, amrgpu_ctx *c, int *cls)
     if (!rc) rc = amrgpu_tagger_features(c, m->X);
     if (!rc) rc = launch_infer(m, m->X, nquad, nullptr, m->cls, (hipStream_t)st);
     if (rc) return rc;
-    MCHK(hipMemcpyAsync(cls, m->cls, sizeof(int) * nquad, hipMemcpyDeviceToHost, (hipStream_t)st));
-    MCHK(hipStreamSynchronize((hipStream_t)st));
-    return AMRGPU_OK;
+    return amrgpu_fetch(c, cls, m->cls, sizeof(int) * (size_t)nquad);
 }
 
 }  // extern "C"

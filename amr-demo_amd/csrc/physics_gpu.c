@@ -154,6 +154,17 @@ static amrgpu_inst_t inst_from_params(void)
     return ip;
 }
 
+/* the interval's arrays on the device, at time *t (NULL: 0) */
+static int setup_faces(int n, const amrgpu_inst_t *ip, int ncell, const int *cell_info, int nface,
+                       const int *face_info, const double *geom, const double *soln, const double *t)
+{
+    if (!face_info) {
+        amr_set_error("amrgpu_setup: bad arguments");
+        return AMRGPU_ERR_ARG;
+    }
+    return amrgpu_setup_from(g_ctx, n, g_p.time_scheme, 1, ip, ncell, cell_info, NULL, nface, face_info, geom, soln, t);
+}
+
 /* steps until the next multiple of interval (the reference stops when
  * istep % interval == 0 after incrementing) */
 static long long to_next(int istep, int interval)
@@ -193,13 +204,11 @@ int physics_go_gpu(int *dim, int *unstructured, int *nfields, int *nelem_subgrid
 
     double t1 = wall();
     amrgpu_inst_t ip = inst_from_params();
-    rc = amrgpu_setup(g_ctx, *nelem_subgrid, g_p.time_scheme, 1, &ip, *ncell, cell_info, NULL,
-                      *nface, face_info, geom, soln);
+    rc = setup_faces(*nelem_subgrid, &ip, *ncell, cell_info, *nface, face_info, geom, soln, &g_time);
     if (rc) {
         fprintf(stderr, "[physics] GPU setup failed: %s\n", amrgpu_last_error());
         return rc;
     }
-    if ((rc = amrgpu_set_time(g_ctx, &g_time))) return rc;
 
     /* steps this interval: physics_runge_kutta_interface.c:213-229 */
     long long n = (long long)g_p.time_steps - *istep;
@@ -284,8 +293,7 @@ int physics_rhs_structured_gpu(int *dim, int *nfields, int *nelem_subgrid, int *
     if ((rc = check_structured(dim, nfields))) return rc;
     if ((rc = ensure_ctx())) return rc;
     amrgpu_inst_t ip = inst_from_params();
-    rc = amrgpu_setup(g_ctx, *nelem_subgrid, g_p.time_scheme, 1, &ip, *ncell, cell_info, NULL,
-                      *nface, face_info, geom, soln);
+    rc = setup_faces(*nelem_subgrid, &ip, *ncell, cell_info, *nface, face_info, geom, soln, NULL);
     if (rc) return rc;
     return amrgpu_rhs(g_ctx, rhs);
 }
@@ -296,19 +304,10 @@ int physics_time_step_gpu(int *dim, int *nfields, int *nelem_subgrid, int *ncell
     int rc;
     if ((rc = check_structured(dim, nfields))) return rc;
     if ((rc = ensure_ctx())) return rc;
-    /* the time step needs no faces: build a boundary-only table */
-    int *fi = (int *)malloc(sizeof(int) * 11 * 4 * (size_t)(*ncell));
-    if (!fi) return AMRGPU_ERR_ARG;
-    for (int c = 0; c < *ncell; ++c)
-        for (int s = 0; s < 4; ++s) {
-            int *f = &fi[11 * (4 * c + s)];
-            for (int e = 0; e < 11; ++e) f[e] = -1;
-            f[0] = 1; f[1] = s; f[2] = c;
-        }
+    /* the time step needs no faces */
     amrgpu_inst_t ip = inst_from_params();
-    rc = amrgpu_setup(g_ctx, *nelem_subgrid, g_p.time_scheme, 1, &ip, *ncell, cell_info, NULL,
-                      4 * (*ncell), fi, geom, soln);
-    free(fi);
+    rc = amrgpu_setup_from(g_ctx, *nelem_subgrid, g_p.time_scheme, 1, &ip, *ncell, cell_info, NULL, 0, NULL, geom, soln,
+                           NULL);
     if (rc) return rc;
     double d;
     if ((rc = amrgpu_cfl(g_ctx, &d))) return rc;
