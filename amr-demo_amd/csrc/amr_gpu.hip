@@ -1580,6 +1580,204 @@ __device__ __forceinline__ unsigned here(unsigned v)
     return v;
 }
 
+// The value that lane l + 32 holds, in lane l < 32.
+__device__ __forceinline__ double upper_half(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)b, hi = (int)(b >> 32);
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __longlong_as_double(((long long)h[1] << 32) | (unsigned)l[1]);
+}
+
+// ---------------------------------------------------------------------------
+// Stage kernel of the 8x8 tiles with one patch a workgroup: one wave,
+// one cell a lane.  A lane evaluates its cell's +x and +y faces, then one face of
+// the patch's edge: cell k of side s with its first neighbour in lane 8 s + k,
+// with the second fine one in lane 32 + 8 s + k, which loads that neighbour's
+// cell itself.  So no round waits on the halo before the first (its loads travel
+// behind the interior faces), every halo cell becomes a record once, there is no
+// task list, and a coarse side's two fluxes are added in registers.  The
+// arithmetic of a face and the order of the sums are stage_kernel's: the results
+// are bit for bit those of the other tiles.
+//
+// What bounds it: on a small mesh the wave's own chain (neighbour ids, halo,
+// three flux rounds).  On a large one the card's power: at 8.4M cells the VALU is
+// busy 87 % of the time and the clock falls to 2.0 GHz, so that an instruction
+// taken out of idle lanes counts as much as one taken out of the stream.  Lanes
+// without an edge face are masked off, their loads included (without that: 4 %
+// slower there), and the LDS layouts are free of bank conflicts but for the
+// edges' own columns against the halo.
+// Measured, us per SSP-RK3 step, stage_kernel (paired faces, +x and +y halo in
+// the first round) -> this: 2.6k quadrants (adaptive) 23.7 -> 21.4, 18.8k
+// 88 -> 84, 159k 700 -> 664, 131k uniform 547 -> 524.
+// ---------------------------------------------------------------------------
+template <int MINW, bool SELF = false>
+__global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
+{
+    constexpr int N = 8;
+    using TL = Tile<N, 1>;
+    constexpr int N2 = N * N, ST = N * (N + 1), FY = NFLD * ST, FACE = TL::face(0);
+    static_assert(TL::SPLIT && 8 * N == N2, "a halo cell of each kind per lane");
+    __shared__ double lds[TL::LDS_DOUBLES];
+    typedef double __attribute__((address_space(1))) gdbl;
+    typedef const double __attribute__((address_space(1))) gcdbl;
+    typedef const int __attribute__((address_space(4))) cint4;
+    typedef const double __attribute__((address_space(4))) cdbl4;
+    typedef const InstDev __attribute__((address_space(4))) cinst4;
+
+    const int c = threadIdx.x, ci = c % N, cj = c / N;
+    const int q = xcd_block(blockIdx.x, gridDim.x);
+    const size_t quad = (size_t)q * (NFLD * N2);
+    // where a cell's record lies: the halves of the upper rows exchanged, so that
+    // a column's eight cells are on banks of their own
+    auto at = [](int cell) { return cell ^ ((cell >> 3) & 4); };
+    // where face i of row j lies among a field's x faces: four rows by column, so
+    // that an access's 32 lanes are on banks of their own
+    auto xface = [](int i, int j) { return (j >> 2) * (4 * N + 4) + i * 4 + (j & 3); };
+
+    double U[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) U[f] = (gptr(a.Us) + quad + f * N2)[c];
+    const cint4 *const nbc = (const cint4 *)a.m.nbr + (size_t)q * 8;
+    int nb[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) nb[k] = nbc[k];
+    const int lev = ((const cint4 *)a.m.level)[q], inst = ((const cint4 *)a.m.inst)[q];
+    const bool any_second = nb[1] >= 0 || nb[3] >= 0 || nb[5] >= 0 || nb[7] >= 0;
+    const bool any_wall = nb[0] < 0 || nb[2] < 0 || nb[4] < 0 || nb[6] < 0;
+    // the lane's edge face: cell k of the side (-x, +x, -y, +y), its first
+    // neighbour in the lower lanes, the second fine one in the upper
+    const bool second = c >= 4 * N;
+    const int side = c / N % 4, k = c % N;
+    const bool sx = side < 2, high = side & 1;
+    const int na = sx ? (high ? nb[2] : nb[0]) : (high ? nb[6] : nb[4]);
+    const int n2 = sx ? (high ? nb[3] : nb[1]) : (high ? nb[7] : nb[5]);
+    const int kb = sx ? k * N : k, far = sx ? N - 1 : (N - 1) * N;
+    const int own = kb + (high ? far : 0);
+    const bool edge = !second || any_second;
+    double G[4];
+    if (edge) {
+        // a wall: the own edge cell, so that the flux stays finite until the
+        // boundary's replaces it (upper lanes without a neighbour: unused)
+        const int id = second ? n2 : na;
+        gcdbl *const g = gptr(a.Us) + (id < 0 ? quad + own : (size_t)id * (NFLD * N2) + kb + (high ? 0 : far));
+#pragma unroll
+        for (int f = 0; f < 4; ++f) G[f] = g[f * N2];
+    }
+    const cinst4 *const ipc = (const cinst4 *)a.m.ip + inst;
+    const double h = ldexp(ipc->h_base, -lev) / (double)N;
+    const double tw = ((const cdbl4 *)(SELF ? a.t_in : a.m.t_step))[inst];
+    double dt = 0.0;
+    if (!SELF && a.mode != MODE_RHS) dt = ((const cdbl4 *)a.dt_cur)[inst];
+
+    // ---- the faces between the patch's cells, while the halo is on its way ------
+    store_rec<N, 1>(lds, 0, at(c), U[0], U[1], U[2], U[3]);
+    lds_order();
+    double FA[4], FB[4];
+    {
+        Prim L, RX, RY;
+        load_prim<N, 1>(lds, 0, at(c), L);
+        load_prim<N, 1>(lds, 0, at(ci == N - 1 ? c : c + 1), RX);
+        load_prim<N, 1>(lds, 0, at(cj == N - 1 ? c : c + N), RY);
+        flux_face<true>(L, RX, h, FA);
+        flux_face<false>(L, RY, h, FB);
+        // both complete here (see stage_kernel)
+        asm volatile("" : "+v"(FA[0]), "+v"(FA[1]), "+v"(FA[2]), "+v"(FA[3]), "+v"(FB[0]), "+v"(FB[1]),
+                     "+v"(FB[2]), "+v"(FB[3]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- the edges' faces ---------------------------------------------------------
+    if (edge) {
+        store_rec<N, 1>(lds, 0, TL::GHOST + c, G[0], G[1], G[2], G[3]);
+        lds_order();
+        const int offn = sx ? N2 : 2 * N2, offt = 3 * N2 - offn;
+        OPrim L, R;
+        load_oprim<N, 1>(lds, 0, high ? at(own) : TL::GHOST + c, offn, offt, L);
+        load_oprim<N, 1>(lds, 0, high ? TL::GHOST + c : at(own), offn, offt, R);
+        flux_normal(L, R, n2 >= 0 ? 0.5 * h : h, G);
+        if (any_wall) {
+            if (na < 0 && !second) {
+                const double nh = high ? h : -h, fe = high ? (double)N : 0.0;
+                const double nrm[2] = {sx ? nh : 0.0, sx ? 0.0 : nh};
+                const double *const u = lds + at(own);
+                const double uo[4] = {u[0], u[N2], u[2 * N2], u[3 * N2]};
+                double F[4];
+                flux_boundary(a.m.ip[inst], side, nrm, uo, a.m.org + 2 * (size_t)q, sx ? fe : k + 0.5,
+                              sx ? k + 0.5 : fe, h, tw, F);
+                const double sg = high ? 1.0 : -1.0;
+                G[0] = sg * F[0]; G[1] = sg * (sx ? F[1] : F[2]); G[2] = sg * (sx ? F[2] : F[1]); G[3] = sg * F[3];
+            }
+        }
+        if (any_second) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                const double S = upper_half(G[f]);
+                if (n2 >= 0) G[f] += S;
+            }
+        }
+    }
+    // the base state is asked for late: an earlier load is no faster on small
+    // meshes and slows the memory on large ones (8.4M cells 566 -> 598 us a step)
+    const bool needB = (a.mode == MODE_SO && a.U0) || a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL;
+    double B[4];
+    if (needB) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) B[f] = (gptr(a.U0) + quad + f * N2)[c];
+    }
+    if constexpr (SELF) {
+        const double cm = a.use_cfl ? slot_min(a.slot_in, inst) : INFINITY;
+        dt = uniform_f64(limited_dt(ipc->dt_cap, ipc->t_end, cm, tw, a.use_cfl));
+        if (q == 0 || ((const cint4 *)a.m.inst)[q - 1] != inst) publish_dt(a, inst, dt, tw);
+    }
+    // ---- the fluxes over the records but for the cells' r, ru, rv, rE --------------
+    lds_order();
+    {
+        double *const fa = lds + FACE + xface(ci + 1, cj), *const fb = lds + FACE + FY + (cj + 1) * N + ci;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            fa[f * ST] = FA[f];
+            fb[f * ST] = FB[f];
+        }
+        lds_order();
+        if (!second) {         // the high edges' over what their cells left there
+            double *const d = lds + FACE + (sx ? xface(high ? N : 0, k) : FY + (high ? N2 : 0) + k);
+            const int on = sx ? ST : 2 * ST;
+            d[0] = G[0]; d[on] = G[1]; d[3 * ST - on] = G[2]; d[3 * ST] = G[3];
+        }
+    }
+    lds_order();
+    // ---- per-cell residual and stage update ----------------------------------------
+    const double ninvV = ldexp(ipc->ninv_vol0, 2 * lev);
+    double k4[4], out[4];
+    {
+        const double *const xr = lds + FACE + xface(ci + 1, cj), *const xl = lds + FACE + xface(ci, cj);
+        const double *const yb = lds + FACE + FY + c;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            U[f] = lds[f * N2 + at(c)];
+            k4[f] = ((xr[f * ST] - xl[f * ST]) + (yb[f * ST + N] - yb[f * ST])) * ninvV;
+        }
+    }
+    stage_update(a, quad + c, N2, dt, U, B, k4, out);
+    // past its stop an instance keeps its state bit for bit (see stage_kernel)
+    if (__builtin_amdgcn_readfirstlane((int)(a.mode != MODE_RHS && dt == 0.0))) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) out[f] = U[f];
+    }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) __builtin_nontemporal_store(out[f], (gdbl *)(a.Uout + quad + f * N2) + c);
+    if (a.role & ROLE_CFL)
+        cfl_reduce<N2>(cfl_candidate_h(out, ldexp(ipc->cfl_h0, -lev)), inst, true, inst, a.slot, nullptr);
+    if (a.norm_part) {
+        double sq = 0.0;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) sq = fma(k4[f], k4[f], sq);
+        sq = wave_sum(sq);
+        if (c == 0) a.norm_part[blockIdx.x] = sq;
+    }
+}
+
 // SELF: the first stage of a step without dt_prep_kernel.
 template <int N, int R, int VEC, bool SELF = false>
 __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
@@ -2377,10 +2575,11 @@ int grid_of(const amrgpu_ctx *c, int v, int nquad)
 
 
 // Stage-kernel tile used until amrgpu_set_tile / amrgpu_autotune picks one
-// (every tile computes the same bits): for n = 8 and 16 the paired-faces
-// tile with one patch per workgroup and five waves per SIMD, the fastest or
-// within 2 % of it on the meshes measured (1k to 16.8M cells; four waves at 8x8:
-// 4096 quadrants 28.0 against 26.9 us a step, 18750 94.5 against 90.2).
+// (every tile computes the same bits): for n = 8 and 16 the tile with one patch
+// per workgroup and five waves per SIMD, the fastest or within 2 % of it on the
+// meshes measured (1k to 16.8M cells; four and five waves at 8x8: 2.6k quadrants
+// 21.4 and 21.4 us a step, 18.8k 85.9 and 84.0, 159k 672 and 664, 131k uniform
+// 522 and 526).
 // n = 2 and 4: the row-marching kernel, faster than the others at every size
 // measured (16 to 262k quadrants).  n = 4 takes two rows a step, with fewer
 // instructions a patch, where its waves of 8 patches fill the chip (256 CUs x
@@ -2426,7 +2625,13 @@ template <int N, int PPB, int MINW, int D>
 int launch_v(amrgpu_ctx *c, const StageArgs &a)
 {
     int nblk = (c->nquad + PPB - 1) / PPB;
-    if constexpr (D == 1 && PPB == 1 && MINW >= 4) {
+    if constexpr (N == 8 && D == 1 && PPB == 1) {
+        if (a.slot_in) hipLaunchKernelGGL((stage_kernel_one<MINW, true>), dim3(nblk), dim3(64), 0, c->stream, a);
+        else hipLaunchKernelGGL((stage_kernel_one<MINW>), dim3(nblk), dim3(64), 0, c->stream, a);
+        HIPCHK(hipGetLastError());
+        return AMRGPU_OK;
+    }
+    if constexpr (N == 16 && D == 1 && PPB == 1 && MINW >= 4) {
         if (a.slot_in) {
             hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D, true>), dim3(nblk), dim3(Tile<N, PPB>::BLK), 0, c->stream, a);
             HIPCHK(hipGetLastError());
