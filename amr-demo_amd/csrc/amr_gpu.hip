@@ -102,6 +102,7 @@ struct StageArgs {
     double *t_step;      // MeshDev's, for the step's other stages
     int use_cfl;
     double *norm_part;
+    bool down;           // the launch goes through the patches from the end (launch_stage)
     int per_block;       // persistent design: patches per workgroup (a contiguous range)
 };
 
@@ -119,12 +120,23 @@ __device__ __forceinline__ const double __attribute__((address_space(1))) *gptr(
 // Logical block index with each XCD receiving a contiguous range, so that
 // Morton-adjacent patches (which share halo cells) are processed by the same
 // XCD and its L2.  Workgroups are dispatched round-robin over the 8 XCDs.
-__device__ __forceinline__ int xcd_block(int b, int nblk)
+// down: each XCD goes through its range from the end.
+__device__ __forceinline__ int xcd_block(int b, int nblk, bool down = false)
 {
     const int NX = 8;
     int q = nblk / NX, r = nblk % NX;
     int x = b % NX, k = b / NX;
+    if (down) k = q - (x < r ? 0 : 1) - k;
     return x * q + (x < r ? x : r) + k;
+}
+
+// Streamed out (no other wave of the launch reads it), or left in the caches for
+// the next launch (streams_out).
+template <bool NT, class T>
+__device__ __forceinline__ void put_state(T *p, double v)
+{
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
 }
 
 struct Prim {
@@ -657,7 +669,7 @@ __device__ __forceinline__ void stage_update(const StageArgs &a, size_t base, in
 }
 
 // SELF: the first stage of a step without dt_prep_kernel (one-patch tiles).
-template <int N, int PPB, int MINW, int DESIGN, bool SELF = false>
+template <int N, int PPB, int MINW, int DESIGN, bool SELF = false, bool NT = true>
 __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(StageArgs a)
 {
     using TL = Tile<N, PPB>;
@@ -674,7 +686,7 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
 
     const int tid = threadIdx.x;
     const int nblk = gridDim.x;
-    const int lb = xcd_block(blockIdx.x, nblk);
+    const int lb = xcd_block(blockIdx.x, nblk, a.down);
     const int p = tid / N2, c = tid % N2;
     const int ci = c % N, cj = c / N;
     const int quad = lb * PPB + p;
@@ -1197,8 +1209,7 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
             for (int f = 0; f < 4; ++f) out[f] = U[f];
         }
 #pragma unroll
-        for (int f = 0; f < 4; ++f)   // streamed out: no other wave of this launch reads it
-            __builtin_nontemporal_store(out[f], &a.Uout[base + f * N2]);
+        for (int f = 0; f < 4; ++f) put_state<NT>(&a.Uout[base + f * N2], out[f]);
         if (a.role & ROLE_CFL) cand = cfl_candidate_h(out, cflh);
     }
     if (a.role & ROLE_CFL) {
@@ -1208,7 +1219,7 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
             if (pquad[k] >= 0 && pinst[k] != uinst) uinst = -1;
         cfl_reduce<TL::BLK>(cand, active ? (SMETA ? inw : pinst[p]) : 0, active, uinst, a.slot, red);
     }
-    if (a.norm_part) sum_reduce_store<TL::BLK>(sq, &a.norm_part[blockIdx.x], red);
+    if (a.norm_part) sum_reduce_store<TL::BLK>(sq, &a.norm_part[lb], red);
 }
 
 
@@ -1302,7 +1313,7 @@ __global__ __launch_bounds__(N * N, MINW) void stage_kernel_pp(StageArgs a)
 
     const int tid = threadIdx.x, c = tid;
     const int ci = c % N, cj = c / N;
-    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int lb = xcd_block(blockIdx.x, gridDim.x, a.down);
     const int q0 = lb * a.per_block;
     const int q1 = min(q0 + a.per_block, a.m.nquad);
     const bool needB = (a.mode == MODE_SO && a.U0) || a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL;
@@ -1503,7 +1514,7 @@ __global__ __launch_bounds__(N * N, MINW) void stage_kernel_pp(StageArgs a)
         for (int k = 0; k < 8; ++k) nbw[k] = nbn[k];
     }
     if ((a.role & ROLE_CFL) && cinst >= 0) cfl_reduce<N2>(cmin, cinst, true, cinst, a.slot, red);
-    if (a.norm_part) sum_reduce_store<N2>(sq, &a.norm_part[blockIdx.x], red);
+    if (a.norm_part) sum_reduce_store<N2>(sq, &a.norm_part[lb], red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1614,7 +1625,7 @@ __device__ __forceinline__ double upper_half(double v)
 // the first round) -> this: 2.6k quadrants (adaptive) 23.7 -> 21.4, 18.8k
 // 88 -> 84, 159k 700 -> 664, 131k uniform 547 -> 524.
 // ---------------------------------------------------------------------------
-template <int MINW, bool SELF = false>
+template <int MINW, bool SELF, bool NT>
 __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
 {
     constexpr int N = 8;
@@ -1629,7 +1640,7 @@ __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
     typedef const InstDev __attribute__((address_space(4))) cinst4;
 
     const int c = threadIdx.x, ci = c % N, cj = c / N;
-    const int q = xcd_block(blockIdx.x, gridDim.x);
+    const int q = xcd_block(blockIdx.x, gridDim.x, a.down);
     const size_t quad = (size_t)q * (NFLD * N2);
     // where a cell's record lies: the halves of the upper rows exchanged, so that
     // a column's eight cells are on banks of their own
@@ -1768,7 +1779,7 @@ __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
         for (int f = 0; f < 4; ++f) out[f] = U[f];
     }
 #pragma unroll
-    for (int f = 0; f < 4; ++f) __builtin_nontemporal_store(out[f], (gdbl *)(a.Uout + quad + f * N2) + c);
+    for (int f = 0; f < 4; ++f) put_state<NT>((gdbl *)(a.Uout + quad + f * N2) + c, out[f]);
     if (a.role & ROLE_CFL)
         cfl_reduce<N2>(cfl_candidate_h(out, ldexp(ipc->cfl_h0, -lev)), inst, true, inst, a.slot, nullptr);
     if (a.norm_part) {
@@ -1776,12 +1787,12 @@ __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
 #pragma unroll
         for (int f = 0; f < 4; ++f) sq = fma(k4[f], k4[f], sq);
         sq = wave_sum(sq);
-        if (c == 0) a.norm_part[blockIdx.x] = sq;
+        if (c == 0) a.norm_part[q] = sq;
     }
 }
 
 // SELF: the first stage of a step without dt_prep_kernel.
-template <int N, int R, int VEC, bool SELF = false>
+template <int N, int R, int VEC, bool SELF, bool NT>
 __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
 {
     constexpr int N2 = N * N, P = 64 / (N * R), STEPS = N / R, QS = NFLD * N2;
@@ -1805,7 +1816,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
     gdbl *const Us = (gdbl *)a.Us;
     const int lane = threadIdx.x;
     const int nq = a.m.nquad;
-    const int g = xcd_block(blockIdx.x, gridDim.x);
+    const int g = xcd_block(blockIdx.x, gridDim.x, a.down);
     const int ci = lane % N, rr = (lane / N) % R, p = lane / (N * R);
     const int e = p * N + ci;                      // position along the wave's -y and +y edges
     // the lane's halo cells: sides -x, -y, +x, +y of the wave's patches in turn
@@ -2072,7 +2083,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
             gcout *const ob = (gcout *)(gout *)(a.Uout + (size_t)g * (P * QS) + R * N * s);
             const unsigned o = here(off);
 #pragma unroll
-            for (int f = 0; f < 4; ++f) __builtin_nontemporal_store(out[f], (gout *)(ob + f * N2 * 8 + o));
+            for (int f = 0; f < 4; ++f) put_state<NT>((gout *)(ob + f * N2 * 8 + o), out[f]);
             if (VEC == VEC_ACC || (VEC == VEC_BOTH && a.mode == MODE_RK4_ACC)) {
                 gcout *const ab = (gcout *)(gout *)(a.Acc + (size_t)g * (P * QS) + R * N * s);
 #pragma unroll
@@ -2096,7 +2107,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
     }
     if (a.norm_part) {
         sq = wave_sum(sq);
-        if (lane == 0) a.norm_part[blockIdx.x] = sq;
+        if (lane == 0) a.norm_part[g] = sq;
     }
 }
 
@@ -2484,6 +2495,7 @@ struct amrgpu_ctx {
     double *d_clock = nullptr;
     unsigned long long *d_slot_sets = nullptr; // three sets of CFL sub-slots, by sb
     int tb = 0, sb = 0;
+    bool sweep_down = false;                   // direction of the next stage launch
     bool self_dt = false;                      // this run's steps have no dt_prep_kernel
     bool all_inst = true;                      // every instance has quadrants
     double *t_now(int ahead = 0) const { return d_clock + (size_t)((tb + ahead) & 1) * cap_inst; }
@@ -2623,24 +2635,52 @@ int launch_pp(amrgpu_ctx *c, const StageArgs &a0)
     return AMRGPU_OK;
 }
 
+// Whether a stage's state is streamed past the caches.  The last-level cache holds
+// 256 MB: where the vectors a step goes through fit, a state left there is read from
+// it by the next stage (us per step streamed / left, launches in alternating
+// directions: 8x8 SSP-RK3 100 MB 69 / 65, 200 MB 128 / 119; 4x4 128 MB 157 / 136;
+// 16x16 LSERK45 100 MB 151 / 132, 229 MB 313 / 282).  Beyond it what fits still
+// counts for the Shu-Osher forms (4x4 270 MB 229 / 212, 400 MB 303 / 285; 8x8
+// 300 to 980 MB equal within 1 %), while the accumulator of the other two, read and
+// written by every stage, is better off with the cache to itself (16x16 LSERK45
+// 302 MB 399 / 433, 400 MB 547 / 554, 805 MB 1040 / 1063; 8x8 RK4 268 MB 221 / 194,
+// 400 MB 327 / 335).  Small states would only be written back from the L2s at the
+// launch's end (16 to 33 MB: 2 to 4 % slower left, 50 MB 0 to 5 % faster).
+bool streams_out(const amrgpu_ctx *c)
+{
+    const int vectors = c->scheme <= 2 ? 2 : c->scheme == 4 ? 4 : 3;
+    const long long bytes = (long long)c->nquad * c->n * c->n * NFLD * sizeof(double) * vectors;
+    return bytes < 40000000 || (c->scheme >= 4 && bytes > 280000000);
+}
+
+// f(self, nt): a first stage that forms the step's dt, a state streamed out.
+template <class F>
+void with_flags(const amrgpu_ctx *c, const StageArgs &a, F f)
+{
+    std::true_type yes;
+    std::false_type no;
+    const bool nt = streams_out(c);
+    if (a.slot_in) nt ? f(yes, yes) : f(yes, no);
+    else nt ? f(no, yes) : f(no, no);
+}
+
 template <int N, int PPB, int MINW, int D>
 int launch_v(amrgpu_ctx *c, const StageArgs &a)
 {
-    int nblk = (c->nquad + PPB - 1) / PPB;
-    if constexpr (N == 8 && D == 1 && PPB == 1) {
-        if (a.slot_in) hipLaunchKernelGGL((stage_kernel_one<MINW, true>), dim3(nblk), dim3(64), 0, c->stream, a);
-        else hipLaunchKernelGGL((stage_kernel_one<MINW>), dim3(nblk), dim3(64), 0, c->stream, a);
-        HIPCHK(hipGetLastError());
-        return AMRGPU_OK;
+    const dim3 nblk((c->nquad + PPB - 1) / PPB), blk(Tile<N, PPB>::BLK);
+    if constexpr (D == 1 && PPB == 1) {
+        with_flags(c, a, [&](auto self, auto nt) {
+            constexpr bool SELF = decltype(self)::value, NT = decltype(nt)::value;
+            if constexpr (SELF && MINW < 4)
+                return;        // (has_self)
+            else if constexpr (N == 8)
+                hipLaunchKernelGGL((stage_kernel_one<MINW, SELF, NT>), nblk, blk, 0, c->stream, a);
+            else
+                hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D, SELF, NT>), nblk, blk, 0, c->stream, a);
+        });
+    } else {
+        hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D>), nblk, blk, 0, c->stream, a);
     }
-    if constexpr (N == 16 && D == 1 && PPB == 1 && MINW >= 4) {
-        if (a.slot_in) {
-            hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D, true>), dim3(nblk), dim3(Tile<N, PPB>::BLK), 0, c->stream, a);
-            HIPCHK(hipGetLastError());
-            return AMRGPU_OK;
-        }
-    }
-    hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D>), dim3(nblk), dim3(Tile<N, PPB>::BLK), 0, c->stream, a);
     HIPCHK(hipGetLastError());
     return AMRGPU_OK;
 }
@@ -2651,9 +2691,10 @@ int launch_rows(amrgpu_ctx *c, const StageArgs &a)
     constexpr int P = 64 / (N * R);
     const dim3 nblk((c->nquad + P - 1) / P);
     auto go = [&](auto vec) {
-        constexpr int VEC = decltype(vec)::value;
-        if (a.slot_in) hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC, true>), nblk, dim3(64), 0, c->stream, a);
-        else hipLaunchKernelGGL((stage_kernel_rows<N, R, VEC>), nblk, dim3(64), 0, c->stream, a);
+        with_flags(c, a, [&](auto self, auto nt) {
+            hipLaunchKernelGGL((stage_kernel_rows<N, R, decltype(vec)::value, decltype(self)::value, decltype(nt)::value>),
+                               nblk, dim3(64), 0, c->stream, a);
+        });
     };
     if (a.mode == MODE_LSERK) go(std::integral_constant<int, VEC_ACC>());
     else if (a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL) go(std::integral_constant<int, VEC_BOTH>());
@@ -2662,8 +2703,15 @@ int launch_rows(amrgpu_ctx *c, const StageArgs &a)
     return AMRGPU_OK;
 }
 
-int launch_stage(amrgpu_ctx *c, const StageArgs &a)
+// Launches go through the patches up and down in turn: a stage begins with what
+// the one before it wrote last, which the last-level cache still holds (us per step
+// always up -> in turn: 8x8 131k quadrants 513 -> 501, 159k 652 -> 641, 4x4 262k
+// 302 -> 285, 16x16 LSERK45 16k 603 -> 554; meshes that fit the cache 0 to 3 %).
+int launch_stage(amrgpu_ctx *c, const StageArgs &a0)
 {
+    StageArgs a = a0;
+    a.down = c->sweep_down;
+    c->sweep_down = !c->sweep_down;
     switch (c->variant) {
     case 0: return launch_v<2, 16, 1, 0>(c, a);
     case 1: return launch_v<2, 16, 1, 1>(c, a);
