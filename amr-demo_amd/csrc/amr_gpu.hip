@@ -357,6 +357,31 @@ __device__ __forceinline__ double dpp_f64(double v)
     hi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
+// The same where the banks (groups of four lanes of a row) of BANKS are written,
+// `old` elsewhere
+template <int CTRL, int BANKS>
+__device__ __forceinline__ double dpp_f64(double old, double v)
+{
+    const long long o = __double_as_longlong(old), b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp((int)o, (int)b, CTRL, 0xf, BANKS, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(b >> 32), CTRL, 0xf, BANKS, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+// a's and b's halves of the wave (H = 32) or odd and even rows (H = 16) exchanged:
+// op of the two is a's reduced by one step in the lower lanes (even rows), b's in
+// the others -- two values for the price of one
+template <int H>
+__device__ __forceinline__ void swap_f64(double &a, double &b)
+{
+    const long long p = __double_as_longlong(a), q = __double_as_longlong(b);
+    auto swap = [](int x, int y) {
+        if constexpr (H == 32) return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        else return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    };
+    const auto lo = swap((int)p, (int)q), hi = swap((int)(p >> 32), (int)(q >> 32));
+    a = __longlong_as_double(((long long)hi[0] << 32) | (unsigned)lo[0]);
+    b = __longlong_as_double(((long long)hi[1] << 32) | (unsigned)lo[1]);
+}
 // A wave-uniform double moved to scalar registers (its value in lane 0):
 // it then holds no vector registers while it waits for its uses.
 __device__ __forceinline__ double uniform_f64(double v)
@@ -2239,7 +2264,10 @@ __global__ void soa_to_aos_kernel(const double *soa, double *aos, long long ncel
 // thread per cell that walks its own sides runs eight more of them per wave
 // with an edge's lanes busy; as one list they are one round (two with hanging
 // sides).  Maxima by DPP instead of LDS atomics on one address per patch.
-// 5.0M cells in 8x8 patches: 52.6 us before, 28.8 now.
+// 8x8 patches go two to a wave (indicator8_kernel), so that the edges' round is
+// full and the two maxima share their reduction.
+// 5.0M cells in 8x8 patches: 52.6 us at first, 25.7 with a wave per patch,
+// 18.4 now.
 __device__ __forceinline__ double rel_jump(double a, double b) { return fabs(a - b) / (0.5 * (a + b)); }
 
 template <int N>
@@ -2280,6 +2308,41 @@ __global__ __launch_bounds__(256) void indicator_kernel(MeshDev m, const double 
     if (active && c == 0) ind[quad] = v;
 }
 
+__global__ __launch_bounds__(256) void indicator8_kernel(MeshDev m, const double *U, double *ind)
+{
+    constexpr int N = 8, QS = NFLD * N * N;
+    const int c = threadIdx.x & 63, ci = c % N, cj = c / N;
+    const int q0 = __builtin_amdgcn_readfirstlane(((int)xcd_block(blockIdx.x, gridDim.x) * 4 + (int)threadIdx.x / 64) * 2);
+    if (q0 >= m.nquad) return;
+    const bool two = q0 + 1 < m.nquad;               // (an odd last patch goes with itself)
+    const double *const Q = U + (size_t)q0 * QS;     // field 0 planes
+    const int d1 = two ? QS : 0;
+    // the lane's edge cell: position k of side s of patch 0 (lower lanes) or 1
+    const int s = c / N % 4, k = c % N;
+    const bool x = s < 2, hi = s & 1, up = c >= 32;
+    const int lo = x ? k * N : k, top = lo + (x ? N - 1 : (N - 1) * N);
+    const int2 nb = *(const int2 *)(m.nbr + (size_t)(q0 + (up && two ? 1 : 0)) * 8 + 2 * s);
+    const int cx = ci + 1 < N ? c + 1 : c, cy = cj + 1 < N ? c + N : c;
+    const double r0 = Q[c], x0 = Q[cx], y0 = Q[cy], r1 = Q[d1 + c], x1 = Q[d1 + cx], y1 = Q[d1 + cy];
+    const double o = Q[(up ? d1 : 0) + (hi ? top : lo)];
+    const int ec = hi ? lo : top;
+    double g = o, h = o;
+    if (nb.x >= 0) g = U[(size_t)nb.x * QS + ec];
+    if (nb.y >= 0) h = U[(size_t)nb.y * QS + ec];
+    // (a cell past the patch's edge: the cell itself, which gives 0 or NaN, and
+    // neither raises a maximum that starts at 0)
+    double v0 = fmax(fmax(0.0, rel_jump(r0, x0)), rel_jump(r0, y0));
+    double v1 = fmax(fmax(0.0, rel_jump(r1, x1)), rel_jump(r1, y1));
+    swap_f64<32>(v0, v1);
+    double v = fmax(v0, v1);
+    v = fmax(v, rel_jump(o, g));
+    if (__any(nb.y >= 0)) v = fmax(v, rel_jump(o, h));
+    double w = v;
+    swap_f64<16>(v, w);
+    v = group_reduce<16>(fmax(v, w), [](double a, double b) { return fmax(a, b); });
+    if (c == 0 || (c == 32 && two)) ind[q0 + c / 32] = v;
+}
+
 // The reference's feature tags (solver_tag_feature.F90:9-52 with
 // tag_density_below / tag_density_above, tagging_methods_module.F90:14-71):
 // a quadrant is tagged when, for some method k, one of its sub-cell
@@ -2296,8 +2359,10 @@ struct FeatureTagArgs {
 
 // One load per cell and two reductions: the loads' latency and the reductions
 // bound it, so a wave takes SPAN patch groups with their loads in flight
-// together and reduces by DPP (shuffles cost an LDS round trip a step).
-// 5.0M cells in 8x8 patches: 23.7 us before, 17.4 now.
+// together and reduces by DPP (shuffles cost an LDS round trip a step); the four
+// 8x8 patches of a wave reduce their eight values together, each exchange halving
+// what is left.  5.0M cells in 8x8 patches: 23.7 us at first, 14.2 with a
+// reduction per value, 8.3 now (4.9 TB/s).
 template <int N>
 __global__ __launch_bounds__(256) void feature_tag_kernel(int nquad, const double *U, FeatureTagArgs t,
                                                           int *tags)
@@ -2314,6 +2379,30 @@ __global__ __launch_bounds__(256) void feature_tag_kernel(int nquad, const doubl
         const int quad = (blockIdx.x * SPAN + k) * PPB + p;
         r[k] = quad < nquad ? U[(size_t)quad * NFLD * N2 + c] : NAN;
     }
+    auto tag_of = [&](double mn, double mx) {
+        int tag = 0;
+        for (int j = 0; j < t.ntags; ++j) {
+            if (t.method[j] == 1 && mn <= t.tol[j]) tag = 1;
+            if (t.method[j] == 2 && mx >= t.tol[j]) tag = 1;
+        }
+        return tag;
+    };
+    if constexpr (N2 == 64) {
+        swap_f64<32>(r[0], r[1]);
+        swap_f64<32>(r[2], r[3]);
+        double n0 = fmin(r[0], r[1]), n1 = fmin(r[2], r[3]), x0 = fmax(r[0], r[1]), x1 = fmax(r[2], r[3]);
+        swap_f64<16>(n0, n1);
+        swap_f64<16>(x0, x1);
+        // patches 0, 2, 1, 3 in the wave's rows: the minimum, and minus the maximum
+        const double n = fmin(n0, n1), x = fmin(-x0, -x1);
+        // lanes 8 apart: the lower banks keep the one, the upper ones the other
+        double v = fmin(dpp_f64<0x108, 0x3>(x, n), dpp_f64<0x118, 0xc>(n, x));
+        v = group_reduce<8>(v, [](double a, double b) { return fmin(a, b); });
+        const double mx = -dpp_f64<0x108, 0x3>(v, v);
+        const int row = c / 16, k = (row & 1) * 2 + row / 2, quad = (blockIdx.x * SPAN + k) * PPB + p;
+        if (quad < nquad && c % 16 == 0) tags[quad] = tag_of(v, mx);
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < SPAN; ++k) {
         const int quad = (blockIdx.x * SPAN + k) * PPB + p;
@@ -2326,14 +2415,7 @@ __global__ __launch_bounds__(256) void feature_tag_kernel(int nquad, const doubl
             mn = fmin(fmin(smin[k][0], smin[k][1]), fmin(smin[k][2], smin[k][3]));
             mx = fmax(fmax(smax[k][0], smax[k][1]), fmax(smax[k][2], smax[k][3]));
         }
-        if (quad < nquad && c == 0) {
-            int tag = 0;
-            for (int j = 0; j < t.ntags; ++j) {
-                if (t.method[j] == 1 && mn <= t.tol[j]) tag = 1;
-                if (t.method[j] == 2 && mx >= t.tol[j]) tag = 1;
-            }
-            tags[quad] = tag;
-        }
+        if (quad < nquad && c == 0) tags[quad] = tag_of(mn, mx);
     }
 }
 
@@ -2766,7 +2848,7 @@ int launch_indicator(amrgpu_ctx *c, double *d_ind)
     switch (c->n) {
     case 2: hipLaunchKernelGGL((indicator_kernel<2>), nblk, dim3(256), 0, c->stream, m, U, d_ind); break;
     case 4: hipLaunchKernelGGL((indicator_kernel<4>), nblk, dim3(256), 0, c->stream, m, U, d_ind); break;
-    case 8: hipLaunchKernelGGL((indicator_kernel<8>), nblk, dim3(256), 0, c->stream, m, U, d_ind); break;
+    case 8: hipLaunchKernelGGL(indicator8_kernel, dim3((c->nquad + 7) / 8), dim3(256), 0, c->stream, m, U, d_ind); break;
     case 16: hipLaunchKernelGGL((indicator_kernel<16>), nblk, dim3(256), 0, c->stream, m, U, d_ind); break;
     default: set_err("unsupported nelem_subgrid %d", c->n); return AMRGPU_ERR_ARG;
     }

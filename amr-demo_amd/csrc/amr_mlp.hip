@@ -60,12 +60,18 @@ typedef short s8v __attribute__((ext_vector_type(8)));
 typedef __bf16 b8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
+// round to nearest even (no NaN here); the device has an instruction for it, equal
+// for every other bit pattern
 __host__ __device__ inline uint16_t f2bf(float x)
 {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_bit_cast(uint16_t, (__bf16)x);
+#else
     uint32_t u;
     memcpy(&u, &x, 4);
-    u += 0x7FFFu + ((u >> 16) & 1u);     // round to nearest even (no NaN here)
+    u += 0x7FFFu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
+#endif
 }
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
@@ -84,12 +90,11 @@ __device__ __forceinline__ double bits2d(unsigned long long b) { return __longlo
 
 // ---------------------------------------------------------------------------
 // features: one wave per 8x8 patch, four patches per workgroup.  Memory is the
-// floor (32 bytes read and 12 written per cell); before, LDS atomics of 64
-// lanes on one address per maximum and six IEEE quotients per cell were what
-// it took.  Now the maxima are DPP reductions, a patch's four maxima are
-// inverted once, and a quotient by one is a product refined to the correctly
-// rounded value.  5.0M cells: 83.5 us before, 53.6 now (4.1
-// TB/s).
+// floor (32 bytes read and 12 written per cell).  The four maxima share one
+// reduction, are inverted once, a lane each, and a quotient by one is a product
+// refined to the correctly rounded value.  5.0M cells: 83.5 us with LDS atomics and
+// six IEEE quotients per cell, 51.7 with a DPP reduction per maximum (350 vector
+// instructions a patch, which bounded it), 40.9 now (220; 5.4 TB/s).
 // ---------------------------------------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ double dpp_move(double v)
@@ -106,17 +111,25 @@ __device__ __forceinline__ double lane_value(double v, int lane)
     const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-// max |u| over the wave, NaN if some lane's is (as the maximum of the bit
-// patterns has it)
-__device__ __forceinline__ double wave_abs_max(double u)
+// The maxima of four values' magnitudes over the wave, ignoring NaN: row k of 16
+// lanes ends with that of u[0], u[2], u[1], u[3].  Two values exchange the wave's
+// halves, then the two results their odd and even rows, so that what is left to
+// reduce is one value.
+__device__ __forceinline__ double four_abs_max(const double u[4])
 {
-    double v = fabs(u);
-    v = fmax(v, dpp_move<0x111>(v));    // row_shr:1, 2, 4, 8: each row's maximum in its last lane
-    v = fmax(v, dpp_move<0x112>(v));
-    v = fmax(v, dpp_move<0x114>(v));
-    v = fmax(v, dpp_move<0x118>(v));
-    v = fmax(fmax(lane_value(v, 15), lane_value(v, 31)), fmax(lane_value(v, 47), lane_value(v, 63)));
-    return __any(u != u) ? NAN : v;
+    auto joint = [](double a, double b, auto swap) {
+        const long long p = __double_as_longlong(a), q = __double_as_longlong(b);
+        const auto lo = swap((int)p, (int)q), hi = swap((int)(p >> 32), (int)(q >> 32));
+        return fmax(fabs(__longlong_as_double(((long long)hi[0] << 32) | (unsigned)lo[0])),
+                    fabs(__longlong_as_double(((long long)hi[1] << 32) | (unsigned)lo[1])));
+    };
+    auto halves = [](int x, int y) { return __builtin_amdgcn_permlane32_swap(x, y, false, false); };
+    auto rows = [](int x, int y) { return __builtin_amdgcn_permlane16_swap(x, y, false, false); };
+    double v = joint(joint(u[0], u[1], halves), joint(u[2], u[3], halves), rows);
+    v = fmax(v, dpp_move<0xB1>(v));                  // quad_perm 1,0,3,2
+    v = fmax(v, dpp_move<0x4E>(v));                  // quad_perm 2,3,0,1
+    v = fmax(v, dpp_move<0x141>(v));                 // row_half_mirror
+    return fmax(v, dpp_move<0x140>(v));              // row_mirror
 }
 
 // RN(a / s) for s in [2^-400, 2^400] and |a| <= 2^400, given r = RN(1 / s): the
@@ -164,30 +177,35 @@ __global__ __launch_bounds__(256) void features_kernel(const double *__restrict_
     if (na >= 0 && nbb >= 0) g = 0.5 * (g + U[(size_t)nbb * 256 + (hi ? lo : top)]);
     rho[w][c] = u[0];
     if (c < 32) rho[w][64 + c] = g;
-    double sm[4];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) sm[f] = wave_abs_max(u[f]);
+    const double m = four_abs_max(u);
     asm volatile("" ::: "memory");                   // the wave's LDS operations execute in order
     const double re = rho[w][ci < 7 ? c + 1 : 64 + 8 + cj], rw = rho[w][ci > 0 ? c - 1 : 64 + cj];
     const double rn = rho[w][cj < 7 ? c + 8 : 64 + 24 + ci], rs = rho[w][cj > 0 ? c - 8 : 64 + 16 + ci];
     const double num[6] = {u[0], u[1], u[2], u[3], re - rw, rn - rs};
     uint16_t *o = X + (size_t)quad * NIN + c;
-    // every maximum zero or in div_by's range, no infinity or NaN across a side
-    bool plain = __all(fabs(num[4]) <= 0x1p400 && fabs(num[5]) <= 0x1p400);
+    constexpr int at[4] = {0, 32, 16, 48};           // a lane with the maximum of field f
+    double sm[4];
 #pragma unroll
-    for (int f = 0; f < 4; ++f) plain = plain && (sm[f] == 0.0 || (sm[f] >= 0x1p-400 && sm[f] <= 0x1p400));
-    if (plain) {
-        // the four reciprocals from one quotient, a lane each
-        const double inv = 1.0 / (c == 0 ? sm[0] : c == 1 ? sm[1] : c == 2 ? sm[2] : sm[3]);
+    for (int f = 0; f < 4; ++f) sm[f] = lane_value(m, at[f]);
+    // every maximum zero or in div_by's range, no infinity or NaN among the numerators
+    const bool nan = u[0] != u[0] || u[1] != u[1] || u[2] != u[2] || u[3] != u[3];
+    if (__all(!nan && fabs(num[4]) <= 0x1p400 && fabs(num[5]) <= 0x1p400 &&
+              (m == 0.0 || (m >= 0x1p-400 && m <= 0x1p400)))) {
+        // the four reciprocals from one quotient
+        const double inv = 1.0 / m;
         double ri[4];
 #pragma unroll
-        for (int f = 0; f < 4; ++f) ri[f] = lane_value(inv, f);
+        for (int f = 0; f < 4; ++f) ri[f] = lane_value(inv, at[f]);
 #pragma unroll
         for (int f = 0; f < 6; ++f) {
             const double d = f < 4 ? sm[f] : sm[0], r = f < 4 ? ri[f] : ri[0];
             o[f * 64] = d == 0.0 ? (uint16_t)0 : quotient_bf16(div_by(num[f], d, r), num[f]);
         }
     } else {
+        // a maximum is NaN where some lane's value is
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+            if (__any(u[f] != u[f])) sm[f] = NAN;
 #pragma unroll
         for (int f = 0; f < 6; ++f) {
             const double d = f < 4 ? sm[f] : sm[0];

@@ -100,3 +100,24 @@ def test_training_step_follows_the_gradient(batch):
     assert abs(losses[0] - loss) <= 1e-5 * abs(loss)
     m.close()
     ts.close()
+
+
+@pytest.mark.parametrize("splits", [0, 1, 2, 24])
+def test_broken_densities_8x8(splits):
+    """NaN, infinite and zero densities in some cells, a whole patch of NaN: the
+    indicator ignores a pair without a quotient and the tags a cell without a
+    value, as the host's do, in a wave's first and last patch alike"""
+    f = forest(8, splits, 70 + splits)
+    q = f.soln()
+    rng = np.random.default_rng(splits)
+    for bad in (np.nan, np.inf, 0.0):
+        q[..., 0][rng.uniform(size=q.shape[:3]) < 0.02] = bad
+    if f.nquad > 1:
+        q[f.nquad - 1, ..., 0] = np.nan
+    g = context(f)
+    assert np.array_equal(g.indicator(), f.indicator(), equal_nan=True)
+    rho = f.soln()[..., 0].reshape(f.nquad, -1)
+    with np.errstate(invalid="ignore"):
+        exp = (rho <= 0.5).any(axis=1) | (rho >= 1.4).any(axis=1)
+    assert np.array_equal(g.feature_tags([1, 2], [0.5, 1.4]), exp.astype(np.int32))
+    g.close()
