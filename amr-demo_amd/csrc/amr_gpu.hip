@@ -648,6 +648,60 @@ __device__ __forceinline__ void load_oprim(const double *lds, int p, int t, int 
     P.H = P.W * ir;
 }
 
+// Which vectors beside the stage state a stage reads: its base state U0, its
+// accumulator, or both; VEC_ANY: told by the mode as it runs.
+enum { VEC_BASE = 0, VEC_ACC = 1, VEC_BOTH = 2, VEC_ANY = 3 };
+
+template <int VEC>
+__device__ __forceinline__ bool reads_base(const StageArgs &a)
+{
+    if (VEC == VEC_ACC) return false;
+    return a.mode == MODE_SO ? a.U0 != nullptr : a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL;
+}
+template <int VEC>
+__device__ __forceinline__ bool reads_acc(const StageArgs &a)
+{
+    return (VEC == VEC_ACC || VEC == VEC_BOTH) && !a.first;
+}
+template <int VEC>
+__device__ __forceinline__ bool writes_acc(const StageArgs &a)
+{
+    return VEC == VEC_ACC || (VEC == VEC_BOTH && a.mode == MODE_RK4_ACC);
+}
+
+// stage_update with the vectors in registers: B the base state, A the accumulator
+// (updated).  They are asked for ahead of the fluxes' exchange and their latency
+// passes beside it; stage_update reads the accumulator at the kernel's end, where
+// nothing else is left to do (us per step there -> here: 16x16 LSERK45 2.4M cells
+// 283 -> 273, 1M 134 -> 128, 3.1M 402 -> 378, RK4 0.4M 58.3 -> 56.4).
+template <int VEC>
+__device__ __forceinline__ void stage_form(const StageArgs &a, double dt, const double U[4], const double B[4],
+                                           double A[4], const double k4[4], double out[4])
+{
+    static_assert(VEC != VEC_ANY, "");
+    const double c2dt = a.c2 * dt;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        if (VEC == VEC_ACC) {
+            A[f] = a.first ? dt * k4[f] : fma(A[f], a.c1, dt * k4[f]);
+            out[f] = fma(a.c2, A[f], U[f]);
+        } else if (VEC == VEC_BOTH) {
+            if (a.mode == MODE_RK4_FINAL) {
+                out[f] = fma(dt / 6.0, A[f] + k4[f], B[f]);
+            } else {
+                A[f] = a.first ? k4[f] : fma(2.0, k4[f], A[f]);
+                out[f] = fma(c2dt, k4[f], B[f]);
+            }
+        } else if (a.mode == MODE_RHS) {
+            out[f] = k4[f];
+        } else if (a.U0) {
+            out[f] = fma(c2dt, k4[f], fma(a.c0, B[f], a.c1 * U[f]));
+        } else {
+            out[f] = fma(c2dt, k4[f], a.c1 * U[f]);
+        }
+    }
+}
+
 // The stage update of one cell from its residual k4 = R(U) / V (the schemes
 // of rk_time_integrators.c: Shu-Osher stages for SSP-RK2/3, the RK4
 // accumulator, the 2N-storage LSERK45 register), shared by the stage
@@ -694,7 +748,7 @@ __device__ __forceinline__ void stage_update(const StageArgs &a, size_t base, in
 }
 
 // SELF: the first stage of a step without dt_prep_kernel (one-patch tiles).
-template <int N, int PPB, int MINW, int DESIGN, bool SELF = false, bool NT = true>
+template <int N, int PPB, int MINW, int DESIGN, bool SELF = false, bool NT = true, int VEC = VEC_ANY>
 __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(StageArgs a)
 {
     using TL = Tile<N, PPB>;
@@ -741,7 +795,8 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
     // initialising them costs a move per register on every path.
     double U[4];
     double B[4];     // base state U0 of the step
-    const bool needB = (a.mode == MODE_SO && a.U0) || a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL;
+    double A[4];     // accumulator (not VEC_ANY)
+    const bool needB = reads_base<VEC>(a);
 #pragma unroll
     for (int f = 0; f < 4; ++f) U[f] = a.Us[base + f * N2];
     int nbw[8];
@@ -1037,6 +1092,10 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
 #pragma unroll
             for (int f = 0; f < 4; ++f) B[f] = gptr(a.U0)[base + f * N2];
         }
+        if (actu && reads_acc<VEC>(a)) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) A[f] = gptr(a.Acc)[base + f * N2];
+        }
         __syncthreads();   // all reads of the primitive tile are done
         const int stride = N * (N + 1);
         if (actu) {
@@ -1222,7 +1281,15 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
         }
         double dt = 0.0;
         if (a.mode != MODE_RHS) dt = UNI ? dtw : pdt[p];
-        stage_update(a, base, N2, dt, U, B, k4, out);
+        if constexpr (VEC == VEC_ANY) {
+            stage_update(a, base, N2, dt, U, B, k4, out);
+        } else {
+            stage_form<VEC>(a, dt, U, B, A, k4, out);
+            if (writes_acc<VEC>(a)) {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) a.Acc[base + f * N2] = A[f];
+            }
+        }
         // an instance past its physical stop (dt = 0) keeps its state bit for
         // bit: every stage state equals U^n then, while a convex combination
         // such as 0.75 U + 0.25 U can round away from U
@@ -1601,10 +1668,6 @@ __device__ __forceinline__ OPrim oprim_of(const Rec &c, bool xdir)
     return o;
 }
 
-// Which vectors beside the stage state a stage reads: its base state U0, its
-// accumulator, or both.
-enum { VEC_BASE = 0, VEC_ACC = 1, VEC_BOTH = 2 };
-
 // LDS accesses before it are not moved past it by the compiler; the wave's
 // LDS operations execute in order, so nothing is waited for.
 __device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
@@ -1650,7 +1713,7 @@ __device__ __forceinline__ double upper_half(double v)
 // the first round) -> this: 2.6k quadrants (adaptive) 23.7 -> 21.4, 18.8k
 // 88 -> 84, 159k 700 -> 664, 131k uniform 547 -> 524.
 // ---------------------------------------------------------------------------
-template <int MINW, bool SELF, bool NT>
+template <int MINW, bool SELF, bool NT, int VEC>
 __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
 {
     constexpr int N = 8;
@@ -1757,11 +1820,14 @@ __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
     }
     // the base state is asked for late: an earlier load is no faster on small
     // meshes and slows the memory on large ones (8.4M cells 566 -> 598 us a step)
-    const bool needB = (a.mode == MODE_SO && a.U0) || a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL;
-    double B[4];
-    if (needB) {
+    double B[4], A[4];
+    if (reads_base<VEC>(a)) {
 #pragma unroll
         for (int f = 0; f < 4; ++f) B[f] = (gptr(a.U0) + quad + f * N2)[c];
+    }
+    if (reads_acc<VEC>(a)) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) A[f] = (gptr(a.Acc) + quad + f * N2)[c];
     }
     if constexpr (SELF) {
         const double cm = a.use_cfl ? slot_min(a.slot_in, inst) : INFINITY;
@@ -1797,7 +1863,15 @@ __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
             k4[f] = ((xr[f * ST] - xl[f * ST]) + (yb[f * ST + N] - yb[f * ST])) * ninvV;
         }
     }
-    stage_update(a, quad + c, N2, dt, U, B, k4, out);
+    if constexpr (VEC == VEC_ANY) {
+        stage_update(a, quad + c, N2, dt, U, B, k4, out);
+    } else {
+        stage_form<VEC>(a, dt, U, B, A, k4, out);
+        if (writes_acc<VEC>(a)) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) ((gdbl *)(a.Acc + quad + f * N2))[c] = A[f];
+        }
+    }
     // past its stop an instance keeps its state bit for bit (see stage_kernel)
     if (__builtin_amdgcn_readfirstlane((int)(a.mode != MODE_RHS && dt == 0.0))) {
 #pragma unroll
@@ -1992,9 +2066,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
     const double hx = hx2 ? 0.5 * h : h;
     const bool frozen = a.mode != MODE_RHS && dt == 0.0;
     const bool any_frozen = __any(frozen);
-    const bool needB = VEC != VEC_ACC && (a.mode == MODE_SO ? a.U0 != nullptr : a.mode != MODE_RHS);
-    const bool needA = VEC != VEC_BASE && !a.first;
-    const double c2dt = a.c2 * dt;
+    const bool needB = reads_base<VEC>(a), needA = reads_acc<VEC>(a);
     double sq = 0.0, eig = 0.0;
 
     constexpr int UNROLL = STEPS <= 2 ? STEPS : 1;
@@ -2028,8 +2100,8 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
             }
         }
         double B[4] = {0.0, 0.0, 0.0, 0.0}, A[4] = {0.0, 0.0, 0.0, 0.0};
-        if (VEC != VEC_ACC && needB) row_load(a.U0, s, B);
-        if (VEC != VEC_BASE && needA) row_load(a.Acc, s, A);
+        if (needB) row_load(a.U0, s, B);
+        if (needA) row_load(a.Acc, s, A);
         // the fluxes of the low faces: the neighbour lane's, the edges', the top
         // row's of the step before
         double *const fx = rec + FX + lane % NE + lane / NE * (NFLD * NE);
@@ -2071,33 +2143,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
 #pragma unroll
             for (int f = 0; f < 4; ++f) sq = fma(k4[f], k4[f], sq);
         }
-        // the stage update (stage_update's arithmetic on the vectors loaded above)
-        if (VEC == VEC_ACC) {
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                A[f] = a.first ? dt * k4[f] : fma(A[f], a.c1, dt * k4[f]);
-                out[f] = fma(a.c2, A[f], U[f]);
-            }
-        } else if (VEC == VEC_BOTH) {
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                if (a.mode == MODE_RK4_FINAL) {
-                    out[f] = fma(dt / 6.0, A[f] + k4[f], B[f]);
-                } else {
-                    A[f] = a.first ? k4[f] : fma(2.0, k4[f], A[f]);
-                    out[f] = fma(c2dt, k4[f], B[f]);
-                }
-            }
-        } else if (a.mode == MODE_RHS) {
-#pragma unroll
-            for (int f = 0; f < 4; ++f) out[f] = k4[f];
-        } else if (needB) {
-#pragma unroll
-            for (int f = 0; f < 4; ++f) out[f] = fma(c2dt, k4[f], fma(a.c0, B[f], a.c1 * U[f]));
-        } else {
-#pragma unroll
-            for (int f = 0; f < 4; ++f) out[f] = fma(c2dt, k4[f], a.c1 * U[f]);
-        }
+        stage_form<VEC>(a, dt, U, B, A, k4, out);
         if (any_frozen && frozen) {            // past its stop an instance keeps its state bit for bit
 #pragma unroll
             for (int f = 0; f < 4; ++f) out[f] = U[f];
@@ -2109,7 +2155,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
             const unsigned o = here(off);
 #pragma unroll
             for (int f = 0; f < 4; ++f) put_state<NT>((gout *)(ob + f * N2 * 8 + o), out[f]);
-            if (VEC == VEC_ACC || (VEC == VEC_BOTH && a.mode == MODE_RK4_ACC)) {
+            if (writes_acc<VEC>(a)) {
                 gcout *const ab = (gcout *)(gout *)(a.Acc + (size_t)g * (P * QS) + R * N * s);
 #pragma unroll
                 for (int f = 0; f < 4; ++f) *(gout *)(ab + f * N2 * 8 + o) = A[f];
@@ -2746,19 +2792,33 @@ void with_flags(const amrgpu_ctx *c, const StageArgs &a, F f)
     else nt ? f(no, yes) : f(no, no);
 }
 
+// f(vec): the vectors that the stage's mode reads; BASE: what stands for VEC_BASE.
+template <int BASE, class F>
+void with_vectors(const StageArgs &a, F f)
+{
+    if (a.mode == MODE_LSERK) f(std::integral_constant<int, VEC_ACC>());
+    else if (a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL) f(std::integral_constant<int, VEC_BOTH>());
+    else f(std::integral_constant<int, BASE>());
+}
+
 template <int N, int PPB, int MINW, int D>
 int launch_v(amrgpu_ctx *c, const StageArgs &a)
 {
     const dim3 nblk((c->nquad + PPB - 1) / PPB), blk(Tile<N, PPB>::BLK);
     if constexpr (D == 1 && PPB == 1) {
+        // (the Shu-Osher stages are up to 1.5 % slower specialised: 8x8 159k quadrants
+        // 655 / 662 us a step, 16x16 15k 236 / 240)
         with_flags(c, a, [&](auto self, auto nt) {
-            constexpr bool SELF = decltype(self)::value, NT = decltype(nt)::value;
-            if constexpr (SELF && MINW < 4)
-                return;        // (has_self)
-            else if constexpr (N == 8)
-                hipLaunchKernelGGL((stage_kernel_one<MINW, SELF, NT>), nblk, blk, 0, c->stream, a);
-            else
-                hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D, SELF, NT>), nblk, blk, 0, c->stream, a);
+            with_vectors<VEC_ANY>(a, [&](auto vec) {
+                constexpr bool SELF = decltype(self)::value, NT = decltype(nt)::value;
+                constexpr int VEC = decltype(vec)::value;
+                if constexpr (SELF && MINW < 4)
+                    return;        // (has_self)
+                else if constexpr (N == 8)
+                    hipLaunchKernelGGL((stage_kernel_one<MINW, SELF, NT, VEC>), nblk, blk, 0, c->stream, a);
+                else
+                    hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D, SELF, NT, VEC>), nblk, blk, 0, c->stream, a);
+            });
         });
     } else {
         hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D>), nblk, blk, 0, c->stream, a);
@@ -2772,15 +2832,12 @@ int launch_rows(amrgpu_ctx *c, const StageArgs &a)
 {
     constexpr int P = 64 / (N * R);
     const dim3 nblk((c->nquad + P - 1) / P);
-    auto go = [&](auto vec) {
-        with_flags(c, a, [&](auto self, auto nt) {
+    with_flags(c, a, [&](auto self, auto nt) {
+        with_vectors<VEC_BASE>(a, [&](auto vec) {
             hipLaunchKernelGGL((stage_kernel_rows<N, R, decltype(vec)::value, decltype(self)::value, decltype(nt)::value>),
                                nblk, dim3(64), 0, c->stream, a);
         });
-    };
-    if (a.mode == MODE_LSERK) go(std::integral_constant<int, VEC_ACC>());
-    else if (a.mode == MODE_RK4_ACC || a.mode == MODE_RK4_FINAL) go(std::integral_constant<int, VEC_BOTH>());
-    else go(std::integral_constant<int, VEC_BASE>());
+    });
     HIPCHK(hipGetLastError());
     return AMRGPU_OK;
 }
