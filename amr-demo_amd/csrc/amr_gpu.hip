@@ -101,6 +101,7 @@ struct StageArgs {
     double *t_out;       // ninst: time at its end
     double *t_step;      // MeshDev's, for the step's other stages
     int use_cfl;
+    unsigned long long empty[2];         // instances without quadrants (bits)
     double *norm_part;
     bool down;           // the launch goes through the patches from the end (launch_stage)
     int per_block;       // persistent design: patches per workgroup (a contiguous range)
@@ -526,6 +527,30 @@ __device__ __forceinline__ void publish_dt(const StageArgs &a, int inst, double 
     for (int k = 0; k < NSLOT / 64; ++k) a.slot_clear[(size_t)inst * NSLOT + lane + 64 * k] = DBL_INF_BITS;
 }
 
+// The same for the instances without quadrants, a lane each, by the wave of the
+// first quadrant: no CFL minimum limits them.
+__device__ __forceinline__ void publish_empty(const StageArgs &a)
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        unsigned long long left = a.empty[w];
+        if (left >> lane & 1) {
+            const int i = 64 * w + lane;
+            const double t = a.t_in[i];
+            const double dt = limited_dt(a.m.ip[i].dt_cap, a.m.ip[i].t_end, INFINITY, t, a.use_cfl);
+            a.dt_cur[i] = dt;
+            a.t_step[i] = t;
+            a.t_out[i] = t + dt;
+        }
+        for (; left; left &= left - 1) {
+            unsigned long long *const s = a.slot_clear + (size_t)(64 * w + __ffsll(left) - 1) * NSLOT;
+#pragma unroll
+            for (int k = 0; k < NSLOT / 64; ++k) s[lane + 64 * k] = DBL_INF_BITS;
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Fused stage kernel: one workgroup = PPB patches of N x N cells, one thread
 // per cell.  LDS holds the patches' primitive variables with a one-cell ghost
@@ -889,6 +914,7 @@ __global__ __launch_bounds__((Tile<N, PPB>::BLK), (MINW)) void stage_kernel(Stag
             const double c = a.use_cfl ? slot_min(a.slot_in, inw) : INFINITY;
             dtw = uniform_f64(limited_dt(ipc[inw].dt_cap, ipc[inw].t_end, c, tw, a.use_cfl));
             if (tid < 64 && (lb == 0 || ((const cint4 *)a.m.inst)[lb - 1] != inw)) publish_dt(a, inw, dtw, tw);
+            if (tid < 64 && lb == 0) publish_empty(a);
         }
         if (!SMETA && c == 0) {
             pquad[p] = actw ? lb * PPB + p : -1;
@@ -1833,6 +1859,7 @@ __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
         const double cm = a.use_cfl ? slot_min(a.slot_in, inst) : INFINITY;
         dt = uniform_f64(limited_dt(ipc->dt_cap, ipc->t_end, cm, tw, a.use_cfl));
         if (q == 0 || ((const cint4 *)a.m.inst)[q - 1] != inst) publish_dt(a, inst, dt, tw);
+        if (q == 0) publish_empty(a);
     }
     // ---- the fluxes over the records but for the cells' r, ru, rv, rE --------------
     lds_order();
@@ -1987,6 +2014,7 @@ __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
             if (inst == i) dt = d;
             todo &= ~__ballot(inst == i);
         } while (todo);
+        if (g == 0) publish_empty(a);
     }
     const double ninvV = ldexp(a.m.ip[inst].ninv_vol0, 2 * lev);
 
@@ -2266,6 +2294,12 @@ __global__ void slot_reset_kernel(unsigned long long *slot, int ninst)
 // time left), publishes it with the step's start time, advances the time and
 // re-arms the sub-slots that the step's last stage fills.  The stages then
 // read the published dt instead of every wave reducing the sub-slots.
+__global__ __launch_bounds__(128) void drop_dt_kernel(unsigned long long lo, unsigned long long hi, double *dt_cur)
+{
+    const int i = threadIdx.x;
+    if ((i < 64 ? lo >> i : hi >> (i - 64)) & 1) dt_cur[i] = 0.0;
+}
+
 __global__ __launch_bounds__(64) void dt_prep_kernel(MeshDev m, int use_cfl, double *dt_cur, double *t_inst,
                                                      double *t_step, unsigned long long *slot)
 {
@@ -2625,7 +2659,8 @@ struct amrgpu_ctx {
     int tb = 0, sb = 0;
     bool sweep_down = false;                   // direction of the next stage launch
     bool self_dt = false;                      // this run's steps have no dt_prep_kernel
-    bool all_inst = true;                      // every instance has quadrants
+    bool empty_known = true;                   // `empty` has every instance without quadrants
+    unsigned long long empty[2] = {0, 0};
     double *t_now(int ahead = 0) const { return d_clock + (size_t)((tb + ahead) & 1) * cap_inst; }
     double *dt_cur() const { return d_clock + (size_t)2 * cap_inst; }
     double *t_step() const { return d_clock + (size_t)3 * cap_inst; }
@@ -3005,11 +3040,14 @@ bool has_self(int v)
 // 16x16, 256 17.4 / 15.7, 4455 83.3 / 83.1, 7159 122.6 / 125.9; the row-marching
 // tiles, whose waves hold several patches: 4x4, 1024 14.0 / 12.2, 16384 30.5 /
 // 29.1, 65536 84.8 / 85.8; 2x2, 37750 35.5 / 34.6, 65536 36.1 / 36.9.
+// Instances without quadrants are kept as two words of bits (publish_empty), so at
+// most 128 instances where there may be some: a batch of 16 adaptive runs that end
+// one after the other 73.7 ms with the kernel as soon as one has ended, 70.6 so.
 bool wants_self(const amrgpu_ctx *c)
 {
     const TileVariant &v = kVariants[c->variant];
     const long long waves = (long long)c->nblocks * (v.design == 1 ? std::max(1, v.n * v.n / 64) : 1);
-    return !c->graphs_enabled && c->all_inst && has_self(c->variant) && waves <= (v.design == 1 ? 20000 : 4000);
+    return !c->graphs_enabled && c->empty_known && has_self(c->variant) && waves <= (v.design == 1 ? 20000 : 4000);
 }
 
 // The step's dt: a kernel ahead of its first stage, or that stage's own.
@@ -3028,6 +3066,8 @@ int begin_step(amrgpu_ctx *c, std::vector<StageArgs> &st)
     f.t_out = c->t_now(1);
     f.t_step = c->t_step();
     f.use_cfl = c->scheme != 2;
+    f.empty[0] = c->empty[0];
+    f.empty[1] = c->empty[1];
     for (auto &a : st) a.slot = c->slots(1);
     c->tb ^= 1;
     c->sb = (c->sb + 1) % 3;
@@ -3369,11 +3409,19 @@ static int new_mesh(amrgpu_ctx *c, int ncell, const int *cell_inst)
     const MeshPlace m = place_mesh(c->d_block + c->mesh_off, ncell);
     c->d_org = m.org; c->d_nbr = m.nbr; c->d_level = m.level; c->d_inst = m.inst; c->d_map = m.map;
     c->nquad = ncell;
-    c->all_inst = c->ninst == 1;
-    if (cell_inst && c->ninst > 1) {
+    c->empty[0] = c->empty[1] = 0;
+    c->empty_known = c->ninst <= 128;
+    if (c->ninst > 1) {
         std::vector<char> has(c->ninst, 0);
-        for (int q = 0; q < ncell; ++q) has[cell_inst[q]] = 1;
-        c->all_inst = std::find(has.begin(), has.end(), 0) == has.end();
+        has[0] = !cell_inst;
+        if (cell_inst)
+            for (int q = 0; q < ncell; ++q) has[cell_inst[q]] = 1;
+        if (c->empty_known) {
+            for (int i = 0; i < c->ninst; ++i)
+                if (!has[i]) c->empty[i / 64] |= 1ull << i % 64;
+        } else {
+            c->empty_known = std::find(has.begin(), has.end(), 0) == has.end();
+        }
     }
     if (!c->tile_chosen || kVariants[c->variant].n != c->n) {
         c->variant = default_variant(c->n, ncell);
@@ -3637,7 +3685,12 @@ static int remesh_to(amrgpu_ctx *c, int ncell, const MeshPlace &h, const int *ce
     // their stop) no longer advances: no wave publishes its dt any more, so
     // its last dt is cleared here and the time bookkeeping of the stages
     // keeps its time as it is
-    if (cell_inst && c->ninst > 1) {
+    if (c->ninst <= 128) {
+        if (cell_inst && (c->empty[0] | c->empty[1])) {
+            hipLaunchKernelGGL(drop_dt_kernel, dim3(1), dim3(128), 0, c->stream, c->empty[0], c->empty[1], c->dt_cur());
+            HIPCHK(hipGetLastError());
+        }
+    } else if (cell_inst) {
         std::vector<char> has(c->ninst, 0);
         for (int q = 0; q < ncell; ++q) has[cell_inst[q]] = 1;
         bool empty = false;
