@@ -61,10 +61,12 @@ typedef __bf16 b8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 // round to nearest even (no NaN here); the device has an instruction for it, equal
-// for every other bit pattern
+// for every other bit pattern.  The empty statement keeps the FP32 value a value of
+// its own: the compiler would round a double once, straight to BF16.
 __host__ __device__ inline uint16_t f2bf(float x)
 {
 #ifdef __HIP_DEVICE_COMPILE__
+    asm("" : "+v"(x));
     return __builtin_bit_cast(uint16_t, (__bf16)x);
 #else
     uint32_t u;

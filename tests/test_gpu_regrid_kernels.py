@@ -121,3 +121,21 @@ def test_broken_densities_8x8(splits):
         exp = (rho <= 0.5).any(axis=1) | (rho >= 1.4).any(axis=1)
     assert np.array_equal(g.feature_tags([1, 2], [0.5, 1.4]), exp.astype(np.int32))
     g.close()
+
+
+@pytest.mark.parametrize("scale", [0, -450, 500])
+def test_features_round_through_fp32(oracle, scale):
+    """quotients just above and below the middle of two BF16 values, closer to it
+    than FP32 tells: they are rounded to FP32 first and then, a tie, to even, in
+    the range of the product form of the quotient and outside it"""
+    f = forest(8, 3, 11)
+    q = f.soln()
+    k = np.arange(64).reshape(8, 8)
+    mid = 0.5 + (2 * (k % 32) + 1) * 2.0 ** -9           # ties between neighbours in BF16
+    for c, eps in ((1, 2.0 ** -31), (2, -2.0 ** -31), (3, 2.0 ** -28)):
+        q[..., c] = (mid + eps) * 2.0 ** scale
+        q[:, 0, 0, c] = 2.0 ** scale                     # the maximum
+    ci, fi, _, soln = f.external()
+    g = context(f)
+    assert np.array_equal(g.tagger_features(), oracle.tagger_features(8, ci, fi, soln))
+    g.close()
