@@ -246,19 +246,19 @@ struct Weights {
     const float *P;                 // FP32 master (biases read from here)
 };
 
-template <class Lds>
+template <int THREADS, class Lds>
 __device__ void stage_weights(Lds &s, const Weights &wt)
 {
     const int tid = threadIdx.x;
-    for (int i = tid; i < NH * NIN / 8; i += BLK) {
+    for (int i = tid; i < NH * NIN / 8; i += THREADS) {
         const int row = i / (NIN / 8), c8 = i % (NIN / 8);
         *(uint4 *)&s.W1[row * SX + c8 * 8] = ((const uint4 *)wt.W1)[i];
     }
-    for (int i = tid; i < NH * NH / 8; i += BLK) {
+    for (int i = tid; i < NH * NH / 8; i += THREADS) {
         const int row = i / (NH / 8), c8 = i % (NH / 8);
         *(uint4 *)&s.W2[row * SH + c8 * 8] = ((const uint4 *)wt.W2)[i];
     }
-    for (int i = tid; i < 16 * NH / 8; i += BLK) {
+    for (int i = tid; i < 16 * NH / 8; i += THREADS) {
         const int row = i / (NH / 8), c8 = i % (NH / 8);
         *(uint4 *)&s.W3[row * SH + c8 * 8] = ((const uint4 *)wt.W3)[i];
     }
@@ -273,29 +273,31 @@ __device__ void stage_weights(Lds &s, const Weights &wt)
 // A wave takes 16 rows at a time; their features go from memory straight to
 // the matrix operands (a lane's eight consecutive ones are 16 bytes), the next
 // 16 rows' while these are evaluated.  Only the weights and a wave's 16 rows of
-// activations are in LDS (74 KB, two workgroups a CU), and nothing but the
-// staging of the weights takes a barrier.  The features' bytes are the floor;
-// staging each chunk in LDS between barriers, one workgroup a CU, bounded it
-// before: 77k rows 44.1 us, now 18.9 (3.1 TB/s).
+// activations are in LDS (79 KB with eight waves, two workgroups a CU), and nothing
+// but the staging of the weights takes a barrier.  The features' bytes are the
+// floor; 77k rows: 44.1 us with each chunk staged in LDS between barriers, 18.8
+// with four waves a workgroup (2.4 tiles a wave, so the last third of them on
+// their own), 16.6 with eight (3.6 TB/s).
+constexpr int IWAVES = 8;
 struct __attribute__((aligned(16))) InferLds {
     uint16_t W1[NH * SX];
     uint16_t W2[NH * SH];
     uint16_t W3[16 * SH];
-    uint16_t H[4][16 * SH];     // a wave's first, then second hidden layer
+    uint16_t H[IWAVES][16 * SH]; // a wave's first, then second hidden layer
     float b[2 * NH + 4];
 };
 
-__global__ __launch_bounds__(BLK) void infer_kernel(Weights wt, const uint16_t *__restrict__ X, int count,
+__global__ __launch_bounds__(64 * IWAVES, 4) void infer_kernel(Weights wt, const uint16_t *__restrict__ X, int count,
                                                     float refine_bias, float *__restrict__ logits,
                                                     int *__restrict__ cls)
 {
     __shared__ InferLds s;
-    stage_weights(s, wt);
+    stage_weights<64 * IWAVES>(s, wt);
     __syncthreads();
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     uint16_t *const H = s.H[w];
     constexpr int KK = NIN / 32;
-    const int tiles = (count + 15) / 16, step = gridDim.x * 4;
+    const int tiles = (count + 15) / 16, step = gridDim.x * IWAVES;
     s8v xn[KK];
     auto load = [&](int tile) {
         // rows past the last read it; nothing of theirs is stored
@@ -303,7 +305,7 @@ __global__ __launch_bounds__(BLK) void infer_kernel(Weights wt, const uint16_t *
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) xn[kk] = *(const s8v *)(row + 32 * kk);
     };
-    int tile = blockIdx.x * 4 + w;
+    int tile = blockIdx.x * IWAVES + w;
     if (tile < tiles) load(tile);
     for (; tile < tiles; tile += step) {
         f4v acc[4];
@@ -741,8 +743,8 @@ Weights weights_of(const amr_mlp *m) { return Weights{m->W1b, m->W2b, m->W3b, m-
 int launch_infer(amr_mlp *m, const uint16_t *dX, int count, float *dlogits, int *dcls, hipStream_t st)
 {
     if (count <= 0) return AMRGPU_OK;
-    const int grid = std::min((count + ROWS - 1) / ROWS, 512);     // two workgroups on each of 256 CUs
-    hipLaunchKernelGGL(infer_kernel, dim3(grid), dim3(BLK), 0, st, weights_of(m), dX, count, m->refine_bias,
+    const int grid = std::min((count + 16 * IWAVES - 1) / (16 * IWAVES), 512);     // two workgroups on each of 256 CUs
+    hipLaunchKernelGGL(infer_kernel, dim3(grid), dim3(64 * IWAVES), 0, st, weights_of(m), dX, count, m->refine_bias,
                        dlogits, dcls);
     MCHK(hipGetLastError());
     return AMRGPU_OK;
