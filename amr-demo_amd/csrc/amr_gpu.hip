@@ -2263,9 +2263,12 @@ __global__ void slot_min_kernel(const unsigned long long *slot, int ninst, doubl
 }
 
 // The instances' time and step start time as given (null: 0) and, with dt, no last
-// dt.  One small workgroup: an instance is 24 bytes.
-__global__ void clock_kernel(double *t, double *dt, double *t_step, const double *t_inst, int ninst)
+// dt, by one workgroup (an instance is 24 bytes); nslot CFL sub-slots emptied by all.
+__global__ void clock_kernel(double *t, double *dt, double *t_step, const double *t_inst, int ninst,
+                             unsigned long long *slot, int nslot)
 {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nslot; i += gridDim.x * blockDim.x) slot[i] = DBL_INF_BITS;
+    if (blockIdx.x) return;
     for (int i = threadIdx.x; i < ninst; i += blockDim.x) {
         const double v = t_inst ? t_inst[i] : 0.0;
         t[i] = v;
@@ -3355,14 +3358,13 @@ static int empty_slots(amrgpu_ctx *c)
 
 // Buffers are kept across setups and remeshes (an adaptive run changes the
 // mesh once per regrid interval) and grown with 25% headroom when the mesh
-// outgrows them.  *fresh tells whether they were reallocated.
-static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need_acc, bool *fresh)
+// outgrows them; new ones hold nothing yet (the CFL sub-slots are not empty).
+static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need_acc)
 {
     const int n2 = n * n;
     const size_t need_state = (size_t)ncell * 4 * n2;
     const bool reuse = c->U[0] && c->n == n && ncell <= c->cap_quad && ninst <= c->cap_inst &&
                        need_state <= c->cap_state && (!need_acc || c->Acc);
-    *fresh = !reuse;
     if (reuse) return AMRGPU_OK;
     free_mesh(c);
     const int capq = ncell + ncell / 4 + 16;
@@ -3399,7 +3401,7 @@ static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need
     c->d_slot_sets = (unsigned long long *)(c->d_block + slot);
     c->d_norm = (double *)(c->d_block + norm);
     c->d_ind = (double *)(c->d_block + ind);
-    return empty_slots(c);
+    return AMRGPU_OK;
 }
 
 // The device mesh is a new one of ncell quadrants with these instance ids (null:
@@ -3449,7 +3451,8 @@ static int take_res(amrgpu_ctx *c, size_t bytes)
     return pin_take(c->res, std::max(bytes, (size_t)65536));
 }
 
-// (called where the stream is idle: nothing else reads the small-results area)
+// The instances' times, and the CFL sub-slots emptied (called where the stream is
+// idle: nothing else reads the small-results area).
 static int set_clocks(amrgpu_ctx *c, const double *t_inst)
 {
     const double *src = nullptr;
@@ -3458,7 +3461,8 @@ static int set_clocks(amrgpu_ctx *c, const double *t_inst)
         memcpy(c->res.p, t_inst, sizeof(double) * c->ninst);
         src = (const double *)c->res.p;
     }
-    hipLaunchKernelGGL(clock_kernel, dim3(1), dim3(64), 0, c->stream, c->t_now(), c->dt_cur(), c->t_step(), src, c->ninst);
+    hipLaunchKernelGGL(clock_kernel, dim3(16), dim3(256), 0, c->stream, c->t_now(), c->dt_cur(), c->t_step(), src, c->ninst,
+                       c->d_slot_sets, 3 * c->cap_inst * NSLOT);
     HIPCHK(hipGetLastError());
     return AMRGPU_OK;
 }
@@ -3522,9 +3526,7 @@ int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int nin
 
     HIPCHK(hipStreamSynchronize(c->stream));
     free_graphs(c);
-    bool fresh;
-    rc = ensure_capacity(c, nelem_subgrid, ncell, ninst, time_scheme == 4 || time_scheme == 5, &fresh);
-    if (!rc && !fresh) rc = empty_slots(c);
+    rc = ensure_capacity(c, nelem_subgrid, ncell, ninst, time_scheme == 4 || time_scheme == 5);
     if (rc) return rc;
     c->n = nelem_subgrid; c->ninst = ninst; c->scheme = time_scheme;
     c->cur = 0;
@@ -3660,8 +3662,8 @@ static int remesh_to(amrgpu_ctx *c, int ncell, const MeshPlace &h, const int *ce
         HIPCHK(hipMemcpyAsync(keep, from, sizeof(double) * old_state, hipMemcpyDeviceToDevice, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
         const int ninst = c->ninst;
-        bool fresh;
-        rc = ensure_capacity(c, c->n, ncell + ncell / 2, ninst, c->scheme == 4 || c->scheme == 5, &fresh);
+        rc = ensure_capacity(c, c->n, ncell + ncell / 2, ninst, c->scheme == 4 || c->scheme == 5);
+        if (!rc) rc = empty_slots(c);
         if (rc) { (void)hipFree(keep); return rc; }
         HIPCHK(hipMemcpyAsync(c->d_ip, c->h_ip.data(), sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
         double *const now[3] = {c->t_now(), c->dt_cur(), c->t_step()};
@@ -3852,12 +3854,25 @@ int amrgpu_rhs(amrgpu_ctx *c, double *rhs)
     return copy_out(c, rhs, c->d_stage, sizeof(double) * 4 * ncells);
 }
 
+// The CFL minimum of the current state into empty sub-slots.  Of the three sets the
+// next one is empty, and the one after it, which an earlier step may have read, is
+// emptied on the way for the first step to fill.  Captured graphs hold one set's
+// address: with them that set is emptied by a launch of its own.
+static int fill_slots(amrgpu_ctx *c)
+{
+    if (!c->graphs_enabled) {
+        c->sb = (c->sb + 1) % 3;
+        return launch_cfl(c, c->U[c->cur], c->slots(), c->slots(1));
+    }
+    hipLaunchKernelGGL(slot_reset_kernel, dim3(1), dim3(256), 0, c->stream, c->slots(), c->ninst);
+    HIPCHK(hipGetLastError());
+    return launch_cfl(c, c->U[c->cur], c->slots(), nullptr);
+}
+
 int amrgpu_cfl(amrgpu_ctx *c, double *dt_inst)
 {
     if (!c || !dt_inst || !c->nquad) { set_err("amrgpu_cfl: no mesh"); return AMRGPU_ERR_ARG; }
-    hipLaunchKernelGGL(slot_reset_kernel, dim3(1), dim3(256), 0, c->stream, c->slots(), c->ninst);
-    HIPCHK(hipGetLastError());
-    int rc = launch_cfl(c, c->U[c->cur], c->slots(), nullptr);
+    int rc = fill_slots(c);
     if (rc) return rc;
     // the sub-slots reduced on the device, straight into pinned memory
     if ((rc = take_res(c, sizeof(double) * c->ninst))) return rc;
@@ -3873,17 +3888,7 @@ static int prime_run(amrgpu_ctx *c)
     if (int rc = geometry_ready(c)) return rc;
     // CFL sub-slots of the current state for the first step's dt
     c->self_dt = wants_self(c);
-    if (c->self_dt) {
-        // of the three sets the next one is empty; the one after it, which the
-        // last step read, is emptied on the way for the first step to fill
-        if (c->scheme == 2) return AMRGPU_OK;
-        c->sb = (c->sb + 1) % 3;
-        return launch_cfl(c, c->U[c->cur], c->slots(), c->slots(1));
-    }
-    hipLaunchKernelGGL(slot_reset_kernel, dim3(1), dim3(256), 0, c->stream, c->slots(), c->ninst);
-    HIPCHK(hipGetLastError());
-    if (c->scheme != 2) return launch_cfl(c, c->U[c->cur], c->slots(), nullptr);
-    return AMRGPU_OK;
+    return c->scheme != 2 ? fill_slots(c) : AMRGPU_OK;
 }
 
 static int graph_for(amrgpu_ctx *c, int cur, hipGraphExec_t *out)
@@ -3984,7 +3989,7 @@ int amrgpu_set_time(amrgpu_ctx *c, const double *t_inst)
     if (int rc = take_res(c, sizeof(double) * c->ninst)) return rc;
     memcpy(c->res.p, t_inst, sizeof(double) * c->ninst);
     hipLaunchKernelGGL(clock_kernel, dim3(1), dim3(64), 0, c->stream, c->t_now(), (double *)nullptr, c->t_step(),
-                       (const double *)c->res.p, c->ninst);
+                       (const double *)c->res.p, c->ninst, (unsigned long long *)nullptr, 0);
     HIPCHK(hipGetLastError());
     return sync_stream(c);
 }

@@ -60,3 +60,28 @@ def test_norm_does_not_depend_on_the_direction(n):
             norms.append(g.run(1))
         assert norms[0] == norms[1], tile
     g.close()
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("n,level", [(4, 3), (8, 3), (8, 8), (16, 2)])
+def test_cfl_of_the_state_at_hand(n, level, graphs):
+    """the CFL minimum turns through the sets of sub-slots: asked for several
+    times in a row, between runs and after a new state, it is that of a context
+    that holds this state alone, and the runs go on as they would without it"""
+    g, ref = uniform(n, level, 2, 3), uniform(n, level, 2, 3)
+    g.set_graphs(graphs)
+    alone = uniform(n, level, 2, 3)
+    for k in (1, 2, 3):
+        g.run(k)
+        ref.run(k)
+        for _ in range(4):
+            got = g.cfl()
+        q = g.soln()
+        assert np.array_equal(q, ref.soln())
+        alone.upload(q)
+        assert np.array_equal(got, alone.cfl())
+    alone.upload(q * 1.25)
+    g.upload(q * 1.25)
+    assert np.array_equal(g.cfl(), alone.cfl())
+    for c in (g, ref, alone):
+        c.close()
