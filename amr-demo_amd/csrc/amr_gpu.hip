@@ -44,8 +44,8 @@ constexpr unsigned long long DBL_INF_BITS = 0x7ff0000000000000ull;
 // folds into sub-slot b % NSLOT): atomics on one address serialise, and on a
 // 16.8M-cell mesh with one patch per workgroup 64 sub-slots still left the
 // last stage ~17 % slower than the others (4096 atomics per address); 256
-// recover most of it, and the one wave per instance of the next step's
-// dt_prep_kernel reduces them with four loads per lane.
+// recover most of it, and a wave of the next step (dt_prep_kernel's, or a first
+// stage's) reduces them with four loads per lane.
 constexpr int NSLOT = 256;
 
 struct InstDev {
@@ -1653,8 +1653,8 @@ __global__ __launch_bounds__(N * N, MINW) void stage_kernel_pp(StageArgs a)
 // one wave needs no barrier (its LDS operations execute in order).  LDS holds
 // the rows in flight and the halo only, 9 KB (R = 4) or 14 KB (R = 2) a wave.
 // Measured, us per SSP-RK3 step, DESIGN 0 -> this: 2x2 patches 262k quadrants
-// 238 -> 104, 16k 26.8 -> 17.6; 4x4 patches 176k quadrants (adaptive) 404 -> 240,
-// 21k 43.3 -> 29.1, 256 21.5 -> 13.3.
+// 237 -> 99.6, 16k 26.6 -> 18.4; 4x4 patches 176k quadrants (adaptive) 391 -> 220,
+// 21k 42.4 -> 25.8, 256 21.8 -> 16.0.
 // ---------------------------------------------------------------------------
 struct Rec {
     double r, ru, rv, rE, p, ir, sr;
@@ -2761,15 +2761,16 @@ int grid_of(const amrgpu_ctx *c, int v, int nquad)
 // 21.4 and 21.4 us a step, 18.8k 85.9 and 84.0, 159k 672 and 664, 131k uniform
 // 522 and 526).
 // n = 2 and 4: the row-marching kernel, faster than the others at every size
-// measured (16 to 262k quadrants).  n = 4 takes two rows a step, with fewer
-// instructions a patch, where its waves of 8 patches fill the chip (256 CUs x
-// 11 waves x 8 = 22k quadrants), else four, with twice the waves: 4k quadrants
-// 18.2 against 15.9 us a step, 20k 29.0 and 29.2, 66k 83.3 and 86.7.
+// measured (16 to 262k quadrants).  n = 4 takes four rows a step, with twice the
+// waves, while these are on the chip together (256 CUs x 12 waves x 4 patches =
+// 12288 quadrants), else two, with fewer instructions a patch: us per SSP-RK3 step
+// with two / four, 4k quadrants 18.7 / 16.9, 12k 24.2 / 23.6 (adaptive 29.4 / 26.0),
+// 16k 25.8 / 29.5, 21k (adaptive) 25.7 / 27.1, 66k 77.9 / 87.1.
 int default_variant(int n, int nquad)
 {
     switch (n) {
     case 2: return 20;
-    case 4: return nquad < 20000 ? 21 : 22;
+    case 4: return nquad <= 12288 ? 21 : 22;
     case 8: return 17;
     case 16: return 19;
     default: return -1;
