@@ -2578,9 +2578,9 @@ namespace {
 
 // Pinned host memory.  Copies between it and the device are plain DMA, where
 // pageable ones go through the runtime's own staging one call at a time; making
-// it costs 70-400 us and more, so contexts borrow it while copies are under way
-// and give it back at the next wait: at most PIN_KEEP bytes wait for the next
-// borrower, the rest is freed.
+// it (and freeing it) costs 70-400 us for small blocks and 15 ms for 75 MB, so contexts take it from
+// a pool and give it back (the chunks at the next wait, the rest when they are
+// destroyed): at most PIN_KEEP bytes wait for the next borrower, the rest is freed.
 struct PinBlock {
     void *p = nullptr;
     size_t cap = 0;
@@ -2691,10 +2691,12 @@ struct amrgpu_ctx {
     // autotuner measures it faster.
     bool graphs_enabled = false;
     std::vector<InstDev> h_ip;
-    // pinned memory: small results (kept); mesh uploads and the chunks that states
-    // and other arrays of the caller travel through, with an event per chunk
-    // (borrowed until nothing is pending on them)
+    // pinned memory: small results and mesh uploads (kept: a mesh of a million
+    // quadrants needs more than the pool holds); the chunks that states and other
+    // arrays of the caller travel through, with an event per chunk (borrowed until
+    // nothing is pending on them)
     PinBlock res, up, ring;
+    bool up_busy = false;                      // copies from `up` may be under way
     hipEvent_t ring_ev[RING_SLOTS] = {};
     int cu_count = 256;        // compute units of the context's device
 };
@@ -3137,7 +3139,7 @@ constexpr size_t MESH_BYTES = 2 * sizeof(double) + 11 * sizeof(int);     // per 
 int sync_stream(amrgpu_ctx *c)
 {
     HIPCHK(hipStreamSynchronize(c->stream));
-    pin_give(c->up);
+    c->up_busy = false;
     pin_give(c->ring);
     return AMRGPU_OK;
 }
@@ -3145,8 +3147,9 @@ int sync_stream(amrgpu_ctx *c)
 // The pinned area of mesh uploads, free for `bytes` to be written.
 int take_up(amrgpu_ctx *c, size_t bytes)
 {
-    if (c->up.p)
+    if (c->up_busy)
         if (int rc = sync_stream(c)) return rc;
+    c->up_busy = true;
     return pin_take(c->up, bytes);
 }
 

@@ -1,0 +1,136 @@
+"""Pinned host memory and the copies of the caller's arrays, without a GPU: a C
+program that brings its own runtime (device memory is malloc, kernels do nothing)
+counts what the library asks of it."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+LIB_DIR = os.path.join(ROOT, "amr-demo_amd")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+pytestmark = pytest.mark.skipif(shutil.which("gcc") is None or not os.path.isdir(os.path.join(ROCM, "include")),
+                                reason="gcc or the HIP headers absent")
+
+RUNTIME = r"""
+#define __HIP_PLATFORM_AMD__
+#include <hip/hip_runtime_api.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include "amr_hip.h"
+
+/* what the library asked for */
+static int host_allocs, copies, launches;
+static const void *copy_src[1024];
+static void *copy_dst[1024];
+/* the caller's pinned array */
+static char *mine;
+static size_t mine_bytes;
+
+hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; ++host_allocs; *p = malloc(n); return hipSuccess; }
+hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n); return hipSuccess; }
+hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
+{
+    (void)k; (void)st;
+    copy_src[copies % 1024] = s;
+    copy_dst[copies++ % 1024] = d;
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
+{
+    memset(a, 0, sizeof(*a));
+    a->type = hipMemoryTypeUnregistered;
+    if (mine && (const char *)p >= mine && (const char *)p < mine + mine_bytes) {
+        a->type = hipMemoryTypeHost;
+        a->hostPointer = (void *)p;
+        a->devicePointer = (void *)p;
+    }
+    return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t e) { (void)e; return "error"; }
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = 256; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { (void)f; *s = (hipStream_t)&copies; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { (void)f; *e = (hipEvent_t)&launches; return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { (void)e; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { (void)e; (void)s; return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e) { (void)e; return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t n, hipStream_t s) { (void)g; (void)b; (void)n; (void)s; return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *n, hipStream_t *s)
+{
+    memset(g, 0, sizeof(*g)); memset(b, 0, sizeof(*b)); *n = 0; *s = 0;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t n, hipStream_t s)
+{
+    (void)f; (void)g; (void)b; (void)a; (void)n; (void)s;
+    ++launches;
+    return hipSuccess;
+}
+
+#define MUST(x) do { int rc_ = (x); if (rc_) { printf("%s: %d %s\n", #x, rc_, amrgpu_last_error()); return 1; } } while (0)
+#define HOLDS(x) do { if (!(x)) { printf("line %d: %s does not hold\n", __LINE__, #x); return 1; } } while (0)
+
+/* nq quadrants of 2x2 cells with a wall on every side, zero state */
+static int set_up(amrgpu_ctx *c, int nq)
+{
+    int *ci = malloc(sizeof(int) * 3 * (size_t)nq), *fi = calloc((size_t)nq * 44, sizeof(int)), rc;
+    double *u = calloc((size_t)nq * 16, sizeof(double));
+    amrgpu_inst_t in;
+    memset(&in, 0, sizeof(in));
+    in.h_base = 1.0; in.cfl = 0.3; in.dt_cap = 1.0;
+    for (int q = 0; q < nq; ++q) {
+        ci[3 * q] = 0; ci[3 * q + 1] = 5; ci[3 * q + 2] = 16 * q;
+        for (int s = 0; s < 4; ++s) { int *f = fi + 11 * (4 * (size_t)q + s); f[0] = 1; f[1] = s; f[2] = q; }
+    }
+    rc = amrgpu_setup(c, 2, 3, 1, &in, nq, ci, NULL, 4 * nq, fi, NULL, u);
+    free(ci); free(fi); free(u);
+    return rc;
+}
+/* the same mesh again through a remesh */
+static int remesh(amrgpu_ctx *c, int nq)
+{
+    int *lev = calloc((size_t)nq, sizeof(int)), *nbr = malloc(sizeof(int) * 8 * (size_t)nq), *src = calloc((size_t)nq, sizeof(int)), rc;
+    for (size_t k = 0; k < 8 * (size_t)nq; ++k) nbr[k] = -1;
+    rc = amrgpu_remesh_nbr(c, nq, lev, NULL, nbr, src);
+    free(lev); free(nbr); free(src);
+    return rc;
+}
+"""
+
+
+def run(tmp_path, body):
+    """the statements `body` of a program with that runtime; 0 is success"""
+    src, exe = tmp_path / "t.c", tmp_path / "t"
+    src.write_text(RUNTIME + "int main(void)\n{\n" + body + "    return 0;\n}\n")
+    r = subprocess.run(["gcc", "-std=gnu11", "-O1", "-Wall", "-Wno-unused-function", f"-I{ROOT}/include",
+                        f"-I{ROCM}/include", str(src), f"-L{LIB_DIR}", "-lamrhip", f"-Wl,-rpath,{LIB_DIR}",
+                        "-rdynamic", f"-Wl,-rpath-link,{ROCM}/lib", "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("nq", [1, 100001, 1000000, 1500000])
+def test_no_pinned_allocation_by_repeated_setups_and_remeshes(tmp_path, nq):
+    """whatever the mesh's size, the pinned area its tables pass through is
+    made once per context"""
+    run(tmp_path, f"""
+    amrgpu_ctx *c = amrgpu_create();
+    for (int k = 0; k < 2; ++k) {{ MUST(set_up(c, {nq})); MUST(remesh(c, {nq})); }}
+    const int before = host_allocs;
+    for (int k = 0; k < 2; ++k) {{ MUST(set_up(c, {nq})); MUST(remesh(c, {nq})); }}
+    HOLDS(host_allocs == before);
+    amrgpu_destroy(c);
+""")
