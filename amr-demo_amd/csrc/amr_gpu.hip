@@ -2577,10 +2577,11 @@ extern "C" void amr_set_error(const char *fmt, ...)
 namespace {
 
 // Pinned host memory.  Copies between it and the device are plain DMA, where
-// pageable ones go through the runtime's own staging one call at a time; making
-// it (and freeing it) costs 70-400 us for small blocks and 15 ms for 75 MB, so contexts take it from
-// a pool and give it back (the chunks at the next wait, the rest when they are
-// destroyed): at most PIN_KEEP bytes wait for the next borrower, the rest is freed.
+// pageable ones go through the runtime's own staging one call at a time; making it
+// (and freeing it) costs 70-400 us for small blocks and 15 ms for 75 MB, so contexts
+// take it from a pool and give it back (the chunks at the next wait, the rest when
+// they are destroyed): at most PIN_KEEP bytes wait for the next borrower, the rest
+// is freed.
 struct PinBlock {
     void *p = nullptr;
     size_t cap = 0;
@@ -3639,12 +3640,38 @@ static int check_src(int ncell, const int *src, int nold, const char *who)
     return AMRGPU_OK;
 }
 
-// Remap the state onto a validated new mesh and upload its table.  `h` is the
-// table packed in the pinned area (corners unset).
-static int remesh_to(amrgpu_ctx *c, int ncell, const MeshPlace &h, const int *cell_inst)
+// A validated new mesh as its caller has it: the face table (null: in the pinned
+// area already), the levels (lstep ints apart), the instance ids (null: all 0).
+struct NewMesh {
+    int ncell;
+    const int *nbr, *level;
+    int lstep;
+    const int *inst;
+};
+
+static void put_table(const NewMesh &m, const MeshPlace &h)
 {
+    if (m.nbr) memcpy(h.nbr, m.nbr, sizeof(int) * 8 * (size_t)m.ncell);
+    if (m.lstep == 1) memcpy(h.level, m.level, sizeof(int) * (size_t)m.ncell);
+    else
+        for (int q = 0; q < m.ncell; ++q) h.level[q] = m.level[(size_t)m.lstep * q];
+    put_ids(h.inst, m.inst, m.ncell);
+}
+
+// Remap the state onto a validated new mesh and upload its table, packed at `h` in
+// the pinned area (corners unset), with the source map.  From REMAP_FIRST quadrants
+// on the map goes ahead, and the remap runs while the host packs the rest: us per
+// remesh with one copy / two, 8x8 patches 256 quadrants 22.5 / 25.5, 16k 95 / 95,
+// 65k 338 / 301, 262k 1198 / 1056; 2x2 patches 1.0M 4850 / 4690.
+constexpr int REMAP_FIRST = 32768;
+static int remesh_to(amrgpu_ctx *c, const NewMesh &m, const MeshPlace &h, const int *src)
+{
+    const int ncell = m.ncell, *const cell_inst = m.inst;
     const int n2 = c->n * c->n, nold = c->nquad;
+    const bool first = ncell >= REMAP_FIRST;
     int rc = AMRGPU_OK;
+    put_ids(h.map, src, ncell);
+    if (!first) put_table(m, h);
     HIPCHK(hipStreamSynchronize(c->stream));
     free_graphs(c);
     const long long ncells = (long long)ncell * n2;
@@ -3680,10 +3707,16 @@ static int remesh_to(amrgpu_ctx *c, int ncell, const MeshPlace &h, const int *ce
     }
     rc = new_mesh(c, ncell, cell_inst);
     if (rc) { (void)hipFree(keep); return rc; }
-    HIPCHK(hipMemcpyAsync(c->d_nbr, h.nbr, (size_t)((char *)h.end - (char *)h.nbr), hipMemcpyHostToDevice, c->stream));
+    int *const part = first ? h.map : h.nbr;
+    HIPCHK(hipMemcpyAsync(first ? c->d_map : c->d_nbr, part, (size_t)((char *)h.end - (char *)part), hipMemcpyHostToDevice,
+                          c->stream));
     hipLaunchKernelGGL(remap_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream, from, c->U[to],
                        c->d_map, ncells, n2);
     HIPCHK(hipGetLastError());
+    if (first) {
+        put_table(m, h);
+        HIPCHK(hipMemcpyAsync(c->d_nbr, h.nbr, (size_t)((char *)h.map - (char *)h.nbr), hipMemcpyHostToDevice, c->stream));
+    }
     c->cur = to;
     if ((rc = sync_stream(c))) return rc;
     (void)hipFree(keep);
@@ -3731,11 +3764,8 @@ int amrgpu_remesh(amrgpu_ctx *c, int ncell, const int *cell_info, const int *cel
     const MeshPlace h = place_mesh((char *)c->up.p, ncell);
     rc = build_nbr(ncell, nface, face_info, h.nbr);
     if (rc) return rc;                 // a refused call leaves the context as it was
-    for (int q = 0; q < ncell; ++q) h.level[q] = cell_info[3 * q + 1];
-    put_ids(h.inst, cell_inst, ncell);
-    put_ids(h.map, src, ncell);
     c->org_ok = false;                 // the new quadrants' coordinates come with amrgpu_set_geometry
-    return remesh_to(c, ncell, h, cell_inst);
+    return remesh_to(c, {ncell, nullptr, cell_info + 1, 3, cell_inst}, h, src);
 }
 
 int amrgpu_remesh_nbr(amrgpu_ctx *c, int ncell, const int *level, const int *cell_inst, const int *nbr,
@@ -3768,12 +3798,8 @@ int amrgpu_remesh_nbr(amrgpu_ctx *c, int ncell, const int *level, const int *cel
     rc = take_up(c, MESH_BYTES * (size_t)ncell);
     if (rc) return rc;
     const MeshPlace h = place_mesh((char *)c->up.p, ncell);
-    memcpy(h.nbr, nbr, sizeof(int) * 8 * (size_t)ncell);
-    put_ids(h.level, level, ncell);
-    put_ids(h.inst, cell_inst, ncell);
-    put_ids(h.map, src, ncell);
     c->org_ok = false;                 // the new quadrants' coordinates come with amrgpu_set_origins
-    return remesh_to(c, ncell, h, cell_inst);
+    return remesh_to(c, {ncell, nbr, level, 1, cell_inst}, h, src);
 }
 
 int amrgpu_set_origins(amrgpu_ctx *c, const double *org)

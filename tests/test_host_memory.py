@@ -24,7 +24,7 @@ RUNTIME = r"""
 #include "amr_hip.h"
 
 /* what the library asked for */
-static int host_allocs, copies, launches;
+static int host_allocs, copies, launches, copies_at_launch;
 static const void *copy_src[1024];
 static void *copy_dst[1024];
 /* the caller's pinned array */
@@ -75,6 +75,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t n, hi
 {
     (void)f; (void)g; (void)b; (void)a; (void)n; (void)s;
     ++launches;
+    copies_at_launch = copies;
     return hipSuccess;
 }
 
@@ -82,21 +83,21 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t n, hi
 #define HOLDS(x) do { if (!(x)) { printf("line %d: %s does not hold\n", __LINE__, #x); return 1; } } while (0)
 
 /* nq quadrants of 2x2 cells with a wall on every side, zero state */
-static int set_up(amrgpu_ctx *c, int nq)
+static int set_up_n(amrgpu_ctx *c, int nq, int ninst)
 {
     int *ci = malloc(sizeof(int) * 3 * (size_t)nq), *fi = calloc((size_t)nq * 44, sizeof(int)), rc;
     double *u = calloc((size_t)nq * 16, sizeof(double));
-    amrgpu_inst_t in;
-    memset(&in, 0, sizeof(in));
-    in.h_base = 1.0; in.cfl = 0.3; in.dt_cap = 1.0;
+    amrgpu_inst_t *in = calloc((size_t)ninst, sizeof(*in));
+    for (int k = 0; k < ninst; ++k) { in[k].h_base = 1.0; in[k].cfl = 0.3; in[k].dt_cap = 1.0; }
     for (int q = 0; q < nq; ++q) {
         ci[3 * q] = 0; ci[3 * q + 1] = 5; ci[3 * q + 2] = 16 * q;
         for (int s = 0; s < 4; ++s) { int *f = fi + 11 * (4 * (size_t)q + s); f[0] = 1; f[1] = s; f[2] = q; }
     }
-    rc = amrgpu_setup(c, 2, 3, 1, &in, nq, ci, NULL, 4 * nq, fi, NULL, u);
-    free(ci); free(fi); free(u);
+    rc = amrgpu_setup(c, 2, 3, ninst, in, nq, ci, NULL, 4 * nq, fi, NULL, u);
+    free(ci); free(fi); free(u); free(in);
     return rc;
 }
+static int set_up(amrgpu_ctx *c, int nq) { return set_up_n(c, nq, 1); }
 /* the same mesh again through a remesh */
 static int remesh(amrgpu_ctx *c, int nq)
 {
@@ -132,5 +133,40 @@ def test_no_pinned_allocation_by_repeated_setups_and_remeshes(tmp_path, nq):
     const int before = host_allocs;
     for (int k = 0; k < 2; ++k) {{ MUST(set_up(c, {nq})); MUST(remesh(c, {nq})); }}
     HOLDS(host_allocs == before);
+    amrgpu_destroy(c);
+""")
+
+
+@pytest.mark.parametrize("faces", [0, 1])
+@pytest.mark.parametrize("nq", [1, 32767, 32768, 100001])
+def test_a_remesh_uploads_the_table_and_remaps_a_large_mesh_ahead_of_it(tmp_path, nq, faces):
+    """the device holds the face table, levels, instance ids and source map of
+    the new mesh, one after the other; from 32768 quadrants on the remap is
+    launched ahead of the table's copy: it runs while the host packs the table"""
+    run(tmp_path, f"""
+    enum {{ nq = {nq} }};
+    static int lev[nq], inst[nq], nbr[8 * nq], src[nq], ci[3 * nq], fi[44 * nq];
+    for (int q = 0; q < nq; ++q) {{
+        lev[q] = q % 30; inst[q] = q % 3; src[q] = nq - 1 - q;
+        ci[3 * q + 1] = lev[q]; ci[3 * q + 2] = 16 * q;
+        for (int s = 0; s < 4; ++s) {{
+            int *f = fi + 11 * (4 * q + s);
+            f[0] = 1; f[1] = s; f[2] = q;
+            nbr[8 * q + 2 * s] = {faces} ? -1 : (q * 7 + s) % nq;
+            nbr[8 * q + 2 * s + 1] = -1;
+        }}
+    }}
+    amrgpu_ctx *c = amrgpu_create();
+    MUST(set_up_n(c, nq, 3));
+    if ({faces}) MUST(amrgpu_remesh(c, nq, ci, inst, 4 * nq, fi, src));
+    else MUST(amrgpu_remesh_nbr(c, nq, lev, inst, nbr, src));
+    const int *d, *p;
+    MUST(amrgpu_device_state(c, NULL, &d, NULL, NULL, NULL));
+    p = d;
+    HOLDS(memcmp(p, nbr, sizeof(nbr)) == 0); p += 8 * nq;
+    HOLDS(memcmp(p, lev, sizeof(lev)) == 0); p += nq;
+    HOLDS(memcmp(p, inst, sizeof(inst)) == 0); p += nq;
+    HOLDS(memcmp(p, src, sizeof(src)) == 0);
+    HOLDS(nq < 3 || (copies > copies_at_launch) == (nq >= 32768));    /* (every instance has quadrants) */
     amrgpu_destroy(c);
 """)
