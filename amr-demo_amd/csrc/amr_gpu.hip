@@ -2607,17 +2607,22 @@ void pin_give(PinBlock &b)
     b = PinBlock();
 }
 
-// A block of at least `bytes` (the smallest that waits, or a new one with a
-// quarter to spare) in place of b, whose contents are dropped.
+// A block of at least `bytes` (the smallest that waits and is no more than four times
+// a new one's size: a small area kept for a context's life must not hold what the
+// next large copy needs; or a new one with a quarter to spare) in place of b, whose
+// contents are dropped.
 int pin_take(PinBlock &b, size_t bytes)
 {
     if (b.cap >= bytes) return AMRGPU_OK;
+    const size_t cap = (bytes + bytes / 4 + 65535) / 65536 * 65536;
     pin_give(b);
     {
         std::lock_guard<std::mutex> hold(g_pin_lock);
         int best = -1;
-        for (int k = 0; k < (int)g_pin_free.size(); ++k)
-            if (g_pin_free[k].cap >= bytes && (best < 0 || g_pin_free[k].cap < g_pin_free[best].cap)) best = k;
+        for (int k = 0; k < (int)g_pin_free.size(); ++k) {
+            const size_t have = g_pin_free[k].cap;
+            if (have >= bytes && have <= 4 * cap && (best < 0 || have < g_pin_free[best].cap)) best = k;
+        }
         if (best >= 0) {
             b = g_pin_free[best];
             g_pin_bytes -= b.cap;
@@ -2625,7 +2630,6 @@ int pin_take(PinBlock &b, size_t bytes)
             return AMRGPU_OK;
         }
     }
-    const size_t cap = (bytes + bytes / 4 + 65535) / 65536 * 65536;
     HIPCHK(hipHostMalloc(&b.p, cap, hipHostMallocPortable));
     b.cap = cap;
     return AMRGPU_OK;

@@ -170,3 +170,18 @@ def test_a_remesh_uploads_the_table_and_remaps_a_large_mesh_ahead_of_it(tmp_path
     HOLDS(nq < 3 || (copies > copies_at_launch) == (nq >= 32768));    /* (every instance has quadrants) */
     amrgpu_destroy(c);
 """)
+
+
+def test_the_small_results_keep_no_transfer_chunks(tmp_path):
+    """a context's small results take a block of their size, not the transfer
+    chunks that wait for the next copy"""
+    run(tmp_path, """
+    amrgpu_ctx *c = amrgpu_create();
+    static double t, dt, u[16 * 256];
+    MUST(set_up(c, 256));
+    MUST(amrgpu_get_time(c, &t, &dt));
+    const int before = host_allocs;
+    for (int k = 0; k < 3; ++k) { MUST(amrgpu_upload_soln(c, u)); MUST(amrgpu_get_time(c, &t, &dt)); }
+    HOLDS(host_allocs == before);
+    amrgpu_destroy(c);
+""")
