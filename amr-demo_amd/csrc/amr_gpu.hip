@@ -2580,8 +2580,8 @@ namespace {
 // pageable ones go through the runtime's own staging one call at a time; making it
 // (and freeing it) costs 70-400 us for small blocks and 15 ms for 75 MB, so contexts
 // take it from a pool and give it back (the chunks at the next wait, the rest when
-// they are destroyed): at most PIN_KEEP bytes wait for the next borrower, the rest
-// is freed.
+// they are destroyed): at most PIN_KEEP bytes wait for the next borrower, those
+// given back last; the rest is freed.
 struct PinBlock {
     void *p = nullptr;
     size_t cap = 0;
@@ -2594,16 +2594,18 @@ size_t g_pin_bytes = 0;
 void pin_give(PinBlock &b)
 {
     if (!b.p) return;
-    bool keep;
+    std::vector<PinBlock> old;
     {
         std::lock_guard<std::mutex> hold(g_pin_lock);
-        keep = g_pin_bytes + b.cap <= PIN_KEEP;
-        if (keep) {
-            g_pin_free.push_back(b);
-            g_pin_bytes += b.cap;
+        g_pin_free.push_back(b);
+        g_pin_bytes += b.cap;
+        while (g_pin_bytes > PIN_KEEP) {
+            old.push_back(g_pin_free.front());
+            g_pin_bytes -= g_pin_free.front().cap;
+            g_pin_free.erase(g_pin_free.begin());
         }
     }
-    if (!keep) (void)hipHostFree(b.p);
+    for (PinBlock &o : old) (void)hipHostFree(o.p);
     b = PinBlock();
 }
 

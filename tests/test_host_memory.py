@@ -185,3 +185,23 @@ def test_the_small_results_keep_no_transfer_chunks(tmp_path):
     HOLDS(host_allocs == before);
     amrgpu_destroy(c);
 """)
+
+
+def test_the_pool_keeps_what_was_given_back_last(tmp_path):
+    """pinned blocks of sizes that nobody asks for any more do not keep the pool
+    full: contexts that come and go with the same mesh make no new ones"""
+    run(tmp_path, """
+    int before = 0;
+    for (int nq = 150000; nq < 600000; nq += nq / 3) {       /* one size after the other, each larger than the last block */
+        amrgpu_ctx *c = amrgpu_create();
+        MUST(set_up(c, nq));
+        amrgpu_destroy(c);
+    }
+    for (int k = 0; k < 4; ++k) {
+        amrgpu_ctx *c = amrgpu_create();
+        MUST(set_up(c, 600000));
+        amrgpu_destroy(c);
+        if (k == 1) before = host_allocs;
+    }
+    HOLDS(host_allocs == before);
+""")
