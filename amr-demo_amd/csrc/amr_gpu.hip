@@ -3170,10 +3170,32 @@ int take_ring(amrgpu_ctx *c)
     return AMRGPU_OK;
 }
 
-// The caller's `bytes` at src to the device; src may change once it returns, the
-// copy is ordered on the stream.
-int copy_in(amrgpu_ctx *c, void *dst, const void *src, size_t bytes)
+// Whether the caller keeps an array in memory that the device reaches by itself
+// (pinned): it needs no chunks.
+bool device_reaches(const void *p)
 {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();       // (how some versions say that they do not know the address)
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
+// The caller's `bytes` at src to the device, ordered on the stream.  src may change
+// once it returns, or with `stays` at the next wait for the stream only: then large
+// arrays are left to the runtime's own staging (us per upload of a state, chunks /
+// runtime once warm: 32 KB 22 / 35, 512 KB 37.5 / 38, 2 MB 98 / 93, 6 MB 195 / 203,
+// 24 MB 678 / 697, 32 MB 1010 / 945, 512 MB 18890 / 18220; for its first tens of calls
+// a process pays it up to 200 us each, so smaller arrays stay with the chunks).
+// Pinned arrays go as they are (8 MB through chunks 260, as it is 171).
+constexpr size_t IN_CHUNKS_MAX = (size_t)24 << 20;
+int copy_in(amrgpu_ctx *c, void *dst, const void *src, size_t bytes, bool stays)
+{
+    if ((stays && bytes > IN_CHUNKS_MAX) || device_reaches(src)) {
+        HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+        return stays ? AMRGPU_OK : sync_stream(c);
+    }
     if (int rc = take_ring(c)) return rc;
     int k = 0;
     for (size_t at = 0; at < bytes; at += RING_CHUNK, ++k) {
@@ -3188,9 +3210,15 @@ int copy_in(amrgpu_ctx *c, void *dst, const void *src, size_t bytes)
     return AMRGPU_OK;
 }
 
-// `bytes` of the device at src, after what the stream holds, to the caller.
+// `bytes` of the device at src, after what the stream holds, to the caller.  Pinned
+// arrays are written as they are: us per download, through chunks / as it is, 512 KB
+// 43.8 / 32.7, 8 MB 380 / 180, 128 MB 4700 / 2420.
 int copy_out(amrgpu_ctx *c, void *dst, const void *src, size_t bytes)
 {
+    if (device_reaches(dst)) {
+        HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        return sync_stream(c);
+    }
     if (int rc = take_ring(c)) return rc;
     const int chunks = (int)((bytes + RING_CHUNK - 1) / RING_CHUNK);
     auto size = [&](int k) { return std::min(RING_CHUNK, bytes - k * RING_CHUNK); };
@@ -3478,12 +3506,13 @@ static int set_clocks(amrgpu_ctx *c, const double *t_inst)
     return AMRGPU_OK;
 }
 
-// The reference-layout state to the device, ordered on the stream.
+// The reference-layout state to the device, ordered on the stream; it stays as it is
+// until the stream is waited for.
 static int start_upload(amrgpu_ctx *c, const double *soln)
 {
     const int n2 = c->n * c->n;
     const long long ncells = (long long)c->nquad * n2;
-    if (int rc = copy_in(c, c->d_stage, soln, sizeof(double) * 4 * ncells)) return rc;
+    if (int rc = copy_in(c, c->d_stage, soln, sizeof(double) * 4 * ncells, true)) return rc;
     c->cur = 0;
     hipLaunchKernelGGL(aos_to_soa_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
                        c->d_stage, c->U[0], ncells, n2);
@@ -3811,7 +3840,7 @@ int amrgpu_remesh_nbr(amrgpu_ctx *c, int ncell, const int *level, const int *cel
 int amrgpu_set_origins(amrgpu_ctx *c, const double *org)
 {
     if (!c || !c->nquad || !org) { set_err("amrgpu_set_origins: no mesh"); return AMRGPU_ERR_ARG; }
-    if (int rc = copy_in(c, c->d_org, org, sizeof(double) * 2 * (size_t)c->nquad)) return rc;
+    if (int rc = copy_in(c, c->d_org, org, sizeof(double) * 2 * (size_t)c->nquad, false)) return rc;
     c->org_ok = true;
     return AMRGPU_OK;
 }

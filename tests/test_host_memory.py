@@ -27,6 +27,7 @@ RUNTIME = r"""
 static int host_allocs, copies, launches, copies_at_launch;
 static const void *copy_src[1024];
 static void *copy_dst[1024];
+static size_t copy_bytes[1024];
 /* the caller's pinned array */
 static char *mine;
 static size_t mine_bytes;
@@ -39,6 +40,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
 {
     (void)k; (void)st;
     copy_src[copies % 1024] = s;
+    copy_bytes[copies % 1024] = n;
     copy_dst[copies++ % 1024] = d;
     memcpy(d, s, n);
     return hipSuccess;
@@ -204,4 +206,64 @@ def test_the_pool_keeps_what_was_given_back_last(tmp_path):
         if (k == 1) before = host_allocs;
     }
     HOLDS(host_allocs == before);
+""")
+
+
+def test_the_callers_pinned_arrays_go_to_the_device_as_they_are(tmp_path):
+    """no pass through the library's own chunks, in either direction"""
+    run(tmp_path, """
+    enum { nq = 4096, bytes = nq * 16 * 8 };
+    mine = calloc(bytes, 1);
+    mine_bytes = bytes;
+    double *u = (double *)mine;
+    amrgpu_ctx *c = amrgpu_create();
+    MUST(set_up(c, nq));
+    int k = copies;
+    MUST(amrgpu_upload_soln(c, u));
+    HOLDS(copies == k + 1 && copy_src[k] == u && copy_bytes[k] == bytes);
+    k = copies;
+    MUST(amrgpu_download_soln(c, u));
+    HOLDS(copies == k + 1 && copy_dst[k] == u && copy_bytes[k] == bytes);
+    k = copies;
+    MUST(amrgpu_rhs(c, u));
+    HOLDS(copies == k + 1 && copy_dst[k] == u && copy_bytes[k] == bytes);
+    k = copies;
+    MUST(amrgpu_indicator(c, u));
+    HOLDS(copies == k + 1 && copy_dst[k] == u && copy_bytes[k] == nq * 8);
+    k = copies;
+    MUST(amrgpu_set_origins(c, u));
+    HOLDS(copies == k + 1 && copy_src[k] == u && copy_bytes[k] == nq * 16);
+    amrgpu_destroy(c);
+""")
+
+
+@pytest.mark.parametrize("nq,parts", [(1, 1), (16384, 1), (16385, 2), (100001, 7), (196608, 12), (196609, 1), (300000, 1)])
+def test_an_upload_arrives_whole(tmp_path, nq, parts):
+    """through the library's chunks of 2 MB up to 24 MB, left to the runtime beyond"""
+    run(tmp_path, f"""
+    const size_t bytes = {nq} * 128ul;
+    unsigned char *u = malloc(bytes);
+    for (size_t i = 0; i < bytes; ++i) u[i] = (unsigned char)(i * 2654435761u >> 13);
+    amrgpu_ctx *c = amrgpu_create();
+    MUST(set_up(c, {nq}));
+    const int k = copies;
+    MUST(amrgpu_upload_soln(c, (double *)u));
+    HOLDS(copies == k + {parts} && (copy_src[k] == u) == (bytes > 24 << 20) && memcmp(copy_dst[k], u, bytes) == 0);
+    amrgpu_destroy(c);
+""")
+
+
+@pytest.mark.parametrize("nq,parts", [(1, 1), (131072, 1), (131073, 2), (400000, 4)])
+def test_the_corners_may_change_once_they_are_set(tmp_path, nq, parts):
+    """they always pass through the chunks of 2 MB"""
+    run(tmp_path, f"""
+    const size_t bytes = {nq} * 16ul;
+    unsigned char *u = malloc(bytes);
+    for (size_t i = 0; i < bytes; ++i) u[i] = (unsigned char)(i * 2654435761u >> 13);
+    amrgpu_ctx *c = amrgpu_create();
+    MUST(set_up(c, {nq}));
+    const int k = copies;
+    MUST(amrgpu_set_origins(c, (double *)u));
+    HOLDS(copies == k + {parts} && copy_src[k] != u && memcmp(copy_dst[k], u, bytes) == 0);
+    amrgpu_destroy(c);
 """)
