@@ -2849,6 +2849,10 @@ void with_vectors(const StageArgs &a, F f)
     else f(std::integral_constant<int, BASE>());
 }
 
+// Tiles whose first stage can form the step's dt itself (compiled for them only).
+constexpr bool forms_dt(int ppb, int minw, int design) { return design == 3 || (design == 1 && ppb == 1 && minw >= 4); }
+bool has_self(int v) { return forms_dt(kVariants[v].ppb, kVariants[v].minw, kVariants[v].design); }
+
 template <int N, int PPB, int MINW, int D>
 int launch_v(amrgpu_ctx *c, const StageArgs &a)
 {
@@ -2860,8 +2864,8 @@ int launch_v(amrgpu_ctx *c, const StageArgs &a)
             with_vectors<VEC_ANY>(a, [&](auto vec) {
                 constexpr bool SELF = decltype(self)::value, NT = decltype(nt)::value;
                 constexpr int VEC = decltype(vec)::value;
-                if constexpr (SELF && MINW < 4)
-                    return;        // (has_self)
+                if constexpr (SELF && !forms_dt(PPB, MINW, D))
+                    return;        // (not compiled; launch_stage refuses it)
                 else if constexpr (N == 8)
                     hipLaunchKernelGGL((stage_kernel_one<MINW, SELF, NT, VEC>), nblk, blk, 0, c->stream, a);
                 else
@@ -2896,6 +2900,11 @@ int launch_rows(amrgpu_ctx *c, const StageArgs &a)
 // 302 -> 285, 16x16 LSERK45 16k 603 -> 554; meshes that fit the cache 0 to 3 %).
 int launch_stage(amrgpu_ctx *c, const StageArgs &a0)
 {
+    const TileVariant &v = kVariants[c->variant];
+    if (a0.slot_in && !forms_dt(v.ppb, v.minw, v.design)) {
+        set_err("tile n=%d ppb=%d minw=%d design=%d has no first stage that forms dt", v.n, v.ppb, v.minw, v.design);
+        return AMRGPU_ERR_ARG;
+    }
     StageArgs a = a0;
     a.down = c->sweep_down;
     c->sweep_down = !c->sweep_down;
@@ -3037,12 +3046,6 @@ int build_step(amrgpu_ctx *c, int cur, std::vector<StageArgs> &st, bool with_nor
     default:
         return -1;
     }
-}
-
-// Tiles whose first stage can form the step's dt itself.
-bool has_self(int v)
-{
-    return kVariants[v].design == 3 || (kVariants[v].design == 1 && kVariants[v].ppb == 1 && kVariants[v].minw >= 4);
 }
 
 // Whether the steps of a run have no dt_prep_kernel.  That saves a launch and its

@@ -32,7 +32,7 @@ static size_t copy_bytes[1024];
 static char *mine;
 static size_t mine_bytes;
 
-hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; ++host_allocs; *p = malloc(n); return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; ++host_allocs; *p = calloc(n, 1); return hipSuccess; }
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n); return hipSuccess; }
 hipError_t hipFree(void *p) { free(p); return hipSuccess; }
@@ -266,4 +266,37 @@ def test_the_corners_may_change_once_they_are_set(tmp_path, nq, parts):
     MUST(amrgpu_set_origins(c, (double *)u));
     HOLDS(copies == k + {parts} && copy_src[k] != u && memcmp(copy_dst[k], u, bytes) == 0);
     amrgpu_destroy(c);
+""")
+
+
+@pytest.mark.parametrize("n", [2, 4, 8, 16])
+def test_every_tile_launches_every_stage(tmp_path, n):
+    """a step is the scheme's stages, after the dt kernel where the first stage
+    does not form dt itself: no tile leaves one out"""
+    run(tmp_path, f"""
+    enum {{ nq = 4, n = {n} }};
+    static int ci[3 * nq], fi[44 * nq], ppb[64], minw[64], design[64];
+    static double u[4 * n * n * nq], rn;
+    amrgpu_inst_t in;
+    memset(&in, 0, sizeof(in));
+    in.h_base = 1.0; in.cfl = 0.3; in.dt_cap = 1.0;
+    for (int q = 0; q < nq; ++q) {{
+        ci[3 * q + 2] = 4 * n * n * q;
+        for (int s = 0; s < 4; ++s) {{ int *f = fi + 11 * (4 * q + s); f[0] = 1; f[1] = s; f[2] = q; }}
+    }}
+    const int tiles = amrgpu_tile_variants(n, ppb, minw, design, 64);
+    HOLDS(tiles > 0 && tiles <= 64);
+    for (int scheme = 1; scheme <= 5; ++scheme)
+        for (int k = 0; k < tiles; ++k) {{
+            amrgpu_ctx *c = amrgpu_create();
+            MUST(amrgpu_setup(c, n, scheme, 1, &in, nq, ci, NULL, 4 * nq, fi, NULL, u));
+            MUST(amrgpu_set_tile(c, ppb[k], minw[k], design[k]));
+            const int l0 = launches;
+            MUST(amrgpu_run(c, 1, 0, &rn));
+            const int l1 = launches;
+            MUST(amrgpu_run(c, 3, 0, &rn));
+            const int step2 = (launches - l1) - (l1 - l0);       /* of two steps */
+            HOLDS(step2 == 2 * scheme || step2 == 2 * (scheme + 1));
+            amrgpu_destroy(c);
+        }}
 """)
