@@ -528,7 +528,7 @@ __device__ __forceinline__ void publish_dt(const StageArgs &a, int inst, double 
 }
 
 // The same for the instances without quadrants, a lane each, by the wave of the
-// first quadrant: no CFL minimum limits them.
+// first quadrant: they do not advance.
 __device__ __forceinline__ void publish_empty(const StageArgs &a)
 {
     const int lane = threadIdx.x & 63;
@@ -538,10 +538,9 @@ __device__ __forceinline__ void publish_empty(const StageArgs &a)
         if (left >> lane & 1) {
             const int i = 64 * w + lane;
             const double t = a.t_in[i];
-            const double dt = limited_dt(a.m.ip[i].dt_cap, a.m.ip[i].t_end, INFINITY, t, a.use_cfl);
-            a.dt_cur[i] = dt;
+            a.dt_cur[i] = 0.0;
             a.t_step[i] = t;
-            a.t_out[i] = t + dt;
+            a.t_out[i] = t;
         }
         for (; left; left &= left - 1) {
             unsigned long long *const s = a.slot_clear + (size_t)(64 * w + __ffsll(left) - 1) * NSLOT;
@@ -2292,23 +2291,26 @@ __global__ void slot_reset_kernel(unsigned long long *slot, int ninst)
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) slot[i] = DBL_INF_BITS;
 }
 
+// No last dt for the instances without quadrants.
+__global__ __launch_bounds__(256) void drop_dt_kernel(const int *has, int ninst, double *dt_cur)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < ninst && !has[i]) dt_cur[i] = 0.0;
+}
+
 // The step's dt and time update, ahead of its first stage: one wave per
 // instance forms min(input dt, CFL minimum over the instance's sub-slots,
 // time left), publishes it with the step's start time, advances the time and
 // re-arms the sub-slots that the step's last stage fills.  The stages then
-// read the published dt instead of every wave reducing the sub-slots.
-__global__ __launch_bounds__(128) void drop_dt_kernel(unsigned long long lo, unsigned long long hi, double *dt_cur)
-{
-    const int i = threadIdx.x;
-    if ((i < 64 ? lo >> i : hi >> (i - 64)) & 1) dt_cur[i] = 0.0;
-}
-
-__global__ __launch_bounds__(64) void dt_prep_kernel(MeshDev m, int use_cfl, double *dt_cur, double *t_inst,
-                                                     double *t_step, unsigned long long *slot)
+// read the published dt instead of every wave reducing the sub-slots.  An
+// instance without quadrants (has) does not advance.
+__global__ __launch_bounds__(64) void dt_prep_kernel(MeshDev m, const int *has, int use_cfl, double *dt_cur,
+                                                     double *t_inst, double *t_step, unsigned long long *slot)
 {
     const int i = blockIdx.x;
     if (i >= m.ninst) return;
-    const double dt = step_dt(m.ip[i], slot, t_inst, i, use_cfl);
+    const double limit = step_dt(m.ip[i], slot, t_inst, i, use_cfl);
+    const double dt = has[i] ? limit : 0.0;
     if (threadIdx.x == 0) {
         dt_cur[i] = dt;
         t_step[i] = t_inst[i];
@@ -2654,10 +2656,11 @@ struct amrgpu_ctx {
     hipStream_t stream = nullptr;
     // one allocation: instances, clocks, CFL sub-slots, norm partials and
     // indicator by capacity (ensure_capacity), then the mesh packed by its own
-    // size (place_mesh): corners, face table, levels, instance ids, source map
+    // size (place_mesh): corners, face table, levels, instance ids, source map, which
+    // instances have quadrants
     char *d_block = nullptr;
     size_t mesh_off = 0;
-    int *d_nbr = nullptr, *d_level = nullptr, *d_inst = nullptr;
+    int *d_nbr = nullptr, *d_level = nullptr, *d_inst = nullptr, *d_has = nullptr;
     InstDev *d_ip = nullptr;
     double *U[3] = {nullptr, nullptr, nullptr};
     double *Acc = nullptr;
@@ -2669,7 +2672,8 @@ struct amrgpu_ctx {
     int tb = 0, sb = 0;
     bool sweep_down = false;                   // direction of the next stage launch
     bool self_dt = false;                      // this run's steps have no dt_prep_kernel
-    bool empty_known = true;                   // `empty` has every instance without quadrants
+    bool any_empty = false;                    // some instance has no quadrants
+    bool empty_known = true;                   // `empty` has all of these
     unsigned long long empty[2] = {0, 0};
     double *t_now(int ahead = 0) const { return d_clock + (size_t)((tb + ahead) & 1) * cap_inst; }
     double *dt_cur() const { return d_clock + (size_t)2 * cap_inst; }
@@ -3071,7 +3075,7 @@ int begin_step(amrgpu_ctx *c, std::vector<StageArgs> &st)
 {
     if (!c->self_dt) {
         hipLaunchKernelGGL(dt_prep_kernel, dim3(std::max(1, c->ninst)), dim3(64), 0, c->stream, mesh_of(c),
-                           c->scheme != 2, c->dt_cur(), c->t_now(), c->t_step(), c->slots());
+                           c->d_has, c->scheme != 2, c->dt_cur(), c->t_now(), c->t_step(), c->slots());
         HIPCHK(hipGetLastError());
         return AMRGPU_OK;
     }
@@ -3117,7 +3121,7 @@ void free_mesh(amrgpu_ctx *c)
     c->d_block = nullptr;
     c->d_map = nullptr; c->d_ind = nullptr; c->d_org = nullptr;
     c->org_ok = false;
-    c->d_nbr = c->d_level = c->d_inst = nullptr; c->d_ip = nullptr;
+    c->d_nbr = c->d_level = c->d_inst = c->d_has = nullptr; c->d_ip = nullptr;
     c->U[0] = c->U[1] = c->U[2] = nullptr; c->Acc = nullptr;
     c->d_clock = nullptr; c->d_slot_sets = nullptr; c->d_norm = nullptr;
     c->d_stage = nullptr;
@@ -3126,13 +3130,14 @@ void free_mesh(amrgpu_ctx *c)
     c->cap_state = 0;
 }
 
-// The packed mesh's arrays in a block that starts at `base`, for ncell quadrants:
-// corners, face table, levels, instance ids, source map.
+// The packed mesh's arrays in a block that starts at `base`, for ncell quadrants of
+// ninst instances: corners, face table, levels, instance ids, source map, which
+// instances have quadrants.
 struct MeshPlace {
     double *org;
-    int *nbr, *level, *inst, *map, *end;
+    int *nbr, *level, *inst, *map, *has, *end;
 };
-MeshPlace place_mesh(char *base, int ncell)
+MeshPlace place_mesh(char *base, int ncell, int ninst)
 {
     MeshPlace m;
     m.org = (double *)base;
@@ -3140,10 +3145,14 @@ MeshPlace place_mesh(char *base, int ncell)
     m.level = m.nbr + 8 * (size_t)ncell;
     m.inst = m.level + ncell;
     m.map = m.inst + ncell;
-    m.end = m.map + ncell;
+    m.has = m.map + ncell;
+    m.end = m.has + ninst;
     return m;
 }
-constexpr size_t MESH_BYTES = 2 * sizeof(double) + 11 * sizeof(int);     // per quadrant
+size_t mesh_bytes(size_t ncell, size_t ninst)
+{
+    return ncell * (2 * sizeof(double) + 11 * sizeof(int)) + ninst * sizeof(int);
+}
 
 // Wait for the stream; the borrowed pinned memory goes back.
 int sync_stream(amrgpu_ctx *c)
@@ -3432,7 +3441,7 @@ static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need
     const size_t ip = part(sizeof(InstDev) * c->cap_inst), clock = part(sizeof(double) * 4 * c->cap_inst);
     const size_t slot = part(sizeof(unsigned long long) * 3 * c->cap_inst * NSLOT);
     const size_t norm = part(sizeof(double) * c->cap_blocks), ind = part(sizeof(double) * cq);
-    c->mesh_off = part(MESH_BYTES * cq);
+    c->mesh_off = part(mesh_bytes(cq, c->cap_inst));
     if (hipMalloc((void **)&c->d_block, at) != hipSuccess) {
         free_mesh(c);
         set_err("%s:%d device allocation of %zu bytes failed", __FILE__, __LINE__, at);
@@ -3447,26 +3456,23 @@ static int ensure_capacity(amrgpu_ctx *c, int n, int ncell, int ninst, bool need
 }
 
 // The device mesh is a new one of ncell quadrants with these instance ids (null:
-// all 0): its arrays' places, the tile and what hangs on them.
-static int new_mesh(amrgpu_ctx *c, int ncell, const int *cell_inst)
+// all 0): its arrays' places, the tile and what hangs on them.  has: which
+// instances have quadrants, for the packed mesh.
+static int new_mesh(amrgpu_ctx *c, int ncell, const int *cell_inst, int *has)
 {
-    const MeshPlace m = place_mesh(c->d_block + c->mesh_off, ncell);
-    c->d_org = m.org; c->d_nbr = m.nbr; c->d_level = m.level; c->d_inst = m.inst; c->d_map = m.map;
+    const MeshPlace m = place_mesh(c->d_block + c->mesh_off, ncell, c->ninst);
+    c->d_org = m.org; c->d_nbr = m.nbr; c->d_level = m.level; c->d_inst = m.inst; c->d_has = m.has; c->d_map = m.map;
     c->nquad = ncell;
+    std::fill(has, has + c->ninst, 0);
+    has[0] = !cell_inst;
+    if (cell_inst)
+        for (int q = 0; q < ncell; ++q) has[cell_inst[q]] = 1;
+    c->any_empty = std::find(has, has + c->ninst, 0) != has + c->ninst;
+    c->empty_known = !c->any_empty || c->ninst <= 128;
     c->empty[0] = c->empty[1] = 0;
-    c->empty_known = c->ninst <= 128;
-    if (c->ninst > 1) {
-        std::vector<char> has(c->ninst, 0);
-        has[0] = !cell_inst;
-        if (cell_inst)
-            for (int q = 0; q < ncell; ++q) has[cell_inst[q]] = 1;
-        if (c->empty_known) {
-            for (int i = 0; i < c->ninst; ++i)
-                if (!has[i]) c->empty[i / 64] |= 1ull << i % 64;
-        } else {
-            c->empty_known = std::find(has.begin(), has.end(), 0) == has.end();
-        }
-    }
+    if (c->any_empty && c->empty_known)
+        for (int i = 0; i < c->ninst; ++i)
+            if (!has[i]) c->empty[i / 64] |= 1ull << i % 64;
     if (!c->tile_chosen || kVariants[c->variant].n != c->n) {
         c->variant = default_variant(c->n, ncell);
         c->tile_chosen = false;
@@ -3550,9 +3556,9 @@ int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int nin
     int rc = validate_cells(n2, ninst, ncell, cell_info, cell_inst, "amrgpu_setup");
     if (rc) return rc;
     // the mesh, packed as it lies on the device, is built in the pinned area
-    rc = take_up(c, MESH_BYTES * (size_t)ncell + (sizeof(InstDev) + 4 * sizeof(double)) * ninst);
+    rc = take_up(c, mesh_bytes(ncell, ninst) + (sizeof(InstDev) + 4 * sizeof(double)) * ninst);
     if (rc) return rc;
-    const MeshPlace h = place_mesh((char *)c->up.p, ncell);
+    const MeshPlace h = place_mesh((char *)c->up.p, ncell, ninst);
     if (face_info) {
         rc = build_nbr(ncell, nface, face_info, h.nbr);
         if (rc) return rc;
@@ -3596,10 +3602,10 @@ int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int nin
         d.ninv_vol0 = -1.0 / v0;
         d.cfl_h0 = inst[i].cfl * sqrt(v0);
     }
-    rc = new_mesh(c, ncell, cell_inst);
+    rc = new_mesh(c, ncell, cell_inst, h.has);
     if (rc) return rc;
     c->org_ok = geom != nullptr;
-    HIPCHK(hipMemcpyAsync(c->d_org, h.org, (size_t)((char *)h.map - (char *)h.org), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->d_org, h.org, (size_t)((char *)h.end - (char *)h.org), hipMemcpyHostToDevice, c->stream));
     // instances and clocks after the mesh in the pinned area
     InstDev *const hip = (InstDev *)h.end;
     memcpy(hip, c->h_ip.data(), sizeof(InstDev) * ninst);
@@ -3704,7 +3710,7 @@ static void put_table(const NewMesh &m, const MeshPlace &h)
 constexpr int REMAP_FIRST = 32768;
 static int remesh_to(amrgpu_ctx *c, const NewMesh &m, const MeshPlace &h, const int *src)
 {
-    const int ncell = m.ncell, *const cell_inst = m.inst;
+    const int ncell = m.ncell;
     const int n2 = c->n * c->n, nold = c->nquad;
     const bool first = ncell >= REMAP_FIRST;
     int rc = AMRGPU_OK;
@@ -3743,7 +3749,7 @@ static int remesh_to(amrgpu_ctx *c, const NewMesh &m, const MeshPlace &h, const 
         from = keep;
         to = 0;
     }
-    rc = new_mesh(c, ncell, cell_inst);
+    rc = new_mesh(c, ncell, m.inst, h.has);
     if (rc) { (void)hipFree(keep); return rc; }
     int *const part = first ? h.map : h.nbr;
     HIPCHK(hipMemcpyAsync(first ? c->d_map : c->d_nbr, part, (size_t)((char *)h.end - (char *)part), hipMemcpyHostToDevice,
@@ -3759,30 +3765,12 @@ static int remesh_to(amrgpu_ctx *c, const NewMesh &m, const MeshPlace &h, const 
     if ((rc = sync_stream(c))) return rc;
     (void)hipFree(keep);
     // an instance left without quadrants (a batch drops those that reached
-    // their stop) no longer advances: no wave publishes its dt any more, so
-    // its last dt is cleared here and the time bookkeeping of the stages
-    // keeps its time as it is
-    if (c->ninst <= 128) {
-        if (cell_inst && (c->empty[0] | c->empty[1])) {
-            hipLaunchKernelGGL(drop_dt_kernel, dim3(1), dim3(128), 0, c->stream, c->empty[0], c->empty[1], c->dt_cur());
-            HIPCHK(hipGetLastError());
-        }
-    } else if (cell_inst) {
-        std::vector<char> has(c->ninst, 0);
-        for (int q = 0; q < ncell; ++q) has[cell_inst[q]] = 1;
-        bool empty = false;
-        for (int i = 0; i < c->ninst; ++i) empty = empty || !has[i];
-        if (empty) {
-            std::vector<double> dt(c->ninst);
-            HIPCHK(hipMemcpyAsync(dt.data(), c->dt_cur(), sizeof(double) * c->ninst, hipMemcpyDeviceToHost,
-                                  c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
-            for (int i = 0; i < c->ninst; ++i)
-                if (!has[i]) dt[i] = 0.0;
-            HIPCHK(hipMemcpyAsync(c->dt_cur(), dt.data(), sizeof(double) * c->ninst, hipMemcpyHostToDevice,
-                                  c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
-        }
+    // their stop) no longer advances: its last dt is cleared here, and the steps
+    // keep its time as it is
+    if (c->any_empty) {
+        hipLaunchKernelGGL(drop_dt_kernel, dim3((c->ninst + 255) / 256), dim3(256), 0, c->stream, c->d_has, c->ninst,
+                           c->dt_cur());
+        HIPCHK(hipGetLastError());
     }
     return AMRGPU_OK;
 }
@@ -3797,9 +3785,9 @@ int amrgpu_remesh(amrgpu_ctx *c, int ncell, const int *cell_info, const int *cel
     int rc = check_src(ncell, src, c->nquad, "amrgpu_remesh");
     if (!rc) rc = validate_cells(c->n * c->n, c->ninst, ncell, cell_info, cell_inst, "amrgpu_remesh");
     if (rc) return rc;
-    rc = take_up(c, MESH_BYTES * (size_t)ncell);
+    rc = take_up(c, mesh_bytes(ncell, c->ninst));
     if (rc) return rc;
-    const MeshPlace h = place_mesh((char *)c->up.p, ncell);
+    const MeshPlace h = place_mesh((char *)c->up.p, ncell, c->ninst);
     rc = build_nbr(ncell, nface, face_info, h.nbr);
     if (rc) return rc;                 // a refused call leaves the context as it was
     c->org_ok = false;                 // the new quadrants' coordinates come with amrgpu_set_geometry
@@ -3833,9 +3821,9 @@ int amrgpu_remesh_nbr(amrgpu_ctx *c, int ncell, const int *level, const int *cel
             }
         }
     }
-    rc = take_up(c, MESH_BYTES * (size_t)ncell);
+    rc = take_up(c, mesh_bytes(ncell, c->ninst));
     if (rc) return rc;
-    const MeshPlace h = place_mesh((char *)c->up.p, ncell);
+    const MeshPlace h = place_mesh((char *)c->up.p, ncell, c->ninst);
     c->org_ok = false;                 // the new quadrants' coordinates come with amrgpu_set_origins
     return remesh_to(c, {ncell, nbr, level, 1, cell_inst}, h, src);
 }

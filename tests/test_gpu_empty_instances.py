@@ -59,3 +59,40 @@ def test_leave_and_come_back(n, own, other, ninst, scheme):
     run(4)
     for g in gs:
         g.close()
+
+
+@pytest.mark.parametrize("scheme", [2, 3])
+@pytest.mark.parametrize("ninst", [3, 129])
+@pytest.mark.parametrize("n,tile", [(4, (4, 3, 3)), (4, (8, 1, 1)), (8, (1, 5, 1)), (8, (2, 4, 1)), (16, (1, 5, 1)), (16, (1, 4, 0))])
+def test_time_of_an_absent_instance_stays(n, tile, ninst, scheme):
+    """an instance without quadrants does not advance: no last dt, and its time
+    where it was, from a remesh or from the setup on, until it comes back"""
+    forest = small_forest(n, 7, True, 1, 2)
+    nq = forest.nquad
+    live = [0, ninst - 1]
+    insts = [amrhip.make_inst(1.0, (0,) * 4, 0.2, 1e-3) for _ in range(ninst)]
+    ci, fi, geom, soln, inst = amrhip.batch_external([forest] * 2)
+    inst = np.asarray(live, np.int32)[np.asarray(inst)]
+    g = amrhip.Gpu()
+    g.setup(n, scheme, insts, ci, fi, geom, soln, inst)
+    g.set_tile(*tile)
+    t0 = 0.25 * np.arange(ninst)
+    g.set_time(t0)
+    g.run(2)
+    t, dt = g.time()
+    absent = np.ones(ninst, bool)
+    absent[live] = False
+    assert np.array_equal(t[absent], t0[absent]) and not dt[absent].any()
+    assert (t[live] > t0[live]).all() and (dt[live] > 0.0).all()
+    one = amrhip.batch_external([forest])
+    g.remesh(one[0], one[1], np.arange(nq, dtype=np.int32), np.zeros(nq, np.int32))
+    assert g.time()[1][-1] == 0.0
+    g.run(3)
+    t1, dt1 = g.time()
+    assert np.array_equal(t1[1:], t[1:]) and not dt1[1:].any() and t1[0] > t[0]
+    g.remesh(ci, fi, np.tile(np.arange(nq, dtype=np.int32), 2), inst)
+    g.run(1)
+    t2, dt2 = g.time()
+    assert np.array_equal(t2[absent], t0[absent]) and not dt2[absent].any()
+    assert t2[-1] == t[-1] + dt2[-1] and dt2[-1] > 0.0
+    g.close()
