@@ -3556,7 +3556,7 @@ int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int nin
     int rc = validate_cells(n2, ninst, ncell, cell_info, cell_inst, "amrgpu_setup");
     if (rc) return rc;
     // the mesh, packed as it lies on the device, is built in the pinned area
-    rc = take_up(c, mesh_bytes(ncell, ninst) + (sizeof(InstDev) + 4 * sizeof(double)) * ninst);
+    rc = take_up(c, mesh_bytes(ncell, ninst) + sizeof(InstDev) * ninst);
     if (rc) return rc;
     const MeshPlace h = place_mesh((char *)c->up.p, ncell, ninst);
     if (face_info) {
@@ -3606,8 +3606,8 @@ int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int nin
     if (rc) return rc;
     c->org_ok = geom != nullptr;
     HIPCHK(hipMemcpyAsync(c->d_org, h.org, (size_t)((char *)h.end - (char *)h.org), hipMemcpyHostToDevice, c->stream));
-    // instances and clocks after the mesh in the pinned area
-    InstDev *const hip = (InstDev *)h.end;
+    // the instances after the mesh in the pinned area (bytes: it may end at any int)
+    char *const hip = (char *)h.end;
     memcpy(hip, c->h_ip.data(), sizeof(InstDev) * ninst);
     HIPCHK(hipMemcpyAsync(c->d_ip, hip, sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
     if ((rc = set_clocks(c, t_inst))) return rc;
