@@ -2775,15 +2775,15 @@ int grid_of(const amrgpu_ctx *c, int v, int nquad)
 // 522 and 526).
 // n = 2 and 4: the row-marching kernel, faster than the others at every size
 // measured (16 to 262k quadrants).  n = 4 takes four rows a step, with twice the
-// waves, while these are on the chip together (256 CUs x 12 waves x 4 patches =
-// 12288 quadrants), else two, with fewer instructions a patch: us per SSP-RK3 step
+// waves, while these are on the chip together (12 waves x 4 patches a CU: 12288
+// quadrants on 256 CUs), else two, with fewer instructions a patch: us per SSP-RK3 step
 // with two / four, 4k quadrants 18.7 / 16.9, 12k 24.2 / 23.6 (adaptive 29.4 / 26.0),
 // 16k 25.8 / 29.5, 21k (adaptive) 25.7 / 27.1, 66k 77.9 / 87.1.
-int default_variant(int n, int nquad)
+int default_variant(const amrgpu_ctx *c, int nquad)
 {
-    switch (n) {
+    switch (c->n) {
     case 2: return 20;
-    case 4: return nquad <= 12288 ? 21 : 22;
+    case 4: return nquad <= c->cu_count * 12 * 4 ? 21 : 22;
     case 8: return 17;
     case 16: return 19;
     default: return -1;
@@ -3474,7 +3474,7 @@ static int new_mesh(amrgpu_ctx *c, int ncell, const int *cell_inst, int *has)
         for (int i = 0; i < c->ninst; ++i)
             if (!has[i]) c->empty[i / 64] |= 1ull << i % 64;
     if (!c->tile_chosen || kVariants[c->variant].n != c->n) {
-        c->variant = default_variant(c->n, ncell);
+        c->variant = default_variant(c, ncell);
         c->tile_chosen = false;
     }
     c->nblocks = grid_of(c, c->variant, ncell);

@@ -725,6 +725,7 @@ struct amr_mlp {
     size_t cap_logits = 0;
     long long step = 0;
     float refine_bias = 0.0f;
+    int cu_count = 256;         // compute units of the device
 };
 
 struct amr_tagset {
@@ -743,7 +744,7 @@ Weights weights_of(const amr_mlp *m) { return Weights{m->W1b, m->W2b, m->W3b, m-
 int launch_infer(amr_mlp *m, const uint16_t *dX, int count, float *dlogits, int *dcls, hipStream_t st)
 {
     if (count <= 0) return AMRGPU_OK;
-    const int grid = std::min((count + 16 * IWAVES - 1) / (16 * IWAVES), 512);     // two workgroups on each of 256 CUs
+    const int grid = std::min((count + 16 * IWAVES - 1) / (16 * IWAVES), 2 * m->cu_count);     // two workgroups a CU
     hipLaunchKernelGGL(infer_kernel, dim3(grid), dim3(64 * IWAVES), 0, st, weights_of(m), dX, count, m->refine_bias,
                        dlogits, dcls);
     MCHK(hipGetLastError());
@@ -797,6 +798,10 @@ extern "C" {
 amr_mlp_t *amr_mlp_create(unsigned long long seed)
 {
     amr_mlp *m = new amr_mlp();
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu > 0)
+        m->cu_count = ncu;
     std::vector<float> P(NP, 0.0f);
     uint64_t s = seed * 0x2545F4914F6CDD1Dull + 1;
     const double a1 = std::sqrt(6.0 / NIN), a2 = std::sqrt(6.0 / NH);

@@ -22,9 +22,11 @@ RUNTIME = r"""
 #include <stdlib.h>
 #include <string.h>
 #include "amr_hip.h"
+#include "amr_tagger.h"
 
 /* what the library asked for */
-static int host_allocs, copies, launches, copies_at_launch;
+static int host_allocs, copies, launches, copies_at_launch, cus = 256;
+static dim3 grid;
 static const void *copy_src[1024];
 static void *copy_dst[1024];
 static size_t copy_bytes[1024];
@@ -36,6 +38,8 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; ++ho
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n); return hipSuccess; }
 hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMemset(void *p, int v, size_t n) { memset(p, v, n); return hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
 {
     (void)k; (void)st;
@@ -59,7 +63,7 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t e) { (void)e; return "error"; }
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
-hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = 256; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = cus; return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { (void)f; *s = (hipStream_t)&copies; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { (void)s; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
@@ -67,7 +71,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { (void)f; *e = (h
 hipError_t hipEventDestroy(hipEvent_t e) { (void)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { (void)e; (void)s; return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t e) { (void)e; return hipSuccess; }
-hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t n, hipStream_t s) { (void)g; (void)b; (void)n; (void)s; return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t n, hipStream_t s) { (void)b; (void)n; (void)s; grid = g; return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *n, hipStream_t *s)
 {
     memset(g, 0, sizeof(*g)); memset(b, 0, sizeof(*b)); *n = 0; *s = 0;
@@ -299,4 +303,39 @@ def test_every_tile_launches_every_stage(tmp_path, n):
             HOLDS(step2 == 2 * scheme || step2 == 2 * (scheme + 1));
             amrgpu_destroy(c);
         }}
+""")
+
+
+@pytest.mark.parametrize("cus", [32, 256, 304])
+def test_limits_follow_the_devices_compute_units(tmp_path, cus):
+    """4x4 patches take four rows a step while their waves fit the device, 12 of
+    4 patches a CU, and the tagger's inference two workgroups a CU at most"""
+    run(tmp_path, f"""
+    enum {{ most = {cus} * 48 + 1, n = 4 }};
+    static int ci[3 * most], fi[44 * most];
+    cus = {cus};
+    amrgpu_inst_t in;
+    memset(&in, 0, sizeof(in));
+    in.h_base = 1.0; in.cfl = 0.3; in.dt_cap = 1.0;
+    for (int q = 0; q < most; ++q) {{
+        ci[3 * q + 2] = 4 * n * n * q;
+        for (int s = 0; s < 4; ++s) {{ int *f = fi + 11 * (4 * q + s); f[0] = 1; f[1] = s; f[2] = q; }}
+    }}
+    amrgpu_ctx *c = amrgpu_create();
+    for (int nq = most - 1; nq <= most; ++nq) {{
+        int ppb, minw, design;
+        MUST(amrgpu_setup(c, n, 3, 1, &in, nq, ci, NULL, 4 * nq, fi, NULL, NULL));
+        MUST(amrgpu_get_tile(c, &ppb, &minw, &design));
+        HOLDS(design == 3 && ppb == (nq < most ? 4 : 8));
+    }}
+    amrgpu_destroy(c);
+    enum {{ rows = 2 * {cus} * 128 }};
+    amr_mlp_t *m = amr_mlp_create(1);
+    unsigned short *X = calloc((rows + 1) * (size_t)AMR_MLP_NIN, 2);
+    float *z = calloc((rows + 1) * 3ul, sizeof(float));
+    MUST(amr_mlp_forward(m, X, rows - 128, z));
+    HOLDS(grid.x == 2 * {cus} - 1);
+    MUST(amr_mlp_forward(m, X, rows + 1, z));
+    HOLDS(grid.x == 2 * {cus});
+    amr_mlp_destroy(m);
 """)
