@@ -191,6 +191,23 @@ def time_steps(amrhip, n, insts, arrays, steps, warmup, tile=None, autotune=True
     return g, tune, ms, stage_ms
 
 
+DESIGNS = ("face task list", "paired faces", "persistent prefetch", "several patches a wave, row by row")
+
+
+def kernel_name(n, tile):
+    """the stage kernel of a tile (patches per workgroup, minimum waves per
+    SIMD, design), as a profiler names it, with the template arguments that
+    the tile sets"""
+    ppb, minw, design = tile
+    if design == 2:
+        return f"stage_kernel_pp<{n}, {minw}>"
+    if design == 3:
+        return f"stage_kernel_rows<{n}, {64 // (n * ppb)}, ...>"
+    if design == 1 and ppb == 1 and n == 8:
+        return f"stage_kernel_one<{minw}, ...>"
+    return f"stage_kernel<{n}, {ppb}, {minw}, {design}, ...>"
+
+
 def roofline_of(cells, ms, steps, n, tile, launch, stage_ms):
     avg_stage = ms / (3 * steps)
     bytes_launch = cells * B_ALG_STAGE
@@ -202,11 +219,11 @@ def roofline_of(cells, ms, steps, n, tile, launch, stage_ms):
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4),
         "traffic": None,
-        "kernel": f"stage_kernel<{n},{tile[0]},{tile[1]},{tile[2]}>",
+        "kernel": kernel_name(n, tile),
         "bytes_per_launch": int(bytes_launch),
         "avg_launch_us": round(avg_stage * 1e3, 3),
-        "avg_launch_from": f"timed region / stage launches, 3 per step, the step's dt prep launch counted in "
-                           f"the time (HIP events on the launch stream, {launch})",
+        "avg_launch_from": f"timed region / stage launches, 3 per step, the launch that forms the step's dt (where "
+                           f"the first stage does not) counted in the time (HIP events on the launch stream, {launch})",
         "stage_launch_us_bracketed": [round(s * 1e3, 3) for s in stage_ms],
     }
 
@@ -680,7 +697,7 @@ def main():
             "quads": nq, "cells": cells, "patch": n,
             "levels": [int(lv.min()), int(lv.max())], "parallelism": "1 GPU, every instance in one launch",
             "tile": {"patches_per_workgroup": tile[0], "min_waves_per_simd": tile[1],
-                     "design": ["face task list", "paired faces", "persistent prefetch"][tile[2]],
+                     "design": DESIGNS[tile[2]],
                      "autotuned": tune is not None, "launch": launch},
         },
         "roofline": roof,
