@@ -31,7 +31,8 @@ U^s+1; 32 B per state), achieved = bytes per launch / average launch
 duration = the timed region / launches.  traffic = FETCH_SIZE (scaled by the
 copy kernel's reading of a known size) + WRITE_SIZE per launch from the
 committed rocprofv3 summary of the same mesh
-(profiles/stage_kernel_<workload>_traffic.txt), when its cell count matches.
+(profiles/stage_kernel_<workload>_traffic.txt), when its kernel and cell count
+match.
 
 cpu_baseline: the C oracle (restatement of the reference CPU path: AoS
 patches, face loop + element loop, k-form SSP-RK3) on the host, one worker per
@@ -228,11 +229,12 @@ def roofline_of(cells, ms, steps, n, tile, launch, stage_ms):
     }
 
 
-def measured_traffic(workload, cells):
+def measured_traffic(workload, cells, kernel):
     """HBM bytes per stage-kernel launch from the committed rocprofv3 --pmc
     summary of this workload (FETCH_SIZE and WRITE_SIZE per dispatch, scaled
-    by the copy kernel's reading of a known size), when it was taken on the
-    same mesh size; None otherwise (the summary names the tile it used)"""
+    by the copy kernel's reading of a known size), when it was taken of the
+    same kernel on the same mesh size; None otherwise (the summary names the
+    tile it used: the minimum waves of a tile do not change what it moves)"""
     path = os.path.join(ROOT, "profiles", f"stage_kernel_{workload}_traffic.txt")
     if not os.path.exists(path):
         return None
@@ -242,7 +244,7 @@ def measured_traffic(workload, cells):
             k, v = line.split(":", 1)
             kv[k.strip()] = v.strip()
     try:
-        if int(kv["cells"]) != cells:
+        if int(kv["cells"]) != cells or kv["kernel"].split("<")[0] != kernel.split("<")[0]:
             return None
         return int(float(kv["hbm_bytes_per_launch"])), kv.get("tile", "")
     except (KeyError, ValueError):
@@ -675,7 +677,7 @@ def main():
         probe = None
     roof = roofline_of(cells, ms, args.steps, n, tile, launch, stage_ms)
     roof["copy_probe_GBs"] = round(probe, 1) if probe else None
-    traffic = measured_traffic(wl_key, cells)
+    traffic = measured_traffic(wl_key, cells, roof["kernel"])
     if traffic is not None:
         roof["traffic"] = traffic[0]
         roof["traffic_tile"] = traffic[1]
