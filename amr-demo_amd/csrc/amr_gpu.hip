@@ -2871,7 +2871,9 @@ int launch_v(amrgpu_ctx *c, const StageArgs &a)
                 if constexpr (SELF && !forms_dt(PPB, MINW, D))
                     return;        // (not compiled; launch_stage refuses it)
                 else if constexpr (N == 8)
-                    hipLaunchKernelGGL((stage_kernel_one<MINW, SELF, NT, VEC>), nblk, blk, 0, c->stream, a);
+                    // (one compilation for the three tiles: left to 1 or 4 waves a SIMD the
+                    // kernel has 92-96 registers and runs at five all the same)
+                    hipLaunchKernelGGL((stage_kernel_one<5, SELF, NT, VEC>), nblk, blk, 0, c->stream, a);
                 else
                     hipLaunchKernelGGL((stage_kernel<N, PPB, MINW, D, SELF, NT, VEC>), nblk, blk, 0, c->stream, a);
             });

@@ -205,7 +205,7 @@ def kernel_name(n, tile):
     if design == 3:
         return f"stage_kernel_rows<{n}, {64 // (n * ppb)}, ...>"
     if design == 1 and ppb == 1 and n == 8:
-        return f"stage_kernel_one<{minw}, ...>"
+        return "stage_kernel_one<5, ...>"       # every such tile's
     return f"stage_kernel<{n}, {ppb}, {minw}, {design}, ...>"
 
 
