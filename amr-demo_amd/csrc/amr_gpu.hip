@@ -1634,27 +1634,7 @@ __global__ __launch_bounds__(N * N, MINW) void stage_kernel_pp(StageArgs a)
     if (a.norm_part) sum_reduce_store<N2>(sq, &a.norm_part[lb], red);
 }
 
-// ---------------------------------------------------------------------------
-// Row-marching stage kernel (DESIGN 3): one wave, its own workgroup, advances
-// P = 64 / (N R) patches together.  The lanes are P patches x R rows x N columns;
-// the wave walks the patches' rows R at a time (N / R steps), every lane
-// evaluating its cell's +x and +y faces from its record in registers and its
-// two neighbours' in LDS.  The faces left over, the -x and -y edges of the P
-// patches, are one round ahead of the march (all 64 lanes busy with R = 2, half
-// of them with R = 4).  The arithmetic of a face is stage_kernel's, operation
-// for operation: the results are bit for bit those of the other designs.
-//
-// What bounds the small patches is the instruction stream: of a 4x4 patch's 40
-// faces 8 are left over, of a 2x2 patch's 12 faces 4, and stage_kernel spends a
-// round with few lanes busy on them (or, DESIGN 0, three rounds for 2.5), decodes
-// a task list per workgroup and passes two workgroup barriers.  Here 8 4x4
-// patches take 2 + 2 + 1 full rounds, every index is a shift of the lane id, and
-// one wave needs no barrier (its LDS operations execute in order).  LDS holds
-// the rows in flight and the halo only, 9 KB (R = 4) or 14 KB (R = 2) a wave.
-// Measured, us per SSP-RK3 step, DESIGN 0 -> this: 2x2 patches 262k quadrants
-// 237 -> 99.6, 16k 26.6 -> 18.4; 4x4 patches 176k quadrants (adaptive) 391 -> 220,
-// 21k 42.4 -> 25.8, 256 21.8 -> 16.0.
-// ---------------------------------------------------------------------------
+// The record of a tile position (Tile) in registers.
 struct Rec {
     double r, ru, rv, rE, p, ir, sr;
 };
@@ -1916,7 +1896,30 @@ __global__ __launch_bounds__(64, MINW) void stage_kernel_one(StageArgs a)
     }
 }
 
+// ---------------------------------------------------------------------------
+// Row-marching stage kernel (DESIGN 3): one wave, its own workgroup, advances
+// P = 64 / (N R) patches together.  The lanes are P patches x R rows x N columns;
+// the wave walks the patches' rows R at a time (N / R steps), every lane
+// evaluating its cell's +x and +y faces from its record in registers and its
+// two neighbours' in LDS.  The faces left over, the -x and -y edges of the P
+// patches, are one round ahead of the march (all 64 lanes busy with R = 2, half
+// of them with R = 4).  The arithmetic of a face is stage_kernel's, operation
+// for operation: the results are bit for bit those of the other designs.
+//
+// What bounds the small patches is the instruction stream: of a 4x4 patch's 40
+// faces 8 are left over, of a 2x2 patch's 12 faces 4, and stage_kernel spends a
+// round with few lanes busy on them (or, DESIGN 0, three rounds for 2.5), decodes
+// a task list per workgroup and passes two workgroup barriers.  Here 8 4x4
+// patches take 2 + 2 + 1 full rounds, every index is a shift of the lane id, and
+// one wave needs no barrier (its LDS operations execute in order).  LDS holds
+// the rows in flight and the halo only, 9 KB (R = 4) or 14 KB (R = 2) a wave.
+// Measured, us per SSP-RK3 step (median of 15 runs), DESIGN 0 -> this: 2x2 patches
+// 262k quadrants 234 -> 103, 16k 27.9 -> 17.7; 4x4 patches 176k quadrants (adaptive)
+// 378 -> 228, 16k 46.9 -> 26.0, 7.5k (adaptive) 32.8 -> 21.4, 256 23.9 -> 14.3.  A
+// step of so few waves is bound by its launches, which run at one of two speeds, by
+// process: 22.2 -> 12.4 the other.
 // SELF: the first stage of a step without dt_prep_kernel.
+// ---------------------------------------------------------------------------
 template <int N, int R, int VEC, bool SELF, bool NT>
 __global__ __launch_bounds__(64, 3) void stage_kernel_rows(StageArgs a)
 {
@@ -2562,10 +2565,6 @@ void set_err(const char *fmt, ...)
         }                                                                           \
     } while (0)
 
-struct StageLaunch {
-    StageArgs a;
-};
-
 }  // namespace
 
 extern "C" void amr_set_error(const char *fmt, ...)
@@ -2770,15 +2769,14 @@ int grid_of(const amrgpu_ctx *c, int v, int nquad)
 // Stage-kernel tile used until amrgpu_set_tile / amrgpu_autotune picks one
 // (every tile computes the same bits): for n = 8 and 16 the tile with one patch
 // per workgroup and five waves per SIMD, the fastest or within 2 % of it on the
-// meshes measured (1k to 16.8M cells; four and five waves at 8x8: 2.6k quadrants
-// 21.4 and 21.4 us a step, 18.8k 85.9 and 84.0, 159k 672 and 664, 131k uniform
-// 522 and 526).
+// meshes measured (1k to 16.8M cells).
 // n = 2 and 4: the row-marching kernel, faster than the others at every size
 // measured (16 to 262k quadrants).  n = 4 takes four rows a step, with twice the
 // waves, while these are on the chip together (12 waves x 4 patches a CU: 12288
-// quadrants on 256 CUs), else two, with fewer instructions a patch: us per SSP-RK3 step
-// with two / four, 4k quadrants 18.7 / 16.9, 12k 24.2 / 23.6 (adaptive 29.4 / 26.0),
-// 16k 25.8 / 29.5, 21k (adaptive) 25.7 / 27.1, 66k 77.9 / 87.1.
+// quadrants on 256 CUs), else two, with fewer instructions a patch: us per SSP-RK3
+// step with two / four (median of 15 runs), 256 quadrants 17.1 / 14.3, 4k 18.3 / 16.1,
+// 7.5k (adaptive) 23.4 / 21.4, 12.9k (adaptive) 29.6 / 28.5, 16k 26.0 / 29.1, 66k
+// 75.8 / 84.7.
 int default_variant(const amrgpu_ctx *c, int nquad)
 {
     switch (c->n) {
@@ -3055,16 +3053,18 @@ int build_step(amrgpu_ctx *c, int cur, std::vector<StageArgs> &st, bool with_nor
 }
 
 // Whether the steps of a run have no dt_prep_kernel.  That saves a launch and its
-// gap, 1.6-2 us a step; every first-stage wave reduces its instance's sub-slots
+// gap, 2 to 4 us a step; every first-stage wave reduces its instance's sub-slots
 // instead (four loads a lane beside the halo's), so meshes of many waves keep the
-// kernel.  us per SSP-RK3 step with / without it, one problem each: 8x8, 256
-// quadrants 15.3 / 13.6, 4137 30.1 / 28.9, 18750 93.7 / 90.2, 41170 180.5 / 182.8;
-// 16x16, 256 17.4 / 15.7, 4455 83.3 / 83.1, 7159 122.6 / 125.9; the row-marching
-// tiles, whose waves hold several patches: 4x4, 1024 14.0 / 12.2, 16384 30.5 /
-// 29.1, 65536 84.8 / 85.8; 2x2, 37750 35.5 / 34.6, 65536 36.1 / 36.9.
+// kernel.  us per SSP-RK3 step with / without it, one problem each (median of 15
+// runs): 8x8, 256 quadrants 18.0 / 14.2, 2638 (adaptive) 24.1 / 21.2, 4096 26.0 /
+// 23.5, 11.6k (adaptive) 55.6 / 54.9, 16k 70.4 / 70.0, 66k 262 / 267; 16x16, 256
+// 20.7 / 17.7, 4096 69.7 / 69.4, 6403 (adaptive) 102.2 / 103.6; the row-marching
+// tiles, whose waves hold several patches: 4x4, 1024 17.4 / 14.3, 16k 28.0 / 26.0,
+// 66k 77.0 / 76.9; 2x2, 16k 21.0 / 17.8, 66k 36.1 / 36.4.
 // Instances without quadrants are kept as two words of bits (publish_empty), so at
 // most 128 instances where there may be some: a batch of 16 adaptive runs that end
-// one after the other 73.7 ms with the kernel as soon as one has ended, 70.6 so.
+// one after the other 73.7 ms with the kernel as soon as one has ended, 70.6 so
+// (medians of 25 passes; single processes differ by up to 5 %).
 bool wants_self(const amrgpu_ctx *c)
 {
     const TileVariant &v = kVariants[c->variant];

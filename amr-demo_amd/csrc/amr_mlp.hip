@@ -88,7 +88,6 @@ __device__ __forceinline__ f4v mfma32(s8v a, s8v b, f4v c)
 }
 
 __device__ __forceinline__ unsigned long long d2bits(double v) { return (unsigned long long)__double_as_longlong(v); }
-__device__ __forceinline__ double bits2d(unsigned long long b) { return __longlong_as_double((long long)b); }
 
 // ---------------------------------------------------------------------------
 // features: one wave per 8x8 patch, four patches per workgroup.  Memory is the
