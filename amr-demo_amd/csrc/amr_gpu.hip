@@ -3197,8 +3197,8 @@ bool device_reaches(const void *p)
 }
 
 // The caller's `bytes` at src to the device, ordered on the stream.  src may change
-// once it returns, or with `stays` at the next wait for the stream only: then large
-// arrays are left to the runtime's own staging (us per upload of a state, chunks /
+// once it returns, or with `stays` (a caller that waits for the stream on every way
+// out) at the next wait only.  Large arrays are left to the runtime's own staging (us per upload of a state, chunks /
 // runtime once warm: 32 KB 22 / 35, 512 KB 37.5 / 38, 2 MB 98 / 93, 6 MB 195 / 203,
 // 24 MB 678 / 697, 32 MB 1010 / 945, 512 MB 18890 / 18220; for its first tens of calls
 // a process pays it up to 200 us each, so smaller arrays stay with the chunks).
@@ -3206,7 +3206,7 @@ bool device_reaches(const void *p)
 constexpr size_t IN_CHUNKS_MAX = (size_t)24 << 20;
 int copy_in(amrgpu_ctx *c, void *dst, const void *src, size_t bytes, bool stays)
 {
-    if ((stays && bytes > IN_CHUNKS_MAX) || device_reaches(src)) {
+    if (bytes > IN_CHUNKS_MAX || device_reaches(src)) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
         return stays ? AMRGPU_OK : sync_stream(c);
     }
@@ -3517,13 +3517,12 @@ static int set_clocks(amrgpu_ctx *c, const double *t_inst)
     return AMRGPU_OK;
 }
 
-// The reference-layout state to the device, ordered on the stream; it stays as it is
-// until the stream is waited for.
-static int start_upload(amrgpu_ctx *c, const double *soln)
+// The reference-layout state to the device, ordered on the stream (stays: copy_in).
+static int start_upload(amrgpu_ctx *c, const double *soln, bool stays)
 {
     const int n2 = c->n * c->n;
     const long long ncells = (long long)c->nquad * n2;
-    if (int rc = copy_in(c, c->d_stage, soln, sizeof(double) * 4 * ncells, true)) return rc;
+    if (int rc = copy_in(c, c->d_stage, soln, sizeof(double) * 4 * ncells, stays)) return rc;
     c->cur = 0;
     hipLaunchKernelGGL(aos_to_soa_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, c->stream,
                        c->d_stage, c->U[0], ncells, n2);
@@ -3531,10 +3530,9 @@ static int start_upload(amrgpu_ctx *c, const double *soln)
     return AMRGPU_OK;
 }
 
-int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
-                      const amrgpu_inst_t *inst, int ncell, const int *cell_info,
-                      const int *cell_inst, int nface, const int *face_info, const double *geom,
-                      const double *soln, const double *t_inst)
+static int setup_mesh(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst, const amrgpu_inst_t *inst,
+                      int ncell, const int *cell_info, const int *cell_inst, int nface, const int *face_info,
+                      const double *geom, const double *soln, const double *t_inst, bool stays)
 {
     if (!c || !inst || !cell_info || ncell <= 0 || ninst <= 0 || nface < 0) {
         set_err("amrgpu_setup: bad arguments");
@@ -3613,8 +3611,17 @@ int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int nin
     memcpy(hip, c->h_ip.data(), sizeof(InstDev) * ninst);
     HIPCHK(hipMemcpyAsync(c->d_ip, hip, sizeof(InstDev) * ninst, hipMemcpyHostToDevice, c->stream));
     if ((rc = set_clocks(c, t_inst))) return rc;
-    if (soln) return start_upload(c, soln);
+    if (soln) return start_upload(c, soln, stays);
     return AMRGPU_OK;
+}
+
+int amrgpu_setup_from(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
+                      const amrgpu_inst_t *inst, int ncell, const int *cell_info,
+                      const int *cell_inst, int nface, const int *face_info, const double *geom,
+                      const double *soln, const double *t_inst)
+{
+    return setup_mesh(c, nelem_subgrid, time_scheme, ninst, inst, ncell, cell_info, cell_inst, nface, face_info, geom, soln,
+                      t_inst, false);
 }
 
 int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
@@ -3623,9 +3630,11 @@ int amrgpu_setup(amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
                  const double *soln)
 {
     if (!face_info) { set_err("amrgpu_setup: bad arguments"); return AMRGPU_ERR_ARG; }
-    int rc = amrgpu_setup_from(c, nelem_subgrid, time_scheme, ninst, inst, ncell, cell_info, cell_inst, nface,
-                               face_info, geom, soln, nullptr);
-    return rc ? rc : sync_stream(c);
+    int rc = setup_mesh(c, nelem_subgrid, time_scheme, ninst, inst, ncell, cell_info, cell_inst, nface, face_info, geom,
+                        soln, nullptr, true);
+    if (!c) return rc;
+    const int waited = sync_stream(c);
+    return rc ? rc : waited;
 }
 
 int amrgpu_set_geometry(amrgpu_ctx *c, const double *geom)
@@ -3854,8 +3863,8 @@ int amrgpu_nbr_from_faces(int ncell, int nface, const int *face_info, int *nbr)
 int amrgpu_upload_soln(amrgpu_ctx *c, const double *soln)
 {
     if (!c || !soln || !c->nquad) { set_err("amrgpu_upload_soln: no mesh"); return AMRGPU_ERR_ARG; }
-    int rc = start_upload(c, soln);
-    return rc ? rc : sync_stream(c);
+    const int rc = start_upload(c, soln, true), waited = sync_stream(c);
+    return rc ? rc : waited;
 }
 
 int amrgpu_download_soln(amrgpu_ctx *c, double *soln)

@@ -39,9 +39,9 @@ AMR_HIDDEN int amrgpu_staging(struct amrgpu_ctx *c, double **buf, size_t *ndoubl
  * the host; complete when it returns. */
 AMR_HIDDEN int amrgpu_fetch(struct amrgpu_ctx *c, void *dst, const void *src, size_t bytes);
 /* amrgpu_setup without its final wait: the device work is ordered on the
- * context's stream, and soln is read until the stream is waited for.  face_info
- * NULL: no faces (every side a boundary), for calls that evaluate none.  t_inst:
- * the instances' times (NULL: 0). */
+ * context's stream, and the caller's arrays may change.  face_info NULL: no faces
+ * (every side a boundary), for calls that evaluate none.  t_inst: the instances'
+ * times (NULL: 0). */
 AMR_HIDDEN int amrgpu_setup_from(struct amrgpu_ctx *c, int nelem_subgrid, int time_scheme, int ninst,
                                  const amrgpu_inst_t *inst, int ncell, const int *cell_info, const int *cell_inst,
                                  int nface, const int *face_info, const double *geom, const double *soln,

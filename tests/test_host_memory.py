@@ -33,6 +33,8 @@ static size_t copy_bytes[1024];
 /* the caller's pinned array */
 static char *mine;
 static size_t mine_bytes;
+static int reads_mine;      /* a copy from it may be under way */
+static hipError_t launch_error = hipSuccess;
 
 hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; ++host_allocs; *p = calloc(n, 1); return hipSuccess; }
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
@@ -46,6 +48,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
     copy_src[copies % 1024] = s;
     copy_bytes[copies % 1024] = n;
     copy_dst[copies++ % 1024] = d;
+    if (mine && (const char *)s >= mine && (const char *)s < mine + mine_bytes) reads_mine = 1;
     memcpy(d, s, n);
     return hipSuccess;
 }
@@ -60,13 +63,13 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
     }
     return hipSuccess;
 }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return launch_error; }
 const char *hipGetErrorString(hipError_t e) { (void)e; return "error"; }
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = cus; return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { (void)f; *s = (hipStream_t)&copies; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { (void)s; return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; reads_mine = 0; return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { (void)f; *e = (hipEvent_t)&launches; return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { (void)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { (void)e; (void)s; return hipSuccess; }
@@ -338,4 +341,52 @@ def test_limits_follow_the_devices_compute_units(tmp_path, cus):
     MUST(amr_mlp_forward(m, X, rows + 1, z));
     HOLDS(grid.x == 2 * {cus});
     amr_mlp_destroy(m);
+""")
+
+
+def test_no_call_returns_while_the_callers_pinned_array_is_read(tmp_path):
+    """not where it fails after the copy has been started, either"""
+    run(tmp_path, """
+    enum { nq = 64, bytes = nq * 16 * 8 };
+    static int ci[3 * nq], fi[44 * nq];
+    static double rhs[nq * 16];
+    for (int q = 0; q < nq; ++q) {
+        ci[3 * q + 2] = 16 * q;
+        for (int s = 0; s < 4; ++s) { int *f = fi + 11 * (4 * q + s); f[0] = 1; f[1] = s; f[2] = q; }
+    }
+    mine = calloc(bytes, 1);
+    mine_bytes = bytes;
+    double *u = (double *)mine, dt = 1.0;
+    amrgpu_ctx *c = amrgpu_create();
+    MUST(set_up(c, nq));
+    MUST(amrgpu_upload_soln(c, u));
+    HOLDS(!reads_mine);
+    MUST(amrgpu_set_origins(c, u));
+    HOLDS(!reads_mine);
+    launch_error = hipErrorInvalidValue;
+    HOLDS(amrgpu_upload_soln(c, u) != 0 && !reads_mine);
+    launch_error = hipSuccess;
+    amrgpu_inst_t in;
+    memset(&in, 0, sizeof(in));
+    in.h_base = 1.0; in.cfl = 0.3; in.dt_cap = 1.0;
+    MUST(amrgpu_setup(c, 2, 3, 1, &in, nq, ci, NULL, 4 * nq, fi, NULL, u));
+    HOLDS(!reads_mine);
+    launch_error = hipErrorInvalidValue;
+    HOLDS(amrgpu_setup(c, 2, 3, 1, &in, nq, ci, NULL, 4 * nq, fi, NULL, u) != 0 && !reads_mine);
+    launch_error = hipSuccess;
+    amrgpu_destroy(c);
+    /* the calls on host arrays, with walls that need the corners that are not given */
+    physics_gpu_params_t p;
+    physics_gpu_get_params(&p);
+    p.dim = 2; p.nfields = 4; p.nelem_subgrid = 2; p.time_scheme = 3; p.time_steps = 10; p.dt = 1.0; p.cfl = 0.3;
+    p.coarse_grid_h = 1.0;
+    for (int s = 0; s < 4; ++s) p.bc[s] = AMRGPU_BC_SHOCK_TOP;
+    physics_gpu_set_params(&p);
+    int dim = 2, nf = 4, n = 2, ncell = nq, nface = 4 * nq, dof = nq * 16, z = 0, one = 1, istep = 0;
+    double sec = 0.0;
+    HOLDS(physics_rhs_structured_gpu(&dim, &nf, &n, &ncell, ci, NULL, &nface, fi, &dof, u, rhs) != 0 && !reads_mine);
+    HOLDS(physics_go_gpu(&dim, &z, &nf, &n, &ncell, &z, &nface, &dof, ci, fi, &z, &z, &z, &z, &z, NULL, u, &istep, &z, &z, &z,
+                         &one, NULL, &sec, &sec, &sec) != 0 && !reads_mine);
+    MUST(physics_time_step_gpu(&dim, &nf, &n, &ncell, ci, NULL, u, &dt));
+    HOLDS(!reads_mine);
 """)
